@@ -74,19 +74,32 @@ template <typename T> struct Vec { typedef T type __attribute__((ext_vector_type
 struct Item { int k, s, jlo, jhi; };    // s >= 0: far chunk s of row k; CHAIN / CSTEP: the row's steps
 constexpr int CHAIN = -1, CSTEP = -2;
 
-// Relaxed polling (an acquire load would invalidate the caches on every
-// poll), then one acquire fence by the polling thread once the flag is seen;
-// a workgroup barrier carries the ordering to the other waves.
+// Values that one workgroup of a launch hands to another (solution blocks, c
+// steps, far partials and the flags): device-scope accesses, which no XCD's
+// L2 or CU's L1 keeps an old copy of.  A release / acquire pair around plain
+// accesses is both slower (an L2 write-back and an invalidation per link of
+// the chain) and not enough here: the polling thread's fence ends in a
+// cache invalidation that nothing waits for, so after the workgroup barrier
+// another wave's plain load could still take the line of an earlier solve
+// (one of some hundred solves at 96 blocks came back 9e-2 off).
+template <typename T>
+__device__ __forceinline__ T dev_load(const T* p) {
+  return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void dev_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Relaxed polling; a workgroup barrier carries the order to the other waves,
+// whose loads of the published values are issued after it.
 __device__ __forceinline__ bool wait_epoch(const unsigned* flag, unsigned epoch, int* err) {
   for (unsigned it = 0; it < SPIN_LIMIT; ++it) {
-    if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      return true;
-    }
-    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
+    if (dev_load(flag) == epoch) return true;
+    if (dev_load(err) != 0) return false;
     __builtin_amdgcn_s_sleep(2);
   }
-  __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  dev_store(err, 1);
   return false;
 }
 
@@ -107,14 +120,13 @@ __device__ __forceinline__ bool group_wait_all(const unsigned* flags, int n, uns
   return *s_ok != 0;
 }
 
-// Every wave first waits for its own global stores to complete (the
-// workgroup barrier alone does not: it orders LDS, and the release of thread 0
-// covers only its own wave's outstanding stores); after the barrier the
-// release store of thread 0 writes back the L2 and publishes the flag.
+// Every wave first waits for its own device-scope stores to complete (the
+// workgroup barrier alone does not: it orders LDS); after the barrier thread 0
+// publishes the flag.
 __device__ __forceinline__ void group_publish(unsigned* flag, unsigned epoch) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_store(flag, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) dev_store(flag, epoch);
 }
 
 // RPW rows of a wave, lane l holding columns VW l .. VW l + VW - 1 of a pass
@@ -309,7 +321,7 @@ __device__ __forceinline__ bool take_ticket(const TrsvCtl& ctl, Item* it, int* s
   if (threadIdx.x == 0) *s_id = (int)(atomicAdd(ctl.ticket, 1ull) - ctl.ticket_base);
   __syncthreads();
   if (*s_id < 0 || *s_id >= ctl.n_items) {                    // ticket counter out of step
-    if (threadIdx.x == 0) __hip_atomic_store(ctl.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) dev_store(ctl.err, 2);
     return false;
   }
   *it = ctl.items[*s_id];
@@ -345,7 +357,7 @@ __device__ __forceinline__ void far_fwd(const Item& it, const T* __restrict__ L,
   T sum = T(0);
   if (ok) {
     const T* x = b + (int64_t)it.jlo * NB;
-    for (int e = threadIdx.x; e < nblk * NB; e += NT) xall[e] = x[e];
+    for (int e = threadIdx.x; e < nblk * NB; e += NT) xall[e] = dev_load(x + e);
     __syncthreads();
     T p[RPW];
 #pragma unroll
@@ -363,7 +375,7 @@ __device__ __forceinline__ void far_fwd(const Item& it, const T* __restrict__ L,
     }
     sum = lane_sums<T>(p, l);
   }
-  if (ok && l < RPW) part[(int64_t)(ctl.rowbase[it.k] + it.s) * NB + row] = sum;
+  if (ok && l < RPW) dev_store(part + (int64_t)(ctl.rowbase[it.k] + it.s) * NB + row, sum);
   group_publish(ctl.pflag + ctl.rowbase[it.k] + it.s, ctl.epoch);
 }
 
@@ -390,7 +402,7 @@ __device__ __forceinline__ void far_bwd(const Item& it, const T* __restrict__ L,
   T sum = T(0);
   if (ok) {
     const T* x = b + (int64_t)it.jlo * NB;
-    for (int e = threadIdx.x; e < nblk * NB; e += NT) xall[e] = x[e];
+    for (int e = threadIdx.x; e < nblk * NB; e += NT) xall[e] = dev_load(x + e);
     __syncthreads();
     vec acc[PS];
 #pragma unroll
@@ -425,7 +437,7 @@ __device__ __forceinline__ void far_bwd(const Item& it, const T* __restrict__ L,
       for (int q = 0; q < NW; ++q) sum += red[q][threadIdx.x];
     }
   }
-  if (ok && threadIdx.x < NB) part[(int64_t)(ctl.rowbase[it.k] + it.s) * NB + threadIdx.x] = sum;
+  if (ok && threadIdx.x < NB) dev_store(part + (int64_t)(ctl.rowbase[it.k] + it.s) * NB + threadIdx.x, sum);
   group_publish(ctl.pflag + ctl.rowbase[it.k] + it.s, ctl.epoch);
 }
 
@@ -476,16 +488,16 @@ void trsv_fwd_kernel(const T* __restrict__ L, int64_t lda, const T* __restrict__
     if (nfar > 1) {
       ok = group_wait_all(ctl.pflag + f0 + 1, nfar - 1, ctl.epoch, ctl.err, &s_ok2);
       if (ok)
-        for (int s = 1; s < nfar; ++s) t -= part[(int64_t)(f0 + s) * NB + row];
+        for (int s = 1; s < nfar; ++s) t -= dev_load(part + (int64_t)(f0 + s) * NB + row);
     }
     if (ok && nfar > 0) {
       ok = group_wait(ctl.pflag + f0, ctl.epoch, ctl.err, &s_ok);
-      if (ok) t -= part[(int64_t)f0 * NB + row];
+      if (ok) t -= dev_load(part + (int64_t)f0 * NB + row);
     }
     if (l < RPW) xs[row] = t;
   } else if (nblk == 0) {
     ok = group_wait(ctl.cflag + it.k, ctl.epoch, ctl.err, &s_ok);
-    if (ok) y = cbuf[k0 + row];
+    if (ok) y = dev_load(cbuf + k0 + row);
   }
   T sum = T(0);
   if (ok) {
@@ -498,13 +510,13 @@ void trsv_fwd_kernel(const T* __restrict__ L, int64_t lda, const T* __restrict__
       if (wflag) {           // chain: c_k (ready links ahead) before the last block's wait
         if (j == nblk - 1) {
           ok = group_wait(ctl.cflag + it.k, ctl.epoch, ctl.err, &s_ok);
-          if (ok) { y = cbuf[k0 + row]; pin1(y); }
+          if (ok) { y = dev_load(cbuf + k0 + row); pin1(y); }
         }
         if (ok) ok = group_wait(wflag + j, ctl.epoch, ctl.err, &s_ok2);
         if (!ok) break;
       }
       if (x) {
-        for (int e = threadIdx.x; e < NB; e += NT) xs[e] = x[(int64_t)j * NB + e];
+        for (int e = threadIdx.x; e < NB; e += NT) xs[e] = dev_load(x + (int64_t)j * NB + e);
       }
       __syncthreads();
       rowacc<T>(R, *reinterpret_cast<const vec*>(xs + Shape<T>::VW * l), p);
@@ -519,10 +531,10 @@ void trsv_fwd_kernel(const T* __restrict__ L, int64_t lda, const T* __restrict__
     sum = lane_sums<T>(p, l);
   }
   if (it.s == CSTEP) {
-    if (ok && l < RPW) cbuf[k0 + row] = sum;
+    if (ok && l < RPW) dev_store(cbuf + k0 + row, sum);
     group_publish(ctl.cflag + it.k, ctl.epoch);
   } else {
-    if (ok && l < RPW) y_out[k0 + row] = y - sum;
+    if (ok && l < RPW) dev_store(y_out + k0 + row, y - sum);
     group_publish(ctl.yflag + it.k, ctl.epoch);
   }
 }
@@ -573,16 +585,16 @@ void trsv_bwd_kernel(const T* __restrict__ L, int64_t lda, const T* __restrict__
     if (nfar > 1) {
       ok = group_wait_all(ctl.pflag + f0 + 1, nfar - 1, ctl.epoch, ctl.err, &s_ok2);
       if (ok && threadIdx.x < NB)
-        for (int s = 1; s < nfar; ++s) t -= part[(int64_t)(f0 + s) * NB + threadIdx.x];
+        for (int s = 1; s < nfar; ++s) t -= dev_load(part + (int64_t)(f0 + s) * NB + threadIdx.x);
     }
     if (ok && nfar > 0) {
       ok = group_wait(ctl.pflag + f0, ctl.epoch, ctl.err, &s_ok);
-      if (ok && threadIdx.x < NB) t -= part[(int64_t)f0 * NB + threadIdx.x];
+      if (ok && threadIdx.x < NB) t -= dev_load(part + (int64_t)f0 * NB + threadIdx.x);
     }
     if (threadIdx.x < NB) xs[threadIdx.x] = t;
   } else if (nblk == 0) {
     ok = group_wait(ctl.cflag + it.k, ctl.epoch, ctl.err, &s_ok);
-    if (ok && threadIdx.x < NB) cv = cbuf[k0 + threadIdx.x];
+    if (ok && threadIdx.x < NB) cv = dev_load(cbuf + k0 + threadIdx.x);
   }
   vec acc[NB / PW];
 #pragma unroll
@@ -597,13 +609,13 @@ void trsv_bwd_kernel(const T* __restrict__ L, int64_t lda, const T* __restrict__
       if (wflag) {           // chain: c'_k (ready links ahead) before the last block's wait
         if (j == nblk - 1) {
           ok = group_wait(ctl.cflag + it.k, ctl.epoch, ctl.err, &s_ok);
-          if (ok && threadIdx.x < NB) { cv = cbuf[k0 + threadIdx.x]; pin1(cv); }
+          if (ok && threadIdx.x < NB) { cv = dev_load(cbuf + k0 + threadIdx.x); pin1(cv); }
         }
         if (ok) ok = group_wait(wflag - j, ctl.epoch, ctl.err, &s_ok2);
         if (!ok) break;
       }
       if (x) {
-        for (int e = threadIdx.x; e < NB; e += NT) xs[e] = x[(int64_t)j * xstride + e];
+        for (int e = threadIdx.x; e < NB; e += NT) xs[e] = dev_load(x + (int64_t)j * xstride + e);
       }
       __syncthreads();
       colacc<T>(R, xs + RPW * w, acc[0]);
@@ -625,10 +637,10 @@ void trsv_bwd_kernel(const T* __restrict__ L, int64_t lda, const T* __restrict__
     }
   }
   if (it.s == CSTEP) {
-    if (ok && threadIdx.x < NB) cbuf[k0 + threadIdx.x] = sum;
+    if (ok && threadIdx.x < NB) dev_store(cbuf + k0 + threadIdx.x, sum);
     group_publish(ctl.cflag + it.k, ctl.epoch);
   } else {
-    if (ok && threadIdx.x < NB) b[k0 + threadIdx.x] = cv - sum;
+    if (ok && threadIdx.x < NB) dev_store(b + k0 + threadIdx.x, cv - sum);
     group_publish(ctl.yflag + it.k, ctl.epoch);
   }
 }
