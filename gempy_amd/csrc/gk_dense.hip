@@ -5,7 +5,7 @@
 //    permuted so that each lane reads its BK/4 consecutive k values with
 //    128-bit LDS loads; MFMA only needs A and B to agree on it.
 //  * Cholesky FP64: recursive on halves of 256-blocks, with a recursive TRSM,
-//    so most flops are large-K GEMMs; Cholesky FP32 and LU without pivoting
+//    so most flops are large-K GEMMs, over right-looking leaves; Cholesky FP32 and LU without pivoting
 //    (FP64): right-looking with 256-wide panels.  Each 256 diagonal block is factored
 //    and inverted as two LDS-resident 128-wide halves joined by 128^3 GEMMs;
 //    a panel solve is a GEMM with the inverted diagonal block.
@@ -77,8 +77,11 @@ template <> struct Mfma<double> {
 // 49-53 (one workgroup per CU leaves the stage barriers uncovered); a second
 // register stage or BK 32 were slower.
 // TM x TN tiles (TN defaults to TM) of WM x WN waves.
-template <int TM_, int WM_, int WN_, int TN_ = TM_>
+// BK: K depth of one LDS stage; RS: register stages of the copy (0: the
+// type's defaults).
+template <int TM_, int WM_, int WN_, int TN_ = TM_, int BK_ = 0, int RS_ = 0>
 struct Tile {
+  static constexpr int BK = BK_, RS = RS_;
   static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, NT = 64 * WM * WN;
   static constexpr int FM = TM / WM / 16, FN = TN / WN / 16;
 };
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(TL::NT) __attribute__((amdgpu_waves_per_eu(WPE, 0))
   C += blockIdx.y * sC;
   constexpr int TM = TL::TM, TN = TL::TN, NT = TL::NT, FM = TL::FM, FN = TL::FN;
   static_assert(!LOWER || TN == TM, "lower-triangle products take square tiles");
-  constexpr int BK = M::BK;
+  constexpr int BK = TL::BK > 0 ? TL::BK : M::BK;
   constexpr int KS = BK / 4;              // k values per lane per stage
   constexpr int PAD = 16 / sizeof(T);     // keep rows 16-byte aligned
   constexpr int LDS_LD = BK + PAD;
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(TL::NT) __attribute__((amdgpu_waves_per_eu(WPE, 0))
   constexpr int NV = TM * BK / VEC / NT, NVB = TN * BK / VEC / NT;
   static_assert(NV >= 1 && NV * NT * VEC == TM * BK, "BK must make the tile a whole number of vectors per thread");
   static_assert(NVB >= 1 && NVB * NT * VEC == TN * BK, "BK must make the tile a whole number of vectors per thread");
-  constexpr int RS = sizeof(T) == 4 ? GK_GEMM_RS_F32 : 1;
+  constexpr int RS = TL::RS > 0 ? TL::RS : (sizeof(T) == 4 ? GK_GEMM_RS_F32 : 1);
   vec_t ra[RS][NV], rb[RS][NVB];
   auto load_global = [&](int64_t k0, vec_t (&xa)[NV], vec_t (&xb)[NVB]) {
 #pragma unroll
@@ -385,6 +388,29 @@ int gemm_launch(int64_t m, int64_t n, int64_t k, const T* A, int64_t lda, const 
       // the GPU.
       gemm_dispatch<T, Tile<64, 1, 4, 128>, 5>(dim3((unsigned)(m / 64), (unsigned)batch), trans_b, false, st, m, n,
                                                k, A, lda, B, ldb, alpha, beta, C, ldc, 1, m / 64, sA, sB, sC);
+      launched = true;
+    }
+  } else {
+    // FP64 products that cannot fill the chip with 128 x 128 tiles (a
+    // factorization's panels, diagonal blocks and small trailing blocks) are
+    // latency-bound: a 128^3 product on one such tile took 24-30 us, eight
+    // 16-deep stages of one global latency each.  Small tiles with 32-deep
+    // stages, two of them in flight, spread them over the chip.
+    constexpr int64_t FEW = 512;          // 128 x 128 tiles: two per CU
+    if (k % 32 == 0 && row_tiles) {       // 16 rows x all 128 columns, 4 waves of 16 x 32
+      gemm_dispatch<T, Tile<16, 1, 4, 128, 32, 2>, 2>(dim3((unsigned)(m / 16), (unsigned)batch), trans_b, false, st, m,
+                                                      n, k, A, lda, B, ldb, alpha, beta, C, ldc, 1, m / 16, sA, sB, sC);
+      launched = true;
+    } else if (k % 32 == 0 && lower && tiles * batch < FEW) {
+      const int64_t t64 = m / 64;
+      gemm_dispatch<T, Tile<64, 2, 2, 64, 32, 2>, 2>(dim3((unsigned)(t64 * (t64 + 1) / 2), (unsigned)batch), trans_b,
+                                                     true, st, m, n, k, A, lda, B, ldb, alpha, beta, C, ldc, t64,
+                                                     t64 * (t64 + 1) / 2, sA, sB, sC);
+      launched = true;
+    } else if (k % 32 == 0 && !lower && tiles * batch < FEW) {
+      const int64_t t = (m / 32) * (n / 64);
+      gemm_dispatch<T, Tile<32, 2, 2, 64, 32, 2>, 2>(dim3((unsigned)t, (unsigned)batch), trans_b, false, st, m, n, k,
+                                                     A, lda, B, ldb, alpha, beta, C, ldc, n / 64, t, sA, sB, sC);
       launched = true;
     }
   }
@@ -800,42 +826,40 @@ __global__ __launch_bounds__(1024) void getrf128_kernel(double* A, int64_t lda, 
 }
 
 // Blocked Cholesky + inverse of a DB x DB block (one workgroup of NT threads),
-// two barriers per PB columns.  Phase 1 (wave 0, registers, lane values
-// broadcast through scalar registers): factor the PB-column panel, then the PB
-// rows of X = L^-1,
+// two barriers per PB = 16 columns.  Phase 1 (wave 0, registers, lane values
+// broadcast through scalar registers): factor the 16-column panel, while the
+// other waves apply the previous panel to the rows of X = L^-1 below it.
+// Phase 2: the last two waves form the panel's 16 rows of X,
 //   X[i][c] = (delta_ic - acc[i][c] - sum_{jb<=k<i} L[i][k] X[k][c]) / L[i][i],
-// where acc[i][c] = sum_{k<jb} L[i][k] X[k][c] was applied eagerly.  Phase 2
-// (all threads): the rank-PB trailing update of L and the eager update of the
-// later rows of X by the new panel and rows, in one sweep per row.
-#ifndef GK_POTRF_PB_F32
-#define GK_POTRF_PB_F32 16
-#endif
-#ifndef GK_POTRF_PB_F64
-#define GK_POTRF_PB_F64 4
-#endif
-// LDS: L and X = L^-1 as packed lower triangles, then two panel buffers P[b]
-// holding the PB columns of the current / next panel column-major (P[b][t][i]
-// = L[i][jb + t]): wave 0 loads its panel rows without per-row branches (16%
-// less time in phase 1 than from the packed rows) and the sweep reads the
-// panel with consecutive addresses.  FP32 72.5 KB, FP64 137 KB.
-template <typename T, int PB>
+// where acc[i][c] = sum_{k<jb} L[i][k] X[k][c] was applied eagerly, and the
+// other waves apply the panel to the trailing tiles of L and write the
+// panel to A.
+// LDS: one packed lower triangle S.  Row i holds X (or -acc) in the columns
+// already factored and the trailing matrix in the others: a column of L is
+// dead there once its panel is factored, which is when X needs its place.
+// Two panel buffers P[b] hold the 16 columns of the current / next panel
+// column-major (P[b][t][i] = L[i][jb + t]): wave 0 loads its panel rows
+// without per-row branches (16% less time in phase 1 than from the packed
+// rows) and the tiles read the panel with consecutive addresses.  FP32
+// 48.5 KB, FP64 97 KB (two triangles and 16-column panels would need 161 KB
+// in FP64, more than a CU has).
+constexpr int GK_POTRF_PB = 16;
+template <typename T>
 struct BlkStore {
+  static constexpr int PB = GK_POTRF_PB;
   T* S;
-  static constexpr int SIZE = DB * (DB + 1) + 2 * PB * DB + PB;
+  static constexpr int SIZE = DB * (DB + 1) / 2 + 2 * PB * DB + PB;
   __device__ static int pl(int i, int c) { return i * (i + 1) / 2 + c; }
-  __device__ T& L(int i, int c) { return S[pl(i, c)]; }
-  __device__ T& X(int i, int c) { return S[DB * (DB + 1) / 2 + pl(i, c)]; }
-  __device__ T& P(int b, int t, int i) { return S[DB * (DB + 1) + (b * PB + t) * DB + i]; }
-  __device__ T& ipv(int j) { return S[DB * (DB + 1) + 2 * PB * DB + j]; }   // 1 / pivot of the current panel
+  __device__ T& V(int i, int c) { return S[pl(i, c)]; }
+  __device__ T& P(int b, int t, int i) { return S[DB * (DB + 1) / 2 + (b * PB + t) * DB + i]; }
+  __device__ T& ipv(int j) { return S[DB * (DB + 1) / 2 + 2 * PB * DB + j]; }   // 1 / pivot of the current panel
 };
-// FP32 diagonal-block kernel: threads.  It runs on the side stream beside the
-// trailing update, whose workgroups (512 threads, 80 VGPRs, 40 KB LDS) sit
-// three to a CU: with 512 threads, < 96 VGPRs and < 80 KB of LDS it fits on a
-// CU where one of them has finished, while a 1024-thread version needs an
-// empty CU and waits for the end of the update.
-#ifndef GK_POTRF_NT_F32
-#define GK_POTRF_NT_F32 512
-#endif
+// Threads of the diagonal-block kernels: 8 waves, so that wave 0 may hold its
+// panel rows in registers (FP64: 64 VGPRs of them; 16 waves would leave 128
+// per wave).  The FP32 kernel runs on the side stream beside the trailing
+// update: with 512 threads it fits on a CU where a workgroup of that update
+// has finished, while a 1024-thread version waits for the end of the update.
+constexpr int GK_POTRF_NT = 512;
 
 // Value of v in lane l (l uniform) as a scalar-register broadcast.
 __device__ __forceinline__ float lane_value(float v, int l) {
@@ -848,20 +872,34 @@ __device__ __forceinline__ double lane_value(double v, int l) {
 }
 
 // Pivot d > 0 -> (sqrt(d), 1/sqrt(d)).  FP32: the hardware reciprocal square
-// root (within 1 ulp), the factor being an FP32 preconditioner; FP64: IEEE.
+// root (within 1 ulp), the factor being an FP32 preconditioner.  FP64: the
+// hardware seed, two Newton steps, then one residual step each for the root
+// and the reciprocal (both within 1 ulp; a chain of 9 dependent FMAs where the
+// IEEE square root and division take several times that).
 __device__ __forceinline__ void pivot_pair(float d, float& piv, float& ip) {
   ip = __builtin_amdgcn_rsqf(d);
   piv = d * ip;
 }
 __device__ __forceinline__ void pivot_pair(double d, double& piv, double& ip) {
-  piv = sqrt(d);
-  ip = 1.0 / piv;
+  double y = __builtin_amdgcn_rsq(d);
+  y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+  y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+  const double s = d * y;
+  piv = fma(0.5 * y, fma(-s, s, d), s);
+  ip = fma(y, fma(-piv, y, 1.0), y);
 }
 
-template <typename T, int PB, int NT>
-__device__ void potrf_blocked(BlkStore<T, PB> B, T* A, int64_t lda, T* X, int64_t ldx, int32_t* info, int64_t gbase) {
-  constexpr int RS = NT / 32;                 // rows of the trailing update in flight
-  const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5, lane = tid & 63, wave = tid >> 6;
+__device__ __forceinline__ f4v mma4(float a, float b, f4v c) { return Mfma<float>::mma(a, b, c); }
+__device__ __forceinline__ d4v mma4(double a, double b, d4v c) { return Mfma<double>::mma(a, b, c); }
+
+// live: columns of the block that belong to the matrix (the rest is identity
+// padding, whose factor and inverse are themselves: its panels are skipped).
+template <typename T, int NT>
+__device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ldx, int32_t* info, int64_t gbase,
+                              int live) {
+  constexpr int PB = GK_POTRF_PB;
+  using acc_t = typename Mfma<T>::acc_t;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // all loads of the block first (in flight together, 16 bytes each), then
   // the LDS stores
   constexpr int VL = 16 / sizeof(T);          // elements per 16-byte load
@@ -883,84 +921,60 @@ __device__ void potrf_blocked(BlkStore<T, PB> B, T* A, int64_t lda, T* X, int64_
 #pragma unroll
     for (int u = 0; u < VL; ++u) {
       if (c + u <= i) {
-        B.L(i, c + u) = vin[q][u];
-        B.X(i, c + u) = T(0);
+        B.V(i, c + u) = vin[q][u];
         if (c + u < PB) B.P(0, c + u, i) = vin[q][u];
       }
     }
   }
   __syncthreads();
+  const int nlive = min(DB, (live + PB - 1) / PB * PB);   // rows and columns that are factored
   int bad_col = 0;                            // first non-positive pivot + 1 (wave 0)
-  // FP32: the rows of X are computed by the last two waves from the stored
-  // panel (64 columns each) while the other waves apply the panel to the
-  // trailing L tiles; the X tiles follow beside the next panel's factor.
-  constexpr bool SPLIT_X = sizeof(T) == 4 && PB == 16 && NT >= 128;
-  constexpr int XW = NT / 64 - 1;             // the last of the two waves of the X rows
-  // ---- rows jb .. jb+PB-1 of X from the panel's diagonal block (lane l holds
-  //      row jb + l in a) and the reciprocal pivots: lane owns columns lane
-  //      and lane + 64
-  // pb >= 0: the panel's entries come from the stored panel P[pb] (LDS
-  // broadcasts: a wave other than the one that factored it), else from a.
-  auto x_rows = [&](int jb, const T (&a)[PB], const T (&ipv)[PB], int pb) {
-    T xa[PB], xb[PB];
-    const int ca = lane, cb = lane + 64;
-#pragma unroll
-    for (int r = 0; r < PB; ++r) {
-      const int i = jb + r;
-      xa[r] = ca < jb ? B.X(i, ca) : (ca == i ? T(1) : T(0));  // B.X holds -acc[i][c] for c < jb
-      xb[r] = cb < jb ? B.X(i, cb) : (cb == i ? T(1) : T(0));
-    }
-    // right-looking: row k is final once the rows above it are applied, and
-    // then goes into every later row (each row takes the same products in the
-    // same order as a row-by-row substitution; the dependent chain is 16
-    // steps, not 120)
-#pragma unroll
-    for (int k = 0; k < PB; ++k) {
-      xa[k] *= ipv[k];
-      xb[k] *= ipv[k];
-#pragma unroll
-      for (int r = k + 1; r < PB; ++r) {
-        const T lrk = pb >= 0 ? B.P(pb, k, jb + r) : lane_value(a[k], r);   // L[jb+r][jb+k]
-        xa[r] -= lrk * xa[k];
-        xb[r] -= lrk * xb[k];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < PB; ++r) {
-      const int i = jb + r;
-      if (ca <= i) B.X(i, ca) = xa[r];
-      if (cb <= i) B.X(i, cb) = xb[r];
-    }
-  };
-  // the same for one column per lane (c = lane + coff), the panel's entries
-  // from the stored panel P[pb] (LDS broadcasts): two waves share the rows
-  auto x_rows1 = [&](int jb, int pb, int coff) {
-    T x[PB], ipv[PB];
+  constexpr int NW = NT / 64, XW = NW - 2;    // phase 2: waves XW, XW + 1 form the X rows
+  // rows jb .. jb+PB-1 of X from the panel's diagonal block in P[pb] (LDS
+  // broadcasts), one column per lane (c = lane + coff).  Right-looking: row k
+  // is final once the rows above it are applied, and then goes into every
+  // later row (each row takes the same products in the same order as a
+  // row-by-row substitution; the dependent chain is 16 steps, not 120).
+  auto x_rows = [&](int jb, int pb, int coff) {
+    T x[PB], col[2][PB];
     const int c = lane + coff;
+    if (c >= jb + PB) return;
 #pragma unroll
     for (int r = 0; r < PB; ++r) {
       const int i = jb + r;
-      x[r] = c < jb ? B.X(i, c) : (c == i ? T(1) : T(0));
-      ipv[r] = B.ipv(r);
+      const T v = B.V(i, min(c, jb));                     // -acc[i][c] for c < jb
+      x[r] = c < jb ? v : (c == i ? T(1) : T(0));
+      col[0][r] = r > 0 ? B.P(pb, 0, i) : B.ipv(0);
     }
+    // column k + 1 of the panel (and its reciprocal pivot, in place of the
+    // diagonal) is read beside step k; the barrier keeps later columns out of
+    // the registers
 #pragma unroll
     for (int k = 0; k < PB; ++k) {
-      x[k] *= ipv[k];
+      const T (&lk)[PB] = col[k & 1];
+      if (k + 1 < PB) {
 #pragma unroll
-      for (int r = k + 1; r < PB; ++r) x[r] -= B.P(pb, k, jb + r) * x[k];   // L[jb+r][jb+k]
+        for (int r = k + 1; r < PB; ++r) col[(k + 1) & 1][r] = r > k + 1 ? B.P(pb, k + 1, jb + r) : B.ipv(r);
+      }
+      x[k] *= lk[k];
+#pragma unroll
+      for (int r = k + 1; r < PB; ++r) x[r] -= lk[r] * x[k];   // L[jb+r][jb+k]
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int r = 0; r < PB; ++r)
-      if (c <= jb + r) B.X(jb + r, c) = x[r];
+      if (c <= jb + r) B.V(jb + r, c) = x[r];
   };
-  // ---- phase 2 on MFMA (16 x 16 x 4 f32), one 16 x 16 tile per wave at a time
-  //      (waves w, w + nw, ...):
-  //      L tiles (ti >= tj >= c0/16):  L[i][c] -= sum_t L[i][jb+t] L[c][jb+t]
-  //      X tiles (ti >= c0/16 > tj):   X[i][c] -= sum_t L[i][jb+t] X[jb+t][c]
+  // rank-16 updates on MFMA (16 x 16 x 4), one 16 x 16 tile per wave at a time
+  // (waves w, w + nw, ...), by the panel of columns jb = c0 - 16:
+  //   L tiles (ti >= tj >= c0/16):  L[i][c] -= sum_t L[i][jb+t] L[c][jb+t]
+  //   X tiles (ti >= c0/16 > tj):   X[i][c] -= sum_t L[i][jb+t] X[jb+t][c]
   // Operands from the column-major panel buffer P[pb] (and the packed X rows
-  // of the panel); a lane holds C[4 (lane/16) + r][lane % 16] of a tile.
-  auto mfma_tiles = [&](auto jb, int pb, int c0, bool is_l, int w, int nw) {
-    const int a = c0 / 16, nt = DB / 16 - a;             // first trailing tile row, tile rows left
+  // of the panel).  The X tiles of the panel's own columns start from 0.  A
+  // lane holds column lane % 16 of a tile, its rows 4 (lane/16) + r (f32) or
+  // lane/16 + 4 r (f64).
+  auto mfma_tiles = [&](int c0, int pb, bool is_l, int w, int nw) {
+    const int jb = c0 - PB, a = c0 / 16, nt = nlive / 16 - a;   // first trailing tile row, tile rows left
     const int count = is_l ? nt * (nt + 1) / 2 : nt * a;
     const int lr = lane & 15, lq = lane >> 4;
     for (int tile = w; tile < count; tile += nw) {
@@ -975,46 +989,44 @@ __device__ void potrf_blocked(BlkStore<T, PB> B, T* A, int64_t lda, T* X, int64_
         tj = tile % a;
       }
       const int i0 = ti * 16, cb = tj * 16;
-      f4v acc;
+      acc_t acc;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = i0 + lq * 4 + r, c = cb + lr;
-        acc[r] = is_l ? (c <= i ? B.L(i, c) : 0.0f) : B.X(i, c);
+        const int i = i0 + (sizeof(T) == 8 ? lq + 4 * r : lq * 4 + r), c = cb + lr;
+        acc[r] = is_l ? (c <= i ? B.V(i, c) : T(0)) : (tj == a - 1 ? T(0) : B.V(i, c));
       }
 #pragma unroll
       for (int ks = 0; ks < PB / 4; ++ks) {
         const int t = ks * 4 + lq;
-        const float av = -B.P(pb, t, i0 + lr);            // A[row][k] = L[i0+lr][jb+t]
-        float bv;
+        const T av = -B.P(pb, t, i0 + lr);                // A[row][k] = L[i0+lr][jb+t]
+        T bv;
         if (is_l) bv = B.P(pb, t, cb + lr);               // B[k][col] = L[cb+lr][jb+t]
-        else bv = (cb + lr <= jb + t) ? B.X(jb + t, cb + lr) : 0.0f;
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
+        else bv = (cb + lr <= jb + t) ? B.V(jb + t, cb + lr) : T(0);
+        acc = mma4(av, bv, acc);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = i0 + lq * 4 + r, c = cb + lr;
+        const int i = i0 + (sizeof(T) == 8 ? lq + 4 * r : lq * 4 + r), c = cb + lr;
         if (is_l) {
           if (c <= i) {
-            B.L(i, c) = acc[r];
+            B.V(i, c) = acc[r];
             if (c < c0 + PB) B.P(pb ^ 1, c - c0, i) = acc[r];
           }
         } else {
-          B.X(i, c) = acc[r];
+          B.V(i, c) = acc[r];
         }
       }
     }
   };
-  for (int jb = 0, pb = 0; jb < DB; jb += PB, pb ^= 1) {
-    if constexpr (SPLIT_X) {
-      // the previous step's X tiles beside this step's panel (they touch
-      // only X, which the panel does not read)
-      if (wave > 0 && jb > 0) mfma_tiles(jb - PB, pb ^ 1, jb, false, wave - 1, NT / 64 - 1);
-    }
+  for (int jb = 0, pb = 0; jb < nlive; jb += PB, pb ^= 1) {
+    // the previous panel's X tiles beside this panel (they touch only X,
+    // which the panel does not read)
+    if (wave > 0 && jb > 0) mfma_tiles(jb, pb ^ 1, false, wave - 1, NW - 1);
     if (wave == 0) {
       // ---- panel: lane l holds rows jb + l (a) and jb + 64 + l (b)
       const int ra = jb + lane, rb = jb + 64 + lane;
       const int rac = min(ra, DB - 1), rbc = min(rb, DB - 1);
-      T a[PB], b[PB], ipv[PB];
+      T a[PB], b[PB];
 #pragma unroll
       for (int c = 0; c < PB; ++c) {
         const T va = B.P(pb, c, rac), vb = B.P(pb, c, rbc);
@@ -1033,7 +1045,7 @@ __device__ void potrf_blocked(BlkStore<T, PB> B, T* A, int64_t lda, T* X, int64_
           }
           T piv, ip;
           pivot_pair(d, piv, ip);
-          ipv[j] = ip;
+          B.ipv(j) = ip;                          // every lane the same value
           const T aj = lane > j ? a[j] * ip : T(0);
           if constexpr (decltype(with_b)::value) b[j] *= ip;
 #pragma unroll
@@ -1049,102 +1061,64 @@ __device__ void potrf_blocked(BlkStore<T, PB> B, T* A, int64_t lda, T* X, int64_
       else factor(std::false_type{});
 #pragma unroll
       for (int c = 0; c < PB; ++c) {
-        if (ra < DB && jb + c <= ra) B.L(ra, jb + c) = a[c];
-        if (rb < DB) B.L(rb, jb + c) = b[c];
         if (ra < DB) B.P(pb, c, ra) = a[c];
         if (rb < DB) B.P(pb, c, rb) = b[c];
       }
-      if constexpr (SPLIT_X) {
-        if (lane < PB) B.ipv(lane) = ipv[lane];
-      } else {
-        x_rows(jb, a, ipv, -1);
-      }
     }
     __syncthreads();
-    const int c0 = jb + PB;
-    if constexpr (SPLIT_X) {
-      if (wave >= XW - 1) {
-        x_rows1(jb, pb, wave == XW ? 64 : 0);
-      } else {
-        mfma_tiles(jb, pb, c0, true, wave, XW - 1);
+    if (wave >= XW) {
+      x_rows(jb, pb, wave == XW ? 0 : 64);
+    } else {
+      mfma_tiles(jb + PB, pb, true, wave, XW);
+      // the panel's columns of L into A: its diagonal tile, then the rows below
+      if (tid < PB * PB) {
+        const int r = tid / PB, c = tid % PB;
+        if (c <= r) A[(jb + r) * lda + jb + c] = B.P(pb, c, jb + r);
       }
-      __syncthreads();
-      continue;                               // (the last step has no X tiles)
-    }
-    // ---- rows i >= c0: L[i][c] -= sum_t L[i][jb+t] L[c][jb+t]   (c0 <= c <= i;
-    //      the next panel's columns also into P[pb^1])
-    //                    -acc[i][c] -= sum_t L[i][jb+t] X[jb+t][c] (c < c0, X lower)
-    for (int i = c0 + ty; i < DB; i += RS) {
-      T li[PB];
+      for (int e = tid; e < (nlive - jb - PB) * (PB / VL); e += XW * 64) {
+        const int i = jb + PB + e / (PB / VL), c = e % (PB / VL) * VL;
+        vt v;
 #pragma unroll
-      for (int t = 0; t < PB; ++t) li[t] = B.P(pb, t, i);
-      for (int c = tx; c <= i; c += 32) {
-        T sacc = T(0);
-        if (c >= c0) {
-#pragma unroll
-          for (int t = 0; t < PB; ++t) sacc = fma(li[t], B.P(pb, t, c), sacc);
-          const T v = B.L(i, c) - sacc;
-          B.L(i, c) = v;
-          if (c < c0 + PB) B.P(pb ^ 1, c - c0, i) = v;
-        } else {
-#pragma unroll
-          for (int t = 0; t < PB; ++t) {
-            const T xv = B.X(jb + t, c);
-            sacc = fma(li[t], jb + t >= c ? xv : T(0), sacc);
-          }
-          B.X(i, c) -= sacc;
-        }
+        for (int u = 0; u < VL; ++u) v[u] = B.P(pb, c + u, i);
+        *reinterpret_cast<vt*>(A + i * lda + jb + c) = v;
       }
     }
-    __syncthreads();
+    __syncthreads();                          // (the last panel has no X tiles)
   }
   if (wave == 0 && lane == 0 && bad_col != 0) atomicCAS(info, 0, (int32_t)(gbase + bad_col));
   for (int e = tid * VL; e < DB * DB; e += NT * VL) {
     const int i = e / DB, c = e % DB;
-    vt l, x;
+    vt x;
 #pragma unroll
-    for (int u = 0; u < VL; ++u) {
-      l[u] = c + u <= i ? B.L(i, c + u) : T(0);
-      x[u] = c + u <= i ? B.X(i, c + u) : T(0);
-    }
-    if (c + VL - 1 <= i) {
-      *reinterpret_cast<vt*>(A + i * lda + c) = l;
-    } else {
-#pragma unroll
-      for (int u = 0; u < VL; ++u)
-        if (c + u <= i) A[i * lda + c + u] = l[u];
-    }
+    for (int u = 0; u < VL; ++u) x[u] = i >= nlive ? (c + u == i ? T(1) : T(0)) : (c + u <= i ? B.V(i, c + u) : T(0));
     *reinterpret_cast<vt*>(X + i * ldx + c) = x;
   }
 }
 
-// FP32: 72.5 KB of LDS, so the kernel fits on a CU beside workgroups of the
+// FP32: 48.5 KB of LDS, so the kernel fits on a CU beside a workgroup of the
 // concurrent trailing update (the look-ahead factorization runs it on a
 // second stream).
-__global__ __launch_bounds__(GK_POTRF_NT_F32) void potrf128b_f32_kernel(float* A, int64_t lda, float* X, int64_t ldx,
-                                                                        int32_t* info, int64_t gbase) {
-  __shared__ float S[BlkStore<float, GK_POTRF_PB_F32>::SIZE];
-  potrf_blocked<float, GK_POTRF_PB_F32, GK_POTRF_NT_F32>(BlkStore<float, GK_POTRF_PB_F32>{S}, A, lda, X, ldx, info,
-                                                         gbase);
+__global__ __launch_bounds__(GK_POTRF_NT) void potrf128b_f32_kernel(float* A, int64_t lda, float* X, int64_t ldx,
+                                                                    int32_t* info, int64_t gbase, int live) {
+  __shared__ __attribute__((aligned(16))) float S[BlkStore<float>::SIZE];
+  potrf_blocked<float, GK_POTRF_NT>(BlkStore<float>{S}, A, lda, X, ldx, info, gbase, live);
 }
 
-__global__ __launch_bounds__(1024) void potrf128b_f64_kernel(double* A, int64_t lda, double* X, int64_t ldx,
-                                                             int32_t* info, int64_t gbase) {
-  __shared__ double S[BlkStore<double, GK_POTRF_PB_F64>::SIZE];
-  potrf_blocked<double, GK_POTRF_PB_F64, 1024>(BlkStore<double, GK_POTRF_PB_F64>{S}, A, lda, X, ldx, info, gbase);
+__global__ __launch_bounds__(GK_POTRF_NT) void potrf128b_f64_kernel(double* A, int64_t lda, double* X, int64_t ldx,
+                                                                    int32_t* info, int64_t gbase, int live) {
+  __shared__ __attribute__((aligned(16))) double S[BlkStore<double>::SIZE];
+  potrf_blocked<double, GK_POTRF_NT>(BlkStore<double>{S}, A, lda, X, ldx, info, gbase, live);
 }
 
-template <typename T> struct Potrf128;
-template <> struct Potrf128<float> {
-  static void launch(float* A, int64_t lda, float* X, int64_t ldx, int32_t* info, int64_t g, hipStream_t st) {
-    hipLaunchKernelGGL(potrf128b_f32_kernel, dim3(1), dim3(GK_POTRF_NT_F32), 0, st, A, lda, X, ldx, info, g);
-  }
-};
-template <> struct Potrf128<double> {
-  static void launch(double* A, int64_t lda, double* X, int64_t ldx, int32_t* info, int64_t g, hipStream_t st) {
-    hipLaunchKernelGGL(potrf128b_f64_kernel, dim3(1), dim3(1024), 0, st, A, lda, X, ldx, info, g);
-  }
-};
+// n: order of the matrix without its identity padding; g: the block's first column
+template <typename T>
+void potrf128(T* A, int64_t lda, T* X, int64_t ldx, int32_t* info, int64_t g, int64_t n, hipStream_t st) {
+  const int live = (int)std::max<int64_t>(0, std::min<int64_t>(DB, n - g));
+  if constexpr (sizeof(T) == 4)
+    hipLaunchKernelGGL(potrf128b_f32_kernel, dim3(1), dim3(GK_POTRF_NT), 0, st, A, lda, X, ldx, info, g, live);
+  else
+    hipLaunchKernelGGL(potrf128b_f64_kernel, dim3(1), dim3(GK_POTRF_NT), 0, st, A, lda, X, ldx, info, g, live);
+}
 
 template <typename T>
 __global__ void zero_block_kernel(T* X, int64_t ldx, int rows, int cols) {
@@ -1219,19 +1193,19 @@ __global__ __launch_bounds__(256) void diag_apply_kernel(const T* Dk, T* b) {
 // later step of the factorization reads it from A).  The upper-right quadrant
 // of Dinv is zeroed once per factorization by the caller.
 template <typename T>
-int diag256_chol(T* A, int64_t lda, int64_t k0, T* dinv, int32_t* dinfo, T* T1, T* T2, hipStream_t st,
+int diag256_chol(T* A, int64_t lda, int64_t n, int64_t k0, T* dinv, int32_t* dinfo, T* T1, T* T2, hipStream_t st,
                  bool copy_l21 = true) {
   T* A11 = A + k0 * lda + k0;
   T* A21 = A + (k0 + DB) * lda + k0;
   T* A22 = A21 + DB;
   T* D = dinv + k0 * NB;                 // 256 x 256, ld NB
-  Potrf128<T>::launch(A11, lda, D, NB, dinfo, k0, st);
+  potrf128<T>(A11, lda, D, NB, dinfo, k0, n, st);
   GK_TRY(gemm_launch<T>(DB, DB, DB, A21, lda, D, NB, true, T(1), T(0), T1, DB, false, st));        // L21
   if (copy_l21)
     hipLaunchKernelGGL(copy_block_kernel<T>, dim3(DB * DB / 256), dim3(256), 0, st, T1, (int64_t)DB, A21,
                        lda, (int64_t)DB, (int64_t)DB);
   GK_TRY(gemm_launch<T>(DB, DB, DB, T1, DB, T1, DB, true, T(-1), T(1), A22, lda, false, st));      // syrk
-  Potrf128<T>::launch(A22, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, st);
+  potrf128<T>(A22, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, n, st);
   GK_TRY(gemm_launch<T>(DB, DB, DB, T1, DB, D, NB, false, T(1), T(0), T2, DB, false, st));         // L21 X11
   GK_TRY(gemm_launch<T>(DB, DB, DB, D + DB * NB + DB, NB, T2, DB, false, T(-1), T(0), D + DB * NB, NB,
                         false, st));
@@ -1287,30 +1261,45 @@ extern "C" int gk_gemm_f64(gk_handle h, int64_t m, int64_t n, int64_t k, const d
                              (hipStream_t)stream);
 }
 
-// Recursive Cholesky (lower, row-major, in place) of the trailing principal
-// block of nblk 256-blocks at k0:
-//   chol(A11); A21 <- A21 L11^-T (recursive TRSM); A22 -= A21 A21^T; chol(A22).
-// Almost all flops land in GEMMs whose K is half the current order, where the
-// MFMA GEMM runs far closer to its peak than with 256-deep rank updates.
+// Lower-left quadrants of the inverses of nb diagonal blocks at once, the first
+// at A / dinv: Dinv21 = -X22 (L21 X11), two batched 128^3 products per block
+// (T: nb x DB x DB scratch).
 template <typename T>
+static int dinv_lower_left(const T* A, int64_t lda, T* dinv, int64_t nb, T* tmp, hipStream_t s) {
+  const int64_t sD = (int64_t)NB * NB;
+  if (nb == 0) return GK_OK;
+  GK_TRY(gemm_launch<T>(DB, DB, DB, A + DB * lda, lda, dinv, NB, false, T(1), T(0), tmp, DB, false, s, nb,
+                        (int64_t)NB * lda + NB, sD, (int64_t)DB * DB));
+  return gemm_launch<T>(DB, DB, DB, dinv + DB * NB + DB, NB, tmp, DB, false, T(-1), T(0), dinv + DB * NB, NB, false,
+                        s, nb, sD, (int64_t)DB * DB, sD);
+}
+
+// FP64 Cholesky (lower, row-major, in place) of the trailing principal block
+// of nblk 256-blocks at k0, recursive on halves:
+//   chol(A11); A21 <- A21 L11^-T (recursive TRSM); A22 -= A21 A21^T; chol(A22).
+// Almost all flops of a large matrix land in GEMMs whose K is half the
+// current order, where the MFMA GEMM runs far closer to its peak than with
+// 256-deep rank updates.  Blocks of at most LEAF 256-blocks are bound by the
+// latency of their panels instead and are factored right-looking (leaf).
 struct CholRec {
   gk_handle h;
-  T* A;
-  int64_t lda;
-  T* dinv;
+  double* A;
+  int64_t lda, n;
+  double* dinv;
   int32_t* dinfo;
-  T* W;            // lda x NB panel buffer
-  T* Tb;           // 2 DB x DB scratch of the diagonal-block kernel
-  hipStream_t st;
-  int64_t done = 0;      // diagonal blocks factored so far
+  double* W;             // lda x NB panel buffer
+  hipStream_t st, s2;
+  hipEvent_t* ev;
+  int64_t done = 0;      // diagonal blocks factored since the last look at the info word
   bool failed = false;
+  static constexpr int64_t LEAF = 16;
 
   // X <- X L^-T for X = A[r0:r0+m, c0:c0+nbk*NB], L = A[c0:, c0:] (nbk blocks)
   int trsm(int64_t r0, int64_t m, int64_t c0, int64_t nbk) {
     if (nbk == 1) {
-      GK_TRY(gemm_launch<T>(m, NB, NB, A + r0 * lda + c0, lda, dinv + c0 * NB, NB, true, T(1), T(0), W, NB, false,
-                            st));
-      hipLaunchKernelGGL(copy_block_kernel<T>, dim3((unsigned)gk_ceil_div(m * NB, 256)), dim3(256), 0, st, W,
+      GK_TRY(gemm_launch<double>(m, NB, NB, A + r0 * lda + c0, lda, dinv + c0 * NB, NB, true, 1.0, 0.0, W, NB, false,
+                                 st));
+      hipLaunchKernelGGL(copy_block_kernel<double>, dim3((unsigned)gk_ceil_div(m * NB, 256)), dim3(256), 0, st, W,
                          (int64_t)NB, A + r0 * lda + c0, lda, m, (int64_t)NB);
       return GK_OK;
     }
@@ -1318,30 +1307,85 @@ struct CholRec {
     const int64_t ca = c0, cb = c0 + a * NB;
     GK_TRY(trsm(r0, m, ca, a));
     // Xb -= Xa Lb^T, Lb = A[cb:cb+b NB, ca:ca+a NB]
-    GK_TRY(gemm_launch<T>(m, b * NB, a * NB, A + r0 * lda + ca, lda, A + cb * lda + ca, lda, true, T(-1), T(1),
-                          A + r0 * lda + cb, lda, false, st));
+    GK_TRY(gemm_launch<double>(m, b * NB, a * NB, A + r0 * lda + ca, lda, A + cb * lda + ca, lda, true, -1.0, 1.0,
+                               A + r0 * lda + cb, lda, false, st));
     return trsm(r0, m, cb, b);
+  }
+
+  // Panel kb of the leaf ending at row `end`, on stream s: with the halves 1,
+  // 2 of the 256-block and the rows below them b,
+  //   X11 = L11^-1;  [L21; W1] = [A21; Ab1] X11^T;  [A22; Ab2] -= [L21; W1] L21^T;
+  //   X22 = L22^-1;  W2 = Ab2 X22^T,
+  // in place on tiles spanning their 128 columns: five kernels in sequence.
+  int panel(int64_t k0, int64_t end, hipStream_t s) {
+    const int64_t rem = end - k0 - NB;
+    double* D = dinv + k0 * NB;                                    // 256 x 256, ld NB
+    double* C1 = A + (k0 + DB) * lda + k0;                         // [A21; Ab1]
+    potrf128<double>(A + k0 * lda + k0, lda, D, NB, dinfo, k0, n, s);
+    if (rem > 0 || k0 + DB < n) {          // (else the second half is padding: identity, and A21 = 0)
+      GK_TRY(gemm_launch<double>(DB + rem, DB, DB, C1, lda, D, NB, true, 1.0, 0.0, C1, lda, false, s, 1, 0, 0, 0, true));
+      GK_TRY(gemm_launch<double>(DB + rem, DB, DB, C1, lda, C1, lda, true, -1.0, 1.0, C1 + DB, lda, false, s));
+    }
+    potrf128<double>(C1 + DB, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, n, s);
+    if (rem > 0) {
+      double* C2 = A + (k0 + NB) * lda + k0 + DB;                  // Ab2
+      GK_TRY(gemm_launch<double>(rem, DB, DB, C2, lda, D + DB * NB + DB, NB, true, 1.0, 0.0, C2, lda, false, s, 1, 0, 0,
+                                 0, true));
+    }
+    return GK_OK;
+  }
+
+  // Right-looking with look-ahead: the chain (a panel, its product with the
+  // next block column, the next panel) runs on the side stream; the caller's
+  // stream applies each panel to the block columns after the next one beside
+  // the next panel.
+  int leaf(int64_t k0, int64_t nblk) {
+    const int64_t end = k0 + nblk * NB;
+    if (nblk == 1) {
+      GK_TRY(panel(k0, end, st));
+    } else {
+      GK_HIP(hipEventRecord(ev[0], st));
+      GK_HIP(hipStreamWaitEvent(s2, ev[0], 0));
+      GK_TRY(panel(k0, end, s2));
+      for (int64_t k = k0; k + NB < end; k += NB) {
+        const int64_t r = k + NB, rem = end - r;           // rows below the panel
+        double* W0 = A + r * lda + k;
+        GK_HIP(hipEventRecord(ev[1], s2));                 // panel k factored
+        if (k > k0) GK_HIP(hipStreamWaitEvent(s2, ev[2], 0));   // the previous panel's update of this column
+        GK_TRY(gemm_launch<double>(rem, NB, NB, W0, lda, W0, lda, true, -1.0, 1.0, A + r * lda + r, lda, false, s2));
+        GK_TRY(panel(r, end, s2));
+        if (rem > NB) {
+          GK_HIP(hipStreamWaitEvent(st, ev[1], 0));
+          GK_TRY(gemm_launch<double>(rem - NB, rem - NB, NB, W0 + NB * lda, lda, W0 + NB * lda, lda, true, -1.0, 1.0,
+                                     A + (r + NB) * lda + r + NB, lda, true, st));
+          GK_HIP(hipEventRecord(ev[2], st));
+        }
+      }
+      GK_HIP(hipEventRecord(ev[0], s2));
+      GK_HIP(hipStreamWaitEvent(st, ev[0], 0));
+    }
+    GK_TRY(dinv_lower_left<double>(A + k0 * lda + k0, lda, dinv + k0 * NB, nblk, W, st));
+    done += nblk;
+    if (done >= 8 && k0 + nblk * NB < lda) {               // stop early once a pivot has failed
+      done = 0;
+      int32_t hinfo = 0;
+      GK_HIP(hipMemcpyAsync(&hinfo, dinfo, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+      GK_HIP(hipStreamSynchronize(st));
+      failed = hinfo != 0;
+    }
+    return GK_OK;
   }
 
   int chol(int64_t k0, int64_t nblk) {
     if (failed) return GK_OK;
-    if (nblk == 1) {
-      GK_TRY(diag256_chol<T>(A, lda, k0, dinv, dinfo, Tb, Tb + DB * DB, st));
-      if (++done % 8 == 0) {          // stop early once a pivot has failed
-        int32_t hinfo = 0;
-        GK_HIP(hipMemcpyAsync(&hinfo, dinfo, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-        GK_HIP(hipStreamSynchronize(st));
-        failed = hinfo != 0;
-      }
-      return GK_OK;
-    }
+    if (nblk <= LEAF) return leaf(k0, nblk);
     const int64_t n1 = nblk / 2, n2 = nblk - n1;
     const int64_t k1 = k0 + n1 * NB;
     GK_TRY(chol(k0, n1));
     if (failed) return GK_OK;
     GK_TRY(trsm(k1, n2 * NB, k0, n1));
-    GK_TRY(gemm_launch<T>(n2 * NB, n2 * NB, n1 * NB, A + k1 * lda + k0, lda, A + k1 * lda + k0, lda, true, T(-1),
-                          T(1), A + k1 * lda + k1, lda, true, st));
+    GK_TRY(gemm_launch<double>(n2 * NB, n2 * NB, n1 * NB, A + k1 * lda + k0, lda, A + k1 * lda + k0, lda, true, -1.0,
+                               1.0, A + k1 * lda + k1, lda, true, st));
     return chol(k1, n2);
   }
 };
@@ -1351,10 +1395,10 @@ struct CholRec {
 // and solve the panel, W = A21 Dinv_kb^T.
 // With P given, the panel is also split into its tiled fp16 hi / lo form for
 // the split-fp16 updates.
-static int chol32_panel(float* A, int64_t lda, int64_t kb, float* dinv, int32_t* dinfo, float* W, float* Tb,
+static int chol32_panel(float* A, int64_t lda, int64_t n, int64_t kb, float* dinv, int32_t* dinfo, float* W, float* Tb,
                         hipStream_t s, _Float16* P = nullptr) {
   const int64_t k0 = kb * NB, rem = lda - k0 - NB;
-  GK_TRY(diag256_chol<float>(A, lda, k0, dinv, dinfo, Tb, Tb + DB * DB, s, false));
+  GK_TRY(diag256_chol<float>(A, lda, n, k0, dinv, dinfo, Tb, Tb + DB * DB, s, false));
   if (rem > 0) {
     GK_TRY(gemm_launch<float>(rem, NB, NB, A + (k0 + NB) * lda + k0, lda, dinv + k0 * NB, NB, true, 1.0f, 0.0f, W,
                               NB, false, s));
@@ -1373,16 +1417,16 @@ static int chol32_panel(float* A, int64_t lda, int64_t kb, float* dinv, int32_t*
 // all panels at the end (dinv_lower_left).  The products run in place in A
 // on tiles spanning their 128 columns, and W is split from A: six kernels in
 // sequence and no copies.
-static int chol32_panel_split(float* A, int64_t lda, int64_t kb, float* dinv, int32_t* dinfo, hipStream_t s,
+static int chol32_panel_split(float* A, int64_t lda, int64_t n, int64_t kb, float* dinv, int32_t* dinfo, hipStream_t s,
                               _Float16* P) {
   const int64_t k0 = kb * NB, rem = lda - k0 - NB;
   float* D = dinv + k0 * NB;                                     // 256 x 256, ld NB
   float* C1 = A + (k0 + DB) * lda + k0;                          // [A21; Ab1]
-  Potrf128<float>::launch(A + k0 * lda + k0, lda, D, NB, dinfo, k0, s);
+  potrf128<float>(A + k0 * lda + k0, lda, D, NB, dinfo, k0, n, s);
   GK_TRY(gemm_launch<float>(DB + rem, DB, DB, C1, lda, D, NB, true, 1.0f, 0.0f, C1, lda, false, s, 1, 0, 0, 0,
                             true));                              // [L21; W1], in place
   GK_TRY(gemm_launch<float>(DB + rem, DB, DB, C1, lda, C1, lda, true, -1.0f, 1.0f, C1 + DB, lda, false, s));
-  Potrf128<float>::launch(C1 + DB, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, s);
+  potrf128<float>(C1 + DB, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, n, s);
   if (rem > 0) {
     float* C2 = A + (k0 + NB) * lda + k0 + DB;                   // Ab2
     GK_TRY(gemm_launch<float>(rem, DB, DB, C2, lda, D + DB * NB + DB, NB, true, 1.0f, 0.0f, C2, lda, false, s, 1, 0, 0,
@@ -1390,18 +1434,6 @@ static int chol32_panel_split(float* A, int64_t lda, int64_t kb, float* dinv, in
     GK_TRY(split_h3(A + (k0 + NB) * lda + k0, rem, P, s, lda));
   }
   return GK_OK;
-}
-
-// Lower-left quadrants of the diagonal blocks' inverses, all panels at once:
-// Dinv21 = -X22 (L21 X11), two batched 128^3 products per panel (T: nb x DB x
-// DB scratch).
-static int dinv_lower_left(const float* A, int64_t lda, float* dinv, float* T, hipStream_t s) {
-  const int64_t nb = lda / NB, sD = (int64_t)NB * NB;
-  if (nb == 0) return GK_OK;
-  GK_TRY(gemm_launch<float>(DB, DB, DB, A + DB * lda, lda, dinv, NB, false, 1.0f, 0.0f, T, DB, false, s, nb,
-                            (int64_t)NB * lda + NB, sD, (int64_t)DB * DB));
-  return gemm_launch<float>(DB, DB, DB, dinv + DB * NB + DB, NB, T, DB, false, -1.0f, 0.0f, dinv + DB * NB, NB, false,
-                            s, nb, sD, (int64_t)DB * DB, sD);
 }
 
 // Chain planes of the triangular solves (planes of lda x 256, D =
@@ -1472,11 +1504,12 @@ static int cholesky_impl(gk_handle h, T* A, int64_t n, int64_t lda, T* dinv, int
     const int64_t tot = (lda - n) * lda + n * (lda - n);
     hipLaunchKernelGGL(pad_identity_kernel<T>, dim3((unsigned)gk_ceil_div(tot, 256)), dim3(256), 0, st, A, lda, n);
   }
-  if (sizeof(T) == 8) {
-    if (nb > 0) {
-      CholRec<T> R{h, A, lda, dinv, dinfo, W, Tb, st};
-      GK_TRY(R.chol(0, nb));
-    }
+  if constexpr (sizeof(T) == 8) {
+    hipStream_t s2;
+    hipEvent_t* ev;
+    GK_TRY(gk_side_stream(h, &s2, &ev));
+    CholRec R{h, A, lda, n, dinv, dinfo, W, st, s2, ev};
+    if (nb > 0) GK_TRY(R.chol(0, nb));
   } else {
     // FP32: right-looking order.  Each rank-256 update rounds the trailing
     // block relative to the Schur complement as it shrinks, which a one-shot
@@ -1508,8 +1541,8 @@ static int cholesky_impl(gk_handle h, T* A, int64_t n, int64_t lda, T* dinv, int
       // split form in sp(kb)); without split16 the copies back into A follow
       auto panel = [&](int64_t kb) -> int {
         T* V = Wb[kb & 1];
-        if (split16) GK_TRY(chol32_panel_split(A, lda, kb, dinv, dinfo, s2, sp(kb)));
-        else GK_TRY(chol32_panel(A, lda, kb, dinv, dinfo, V, Tb, s2));
+        if (split16) GK_TRY(chol32_panel_split(A, lda, n, kb, dinv, dinfo, s2, sp(kb)));
+        else GK_TRY(chol32_panel(A, lda, n, kb, dinv, dinfo, V, Tb, s2));
         GK_HIP(hipEventRecord(ev[1], s2));
         if (split16) return GK_OK;
         return chol32_panel_post(A, lda, kb, V, Tb, s2);
@@ -1573,7 +1606,7 @@ static int cholesky_impl(gk_handle h, T* A, int64_t n, int64_t lda, T* dinv, int
       }
       GK_HIP(hipEventRecord(ev[2], s2));
       GK_HIP(hipStreamWaitEvent(st, ev[2], 0));
-      if (split16) GK_TRY(dinv_lower_left(A, lda, dinv, Wb[0], st));
+      if (split16) GK_TRY(dinv_lower_left<float>(A, lda, dinv, nb, Wb[0], st));
     }
   }
   GK_TRY(chain_planes<T>(A, lda, dinv, st));   // chain planes of the triangular solves
