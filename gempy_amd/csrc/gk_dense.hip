@@ -826,33 +826,43 @@ __global__ __launch_bounds__(1024) void getrf128_kernel(double* A, int64_t lda, 
 }
 
 // Blocked Cholesky + inverse of a DB x DB block (one workgroup of NT threads),
-// two barriers per PB = 16 columns.  Phase 1 (wave 0, registers, lane values
-// broadcast through scalar registers): factor the 16-column panel, while the
-// other waves apply the previous panel to the rows of X = L^-1 below it.
-// Phase 2: the last two waves form the panel's 16 rows of X,
-//   X[i][c] = (delta_ic - acc[i][c] - sum_{jb<=k<i} L[i][k] X[k][c]) / L[i][i],
-// where acc[i][c] = sum_{k<jb} L[i][k] X[k][c] was applied eagerly, and the
-// other waves apply the panel to the trailing tiles of L and write the
-// panel to A.
+// two barriers per PB = 16 columns, bound by the latency of its steps.  Step s:
+//   phase A, a 16 x 16 tile per wave on MFMA: panel s into the columns of
+//     panel s + 1, and panel s - 1 into the rows of X = L^-1 of panel s;
+//   phase B: waves 0-2 factor panel s + 1 in registers (each the panel's 16
+//     diagonal rows and up to 48 rows below them, lane values broadcast
+//     through scalar registers); the last two waves form the rows of X of
+//     panel s,
+//       X[i][c] = (delta_ic - acc[i][c] - sum_{jb<=k<i} L[i][k] X[k][c]) / L[i][i],
+//     where acc[i][c] = sum_{k<jb} L[i][k] X[k][c] was applied eagerly; the
+//     others write panel s of L to A; and all but the first take the other
+//     tiles of L under panel s and of X under panel s - 1.
 // LDS: one packed lower triangle S.  Row i holds X (or -acc) in the columns
 // already factored and the trailing matrix in the others: a column of L is
-// dead there once its panel is factored, which is when X needs its place.
-// Two panel buffers P[b] hold the 16 columns of the current / next panel
-// column-major (P[b][t][i] = L[i][jb + t]): wave 0 loads its panel rows
-// without per-row branches (16% less time in phase 1 than from the packed
-// rows) and the tiles read the panel with consecutive addresses.  FP32
-// 48.5 KB, FP64 97 KB (two triangles and 16-column panels would need 161 KB
-// in FP64, more than a CU has).
+// dead there once its panel is factored, before X needs its place.  Three
+// panel buffers P[b] hold the 16 columns of panels s - 1, s and s + 1
+// column-major (P[b][t][i] = L[i][jb + t], columns 144 apart for the banks):
+// panel rows are loaded without per-row branches and the tiles read the panel
+// with consecutive addresses.  FP32 61 KB, FP64 122 KB (two triangles and two
+// panels would need 161 KB in FP64, more than a CU has).  Measured cycle by
+// cycle (FP64): with branches per element a tile took 2,100 cycles, the block
+// load 19,000 and the whole 73 us; with masked accesses, the pivot chain beside
+// the column updates and the tiles beside the next panel 48 us (FP32 42 -> 34).
 constexpr int GK_POTRF_PB = 16;
 template <typename T>
 struct BlkStore {
   static constexpr int PB = GK_POTRF_PB;
   T* S;
-  static constexpr int SIZE = DB * (DB + 1) / 2 + 2 * PB * DB + PB;
-  __device__ static int pl(int i, int c) { return i * (i + 1) / 2 + c; }
+  static constexpr int PS = DB + 16;          // column stride of the panel buffers
+  static constexpr int TRI = DB * (DB + 1) / 2, IPV = TRI + 3 * PB * PS, SPARE = IPV + 2 * PB;
+  static constexpr int SIZE = SPARE + 64 + 2;
+  __device__ static int pl(int i, int c) { return (int)__umul24(i, i + 1) / 2 + c; }
+  __device__ static int po(int b, int t, int i) { return TRI + (b * PB + t) * PS + i; }
   __device__ T& V(int i, int c) { return S[pl(i, c)]; }
-  __device__ T& P(int b, int t, int i) { return S[DB * (DB + 1) / 2 + (b * PB + t) * DB + i]; }
-  __device__ T& ipv(int j) { return S[DB * (DB + 1) / 2 + 2 * PB * DB + j]; }   // 1 / pivot of the current panel
+  __device__ T& P(int b, int t, int i) { return S[po(b, t, i)]; }
+  __device__ T& ipv(int s, int j) { return S[IPV + (s & 1) * PB + j]; }     // 1 / pivot j of panel s
+  __device__ int spare() const { return SPARE + (threadIdx.x & 63); }       // where masked stores go
+  __device__ int* next() { return reinterpret_cast<int*>(&S[SPARE + 64]); }  // next tile of phase B
 };
 // Threads of the diagonal-block kernels: 8 waves, so that wave 0 may hold its
 // panel rows in registers (FP64: 64 VGPRs of them; 16 waves would leave 128
@@ -871,23 +881,39 @@ __device__ __forceinline__ double lane_value(double v, int l) {
   return __hiloint2double(hi, lo);
 }
 
-// Pivot d > 0 -> (sqrt(d), 1/sqrt(d)).  FP32: the hardware reciprocal square
-// root (within 1 ulp), the factor being an FP32 preconditioner.  FP64: the
-// hardware seed, two Newton steps, then one residual step each for the root
-// and the reciprocal (both within 1 ulp; a chain of 9 dependent FMAs where the
-// IEEE square root and division take several times that).
-__device__ __forceinline__ void pivot_pair(float d, float& piv, float& ip) {
-  ip = __builtin_amdgcn_rsqf(d);
-  piv = d * ip;
-}
-__device__ __forceinline__ void pivot_pair(double d, double& piv, double& ip) {
-  double y = __builtin_amdgcn_rsq(d);
-  y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
-  y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
-  const double s = d * y;
-  piv = fma(0.5 * y, fma(-s, s, d), s);
-  ip = fma(y, fma(-piv, y, 1.0), y);
-}
+// Pivot d > 0 -> (sqrt(d), 1/sqrt(d)), one dependent operation per call of
+// step(), so that the caller can place other work between them.  FP32: the
+// hardware reciprocal square root (within 1 ulp), the factor being an FP32
+// preconditioner.  FP64: the hardware seed (2^-24), one Newton step (2^-47),
+// then one residual step each for the root and the reciprocal, which leaves
+// both within 1 ulp: a chain of 9 operations where the IEEE square root and
+// division take several times that.
+template <typename T> struct PivotChain;
+template <> struct PivotChain<float> {
+  static constexpr int STEPS = 2;
+  float d, piv, ip;
+  __device__ __forceinline__ void step(int k) {
+    if (k == 0) ip = __builtin_amdgcn_rsqf(d);
+    else piv = d * ip;
+  }
+};
+template <> struct PivotChain<double> {
+  static constexpr int STEPS = 9;
+  double d, piv, ip, y, h, e;
+  __device__ __forceinline__ void step(int k) {
+    switch (k) {
+      case 0: y = __builtin_amdgcn_rsq(d); break;
+      case 1: e = -d * y; h = 0.5 * y; break;
+      case 2: e = fma(e, y, 1.0); break;
+      case 3: y = fma(h, e, y); break;
+      case 4: piv = d * y; h = 0.5 * y; break;
+      case 5: e = fma(-piv, piv, d); break;
+      case 6: piv = fma(h, e, piv); break;
+      case 7: e = fma(-piv, y, 1.0); break;
+      default: ip = fma(y, e, y); break;
+    }
+  }
+};
 
 __device__ __forceinline__ f4v mma4(float a, float b, f4v c) { return Mfma<float>::mma(a, b, c); }
 __device__ __forceinline__ d4v mma4(double a, double b, d4v c) { return Mfma<double>::mma(a, b, c); }
@@ -899,203 +925,234 @@ __device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ld
                               int live) {
   constexpr int PB = GK_POTRF_PB;
   using acc_t = typename Mfma<T>::acc_t;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // all loads of the block first (in flight together, 16 bytes each), then
-  // the LDS stores
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int NW = NT / 64;
   constexpr int VL = 16 / sizeof(T);          // elements per 16-byte load
+  typedef T vt __attribute__((ext_vector_type(VL)));
+  // the whole block (in flight together, 16 bytes per load), then the LDS
+  // stores; entries above the diagonal go to the spare slots
   constexpr int PER = DB * DB / (NT * VL);
   static_assert(PER * NT * VL == DB * DB, "the block must be a whole number of vectors per thread");
-  typedef T vt __attribute__((ext_vector_type(VL)));
   vt vin[PER];
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
-    const int e = (tid + q * NT) * VL, i = e / DB, c = e % DB;
-    if (c <= i) vin[q] = *reinterpret_cast<const vt*>(A + i * lda + c);
-    else
-#pragma unroll
-      for (int u = 0; u < VL; ++u) vin[q][u] = T(0);
+    const int e = (tid + q * NT) * VL;
+    vin[q] = *reinterpret_cast<const vt*>(A + (e / DB) * lda + e % DB);
   }
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
     const int e = (tid + q * NT) * VL, i = e / DB, c = e % DB;
 #pragma unroll
-    for (int u = 0; u < VL; ++u) {
-      if (c + u <= i) {
-        B.V(i, c + u) = vin[q][u];
-        if (c + u < PB) B.P(0, c + u, i) = vin[q][u];
-      }
+    for (int u = 0; u < VL; ++u) B.S[c + u <= i ? B.pl(i, c + u) : B.spare()] = vin[q][u];
+    if (c < PB) {                             // (a multiple of VL)
+#pragma unroll
+      for (int u = 0; u < VL; ++u) B.P(0, c + u, i) = vin[q][u];
     }
   }
   __syncthreads();
-  const int nlive = min(DB, (live + PB - 1) / PB * PB);   // rows and columns that are factored
+  const int nlive = min(DB, (live + PB - 1) / PB * PB), steps = nlive / PB;   // what is factored
   int bad_col = 0;                            // first non-positive pivot + 1 (wave 0)
-  constexpr int NW = NT / 64, XW = NW - 2;    // phase 2: waves XW, XW + 1 form the X rows
-  // rows jb .. jb+PB-1 of X from the panel's diagonal block in P[pb] (LDS
-  // broadcasts), one column per lane (c = lane + coff).  Right-looking: row k
-  // is final once the rows above it are applied, and then goes into every
-  // later row (each row takes the same products in the same order as a
-  // row-by-row substitution; the dependent chain is 16 steps, not 120).
-  auto x_rows = [&](int jb, int pb, int coff) {
-    T x[PB], col[2][PB];
-    const int c = lane + coff;
-    if (c >= jb + PB) return;
+  const int lr = lane & 15, lq = lane >> 4;
+
+  // panel s: wave w (0..2) holds the diagonal rows in lanes 0-15 and rows
+  // jb + 16 + 48 w + (lane - 16) in the others
+  auto panel = [&](int s, int w) {
+    const int jb = s * PB, pb = s % 3;
+    const int r = lane < PB ? jb + lane : jb + 48 * w + lane;
+    const int rc = min(r, DB - 1);
+    T a[PB];
+#pragma unroll
+    for (int c = 0; c < PB; ++c) {
+      const T v = B.P(pb, c, rc);
+      a[c] = c <= r - jb ? v : T(0);
+    }
+    PivotChain<T> pv;
+    auto start = [&](int j) {                 // the pivot of column j (held by lane j), made positive
+      T d = lane_value(a[j], j);
+      const bool bad = !(d > T(0));
+      bad_col = bad && bad_col == 0 ? jb + j + 1 : bad_col;
+      pv.d = bad ? T(1) : d;
+    };
+    start(0);
+#pragma unroll
+    for (int k = 0; k < pv.STEPS; ++k) pv.step(k);
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      const T piv = pv.piv, ip = pv.ip;
+      if (w == 0) B.ipv(s, j) = ip;           // every lane the same value
+      const T aj = lane > j ? a[j] * ip : T(0);
+      // column j below the diagonal (0 on and above it) goes into the later
+      // columns unmasked: the next one first, whose pivot chain then runs
+      // beside the updates of the others
+      if (j + 1 < PB) {
+        a[j + 1] -= aj * lane_value(aj, j + 1);
+        start(j + 1);
+      }
+      int k = 0;
+#pragma unroll
+      for (int c = j + 2; c < PB; ++c) {
+        a[c] -= aj * lane_value(aj, c);       // L[jb+c][jb+j]
+        if (k < pv.STEPS) pv.step(k++);
+      }
+      if (j + 1 < PB) {
+#pragma unroll
+        for (; k < pv.STEPS; ++k) pv.step(k);
+      }
+      a[j] = lane == j ? piv : (lane > j ? aj : a[j]);
+    }
+    if (r < DB && (lane >= PB || w == 0)) {
+#pragma unroll
+      for (int c = 0; c < PB; ++c) B.P(pb, c, r) = a[c];
+    }
+  };
+
+  // rows jb .. jb+PB-1 of X from the diagonal block of panel s (LDS
+  // broadcasts of 16 bytes), one column per lane (c = lane + coff).
+  // Right-looking: row k is final once the rows above it are applied, and
+  // then goes into every later row (each row takes the same products in the
+  // same order as a row-by-row substitution; the dependent chain is 16 steps,
+  // not 120).
+  auto x_rows = [&](int s, int coff) {
+    const int jb = s * PB, pb = s % 3, c = lane + coff;
+    T x[PB], ipv[PB];
+    vt col[2][PB / VL];
 #pragma unroll
     for (int r = 0; r < PB; ++r) {
-      const int i = jb + r;
-      const T v = B.V(i, min(c, jb));                     // -acc[i][c] for c < jb
-      x[r] = c < jb ? v : (c == i ? T(1) : T(0));
-      col[0][r] = r > 0 ? B.P(pb, 0, i) : B.ipv(0);
+      const T v = B.V(jb + r, min(c, jb));                // -acc[i][c] for c < jb
+      x[r] = c < jb ? v : (c == jb + r ? T(1) : T(0));
     }
-    // column k + 1 of the panel (and its reciprocal pivot, in place of the
-    // diagonal) is read beside step k; the barrier keeps later columns out of
-    // the registers
 #pragma unroll
-    for (int k = 0; k < PB; ++k) {
-      const T (&lk)[PB] = col[k & 1];
+    for (int r = 0; r < PB; r += VL) {
+      const vt v = *reinterpret_cast<const vt*>(&B.ipv(s, r));
+#pragma unroll
+      for (int u = 0; u < VL; ++u) ipv[r + u] = v[u];
+      col[0][r / VL] = *reinterpret_cast<const vt*>(&B.P(pb, 0, jb + r));
+    }
+#pragma unroll
+    for (int k = 0; k < PB; ++k) {            // the next column is read beside step k
       if (k + 1 < PB) {
 #pragma unroll
-        for (int r = k + 1; r < PB; ++r) col[(k + 1) & 1][r] = r > k + 1 ? B.P(pb, k + 1, jb + r) : B.ipv(r);
+        for (int r = (k + 2) / VL * VL; r < PB; r += VL)
+          col[(k + 1) & 1][r / VL] = *reinterpret_cast<const vt*>(&B.P(pb, k + 1, jb + r));
       }
-      x[k] *= lk[k];
+      x[k] *= ipv[k];
 #pragma unroll
-      for (int r = k + 1; r < PB; ++r) x[r] -= lk[r] * x[k];   // L[jb+r][jb+k]
+      for (int r = k + 1; r < PB; ++r) x[r] -= col[k & 1][r / VL][r % VL] * x[k];   // L[jb+r][jb+k]
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int r = 0; r < PB; ++r)
-      if (c <= jb + r) B.V(jb + r, c) = x[r];
+    for (int r = 0; r < PB; ++r) B.S[c <= jb + r ? B.pl(jb + r, c) : B.spare()] = x[r];
   };
-  // rank-16 updates on MFMA (16 x 16 x 4), one 16 x 16 tile per wave at a time
-  // (waves w, w + nw, ...), by the panel of columns jb = c0 - 16:
-  //   L tiles (ti >= tj >= c0/16):  L[i][c] -= sum_t L[i][jb+t] L[c][jb+t]
-  //   X tiles (ti >= c0/16 > tj):   X[i][c] -= sum_t L[i][jb+t] X[jb+t][c]
-  // Operands from the column-major panel buffer P[pb] (and the packed X rows
-  // of the panel).  The X tiles of the panel's own columns start from 0.  A
-  // lane holds column lane % 16 of a tile, its rows 4 (lane/16) + r (f32) or
-  // lane/16 + 4 r (f64).
-  auto mfma_tiles = [&](int c0, int pb, bool is_l, int w, int nw) {
-    const int jb = c0 - PB, a = c0 / 16, nt = nlive / 16 - a;   // first trailing tile row, tile rows left
-    const int count = is_l ? nt * (nt + 1) / 2 : nt * a;
-    const int lr = lane & 15, lq = lane >> 4;
-    for (int tile = w; tile < count; tile += nw) {
-      int ti, tj;
-      if (is_l) {                                         // lower triangle of the trailing tiles
-        int t = tile, r = 0;
-        while (t > r) { t -= r + 1; ++r; }
-        ti = a + r;
-        tj = a + t;
-      } else {
-        ti = a + tile / a;
-        tj = tile % a;
-      }
-      const int i0 = ti * 16, cb = tj * 16;
-      acc_t acc;
+
+  // panel s of L into A (thread t of nt): its diagonal tile, then the rows below
+  auto write_panel = [&](int s, int t, int nt) {
+    const int jb = s * PB, pb = s % 3;
+    for (int e = t; e < PB * PB; e += nt) {
+      const int r = e / PB, c = e % PB;
+      if (c <= r) A[(jb + r) * lda + jb + c] = B.P(pb, c, jb + r);
+    }
+    for (int e = t; e < (nlive - jb - PB) * (PB / VL); e += nt) {
+      const int i = jb + PB + e / (PB / VL), c = e % (PB / VL) * VL;
+      vt v;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + (sizeof(T) == 8 ? lq + 4 * r : lq * 4 + r), c = cb + lr;
-        acc[r] = is_l ? (c <= i ? B.V(i, c) : T(0)) : (tj == a - 1 ? T(0) : B.V(i, c));
-      }
-#pragma unroll
-      for (int ks = 0; ks < PB / 4; ++ks) {
-        const int t = ks * 4 + lq;
-        const T av = -B.P(pb, t, i0 + lr);                // A[row][k] = L[i0+lr][jb+t]
-        T bv;
-        if (is_l) bv = B.P(pb, t, cb + lr);               // B[k][col] = L[cb+lr][jb+t]
-        else bv = (cb + lr <= jb + t) ? B.V(jb + t, cb + lr) : T(0);
-        acc = mma4(av, bv, acc);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + (sizeof(T) == 8 ? lq + 4 * r : lq * 4 + r), c = cb + lr;
-        if (is_l) {
-          if (c <= i) {
-            B.V(i, c) = acc[r];
-            if (c < c0 + PB) B.P(pb ^ 1, c - c0, i) = acc[r];
-          }
-        } else {
-          B.V(i, c) = acc[r];
-        }
-      }
+      for (int u = 0; u < VL; ++u) v[u] = B.P(pb, c + u, i);
+      *reinterpret_cast<vt*>(A + i * lda + jb + c) = v;
     }
   };
-  for (int jb = 0, pb = 0; jb < nlive; jb += PB, pb ^= 1) {
-    // the previous panel's X tiles beside this panel (they touch only X,
-    // which the panel does not read)
-    if (wave > 0 && jb > 0) mfma_tiles(jb, pb ^ 1, false, wave - 1, NW - 1);
-    if (wave == 0) {
-      // ---- panel: lane l holds rows jb + l (a) and jb + 64 + l (b)
-      const int ra = jb + lane, rb = jb + 64 + lane;
-      const int rac = min(ra, DB - 1), rbc = min(rb, DB - 1);
-      T a[PB], b[PB];
+
+  // a 16 x 16 tile of L (rows ti >= columns tj, both past panel p),
+  //   L[i][c] -= sum_t L[i][jb+t] L[c][jb+t]
+  // (copied into buffer `to` when it holds the next panel's columns), or of X
+  // (rows past panel p, columns up to it),
+  //   X[i][c] -= sum_t L[i][jb+t] X[jb+t][c],
+  // which starts from 0 in the panel's own columns.  A lane holds column
+  // lane % 16 of a tile, its rows 4 (lane/16) + r (f32) or lane/16 + 4 r (f64).
+  auto tile = [&](bool is_l, int p, int ti, int tj, int to) {
+    constexpr int RD = sizeof(T) == 8 ? 4 : 1;                   // distance of a lane's rows
+    const int i0 = ti * 16 + (sizeof(T) == 8 ? lq : lq * 4), c = tj * 16 + lr, pb = p % 3, xb = p * PB;
+    acc_t acc;
+    T av[PB / 4], bv[PB / 4];
+    const int pa = B.po(pb, lq, ti * 16 + lr);
+    const int b0 = is_l ? B.po(pb, lq, c) : 0;
+    int xr = xb + lq, xo = B.pl(xr, 0);                          // X rows xb + lq + 4 ks
 #pragma unroll
-      for (int c = 0; c < PB; ++c) {
-        const T va = B.P(pb, c, rac), vb = B.P(pb, c, rbc);
-        a[c] = (ra < DB && jb + c <= ra) ? va : T(0);
-        b[c] = rb < DB ? vb : T(0);
-      }
-      // column j below the diagonal (aj, 0 on and above it) goes into the later
-      // columns unmasked; the rows jb + 64 + l exist only while jb < 64
-      auto factor = [&](auto with_b) {
+    for (int ks = 0; ks < PB / 4; ++ks) {
+      av[ks] = -B.S[pa + 4 * ks * B.PS];                         // A[row][k] = L[ti 16 + lr][jb+t]
+      const T v = B.S[is_l ? b0 + 4 * ks * B.PS : xo + min(c, xr)];   // B[k][col]
+      bv[ks] = is_l || c <= xr ? v : T(0);
+      xo += 4 * xr + 10;
+      xr += 4;
+    }
+    int row[4];                                                  // offsets of the lane's rows
+    row[0] = B.pl(i0, 0);
 #pragma unroll
-        for (int j = 0; j < PB; ++j) {
-          T d = lane_value(a[j], j);              // L[jb+j][jb+j], held by lane j
-          if (!(d > T(0))) {
-            if (bad_col == 0) bad_col = jb + j + 1;
-            d = T(1);
-          }
-          T piv, ip;
-          pivot_pair(d, piv, ip);
-          B.ipv(j) = ip;                          // every lane the same value
-          const T aj = lane > j ? a[j] * ip : T(0);
-          if constexpr (decltype(with_b)::value) b[j] *= ip;
+    for (int r = 1; r < 4; ++r) row[r] = row[r - 1] + RD * (i0 + RD * (r - 1)) + RD * (RD + 1) / 2;
 #pragma unroll
-          for (int c = j + 1; c < PB; ++c) {
-            const T lcj = lane_value(aj, c);      // L[jb+c][jb+j]
-            a[c] -= aj * lcj;
-            if constexpr (decltype(with_b)::value) b[c] -= b[j] * lcj;
-          }
-          a[j] = lane == j ? piv : (lane > j ? aj : a[j]);
-        }
-      };
-      if (jb < 64) factor(std::true_type{});
-      else factor(std::false_type{});
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + RD * r;
+      const T v = B.S[row[r] + min(c, i)];
+      acc[r] = (is_l ? c > i : tj == p) ? T(0) : v;
+    }
 #pragma unroll
-      for (int c = 0; c < PB; ++c) {
-        if (ra < DB) B.P(pb, c, ra) = a[c];
-        if (rb < DB) B.P(pb, c, rb) = b[c];
+    for (int ks = 0; ks < PB / 4; ++ks) acc = mma4(av[ks], bv[ks], acc);
+    if (to >= 0) {                                               // the next panel's columns live in its buffer
+#pragma unroll
+      for (int r = 0; r < 4; ++r) B.P(to, lr, i0 + RD * r) = acc[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) B.S[c <= i0 + RD * r ? row[r] + c : B.spare()] = acc[r];
+    }
+  };
+
+  if (wave < 3 && steps > 0) panel(0, wave);
+  __syncthreads();
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    const int nt = steps - s - 1;             // tile rows past panel s
+    if (wave < nt) tile(true, s, s + 1 + wave, s + 1, (s + 1) % 3);
+    else if (wave < nt + s) tile(false, s - 1, s, wave - nt, -1);
+    if (tid == 0) *B.next() = 0;
+    __syncthreads();
+    if (wave < 3) {
+      if (nt > 0) panel(s + 1, wave);
+    } else if (wave >= NW - 2) {
+      x_rows(s, (wave - (NW - 2)) * 64);
+    } else {
+      write_panel(s, tid - 192, NT - 320);
+    }
+    // the other tiles, drawn from a counter: L (ti >= tj >= s + 2), then X (ti > s)
+    const int nl = nt * (nt - 1) / 2, all = nl + nt * s;
+    const float inv = __builtin_amdgcn_rcpf((float)max(s, 1));
+    while (wave > 0) {
+      int q = 0;
+      if (lane == 0) q = atomicAdd(B.next(), 1);
+      q = __builtin_amdgcn_readfirstlane(q);
+      if (q >= all) break;
+      if (q < nl) {                           // row r of the triangle: r (r + 1) / 2 <= q
+        const int r = (int)(0.5f * __builtin_amdgcn_sqrtf(8.0f * q + 1.01f) - 0.5f);
+        tile(true, s, s + 2 + r, s + 2 + q - r * (r + 1) / 2, -1);
+      } else {
+        const int r = (int)((q - nl + 0.5f) * inv);
+        tile(false, s - 1, s + 1 + r, q - nl - r * s, -1);
       }
     }
     __syncthreads();
-    if (wave >= XW) {
-      x_rows(jb, pb, wave == XW ? 0 : 64);
-    } else {
-      mfma_tiles(jb + PB, pb, true, wave, XW);
-      // the panel's columns of L into A: its diagonal tile, then the rows below
-      if (tid < PB * PB) {
-        const int r = tid / PB, c = tid % PB;
-        if (c <= r) A[(jb + r) * lda + jb + c] = B.P(pb, c, jb + r);
-      }
-      for (int e = tid; e < (nlive - jb - PB) * (PB / VL); e += XW * 64) {
-        const int i = jb + PB + e / (PB / VL), c = e % (PB / VL) * VL;
-        vt v;
-#pragma unroll
-        for (int u = 0; u < VL; ++u) v[u] = B.P(pb, c + u, i);
-        *reinterpret_cast<vt*>(A + i * lda + jb + c) = v;
-      }
-    }
-    __syncthreads();                          // (the last panel has no X tiles)
   }
   if (wave == 0 && lane == 0 && bad_col != 0) atomicCAS(info, 0, (int32_t)(gbase + bad_col));
+#pragma unroll 4
   for (int e = tid * VL; e < DB * DB; e += NT * VL) {
     const int i = e / DB, c = e % DB;
     vt x;
 #pragma unroll
-    for (int u = 0; u < VL; ++u) x[u] = i >= nlive ? (c + u == i ? T(1) : T(0)) : (c + u <= i ? B.V(i, c + u) : T(0));
+    for (int u = 0; u < VL; ++u) {
+      const T v = B.V(i, min(c + u, i));
+      x[u] = i >= nlive ? (c + u == i ? T(1) : T(0)) : (c + u <= i ? v : T(0));
+    }
     *reinterpret_cast<vt*>(X + i * ldx + c) = x;
   }
 }
 
-// FP32: 48.5 KB of LDS, so the kernel fits on a CU beside a workgroup of the
+// FP32: 61 KB of LDS, so the kernel fits on a CU beside a workgroup of the
 // concurrent trailing update (the look-ahead factorization runs it on a
 // second stream).
 __global__ __launch_bounds__(GK_POTRF_NT) void potrf128b_f32_kernel(float* A, int64_t lda, float* X, int64_t ldx,
