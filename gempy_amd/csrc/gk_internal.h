@@ -77,6 +77,8 @@ struct gk_context {
   char* eval_scratch = nullptr;
   // where the marching-cubes case tables were last uploaded (inside WS_MESH)
   void* mesh_tables = nullptr;
+  // pinned pair of counts that the isosurface extraction's kernels write
+  uint32_t* mesh_counts = nullptr;
 };
 
 // Takes the device address of the evaluation scratch array for h's device

@@ -15,8 +15,14 @@
 // loop is triangulated as a fan.  Triangles wind so that their normals
 // (right-hand rule) point towards increasing field values.
 //
-// Passes: classify cubes (case byte, triangle count, used-edge flags) ->
-// exclusive scans (vertex ids, face offsets) -> vertex positions -> faces.
+// The field is read once: a first pass packs every z row into words of 64
+// points (above the level, NaN, masked), and everything that follows works on
+// those words - 3/64 of a byte per point and flag - until the crossed edges
+// and the cubes with triangles, few and known, are written.  What it is bound
+// by is that one read (8 bytes a point, 9 with a mask).  Per-point flags, edge
+// ids and cube cases in memory with scans over them moved about 500 bytes a
+// point: 200^3 cells with a mask took 400 us so and take 90 us now, of which the
+// packing 26 us (72 MB, 2.8 TB/s) and the writing pass 35 us.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -129,139 +135,287 @@ McTables build_tables() {
 struct McArgs {
   const double* f;
   const uint8_t* mask;
-  int64_t nx, ny, nz;
+  int64_t nx, ny, nz, W, words;        // W words of 64 points per z row, words = nx ny W
   double level;
   const McTables* T;
+  uint64_t *above, *nan, *msk;         // bit z: value > level / NaN / mask set
+  uint64_t *valid;                     // bit z: cube (x, y, z) is meshed
+  uint64_t *edge[3];                   // bit z: a meshed cube uses the edge from (x, y, z) along the axis
+  uint32_t *vpre, *tpre;               // vertices / triangles of the block's earlier words
+  uint32_t *vsum, *tsum;               // vertices / triangles of each block of MC_WORDS words, then of the earlier ones
+  uint32_t *total;                     // both, of all words
 };
 
-__device__ __forceinline__ int64_t pidx(const McArgs& a, int64_t x, int64_t y, int64_t z) {
-  return (x * a.ny + y) * a.nz + z;
-}
+constexpr int MC_WORDS = 256;          // words (threads) per counting block
+constexpr int MC_PER_WAVE = 8;         // words a wave packs: that many loads in flight
 
-// global edge of local edge e of cube (x, y, z): 3 * point + axis
-__device__ __forceinline__ int64_t gedge(const McArgs& a, int64_t x, int64_t y, int64_t z, int e) {
-  const int axis = e >> 2, k = e & 3;
-  int o[3] = {0, 0, 0}, j = 0;
-  for (int d = 0; d < 3; ++d)
-    if (d != axis) o[d] = (k >> j++) & 1;
-  return 3 * pidx(a, x + o[0], y + o[1], z + o[2]) + axis;
-}
-
-__global__ void mc_classify_kernel(McArgs a, uint8_t* cases, uint32_t* ntri, uint32_t* eflag) {
-  const int64_t ncx = a.nx - 1, ncy = a.ny - 1, ncz = a.nz - 1;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncx * ncy * ncz) return;
-  const int64_t z = c % ncz, y = (c / ncz) % ncy, x = c / (ncz * ncy);
-  int cs = 0;
-  // a cube is meshed when the mask is set at its far corner (+1, +1, +1)
-  bool ok = !a.mask || a.mask[pidx(a, x + 1, y + 1, z + 1)];
-  if (ok) {
-    for (int k = 0; k < 8; ++k) {
-      const double v = a.f[pidx(a, x + (k & 1), y + ((k >> 1) & 1), z + ((k >> 2) & 1))];
-      if (v != v) { ok = false; break; }
-      cs |= (v > a.level ? 1 : 0) << k;
+// One wave per word: lane l looks at point z = 64 w + l of the row.
+__global__ __launch_bounds__(256) void mc_bits_kernel(McArgs a) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t w0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * MC_PER_WAVE;   // the words of a lattice fit 32 bits
+  double v[MC_PER_WAVE];
+  uint8_t m[MC_PER_WAVE];
+#pragma unroll
+  for (int i = 0; i < MC_PER_WAVE; ++i) {
+    const uint32_t w = w0 + i, row = w / (uint32_t)a.W, z = (w - row * (uint32_t)a.W) * 64 + lane;
+    const bool in = w < a.words && z < a.nz;
+    v[i] = in ? a.f[row * a.nz + z] : a.level;          // not above, and no cube reaches it
+    m[i] = in && a.mask ? a.mask[row * a.nz + z] : 1;
+  }
+#pragma unroll
+  for (int i = 0; i < MC_PER_WAVE; ++i) {
+    const uint64_t up = __ballot(v[i] > a.level), nn = __ballot(v[i] != v[i]), mk = __ballot(m[i] != 0);
+    if (lane == 0 && w0 + i < a.words) {
+      a.above[w0 + i] = up;
+      a.nan[w0 + i] = nn;
+      a.msk[w0 + i] = mk;
     }
   }
-  if (!ok) cs = 0;
-  cases[c] = (uint8_t)cs;
-  ntri[c] = a.T->ntri[cs];
-  const uint16_t used = a.T->edges[cs];
-  for (int e = 0; e < 12; ++e)
-    if (used & (1u << e)) eflag[gedge(a, x, y, z, e)] = 1u;
 }
 
-__global__ void mc_vertices_kernel(McArgs a, const uint32_t* eflag, const uint32_t* vid, double ox, double oy,
-                                   double oz, double hx, double hy, double hz, double* verts) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= 3 * a.nx * a.ny * a.nz || !eflag[g]) return;
-  const int axis = (int)(g % 3);
-  const int64_t p = g / 3;
-  const int64_t z = p % a.nz, y = (p / a.nz) % a.ny, x = p / (a.nz * a.ny);
-  const int64_t q = axis == 0 ? pidx(a, x + 1, y, z) : (axis == 1 ? pidx(a, x, y + 1, z) : pidx(a, x, y, z + 1));
-  const double v0 = a.f[p], v1 = a.f[q];
-  const double t = (a.level - v0) / (v1 - v0);
-  double P[3] = {(double)x, (double)y, (double)z};
-  P[axis] += t;
-  double* o = verts + 3 * (int64_t)vid[g];
-  o[0] = ox + P[0] * hx;
-  o[1] = oy + P[1] * hy;
-  o[2] = oz + P[2] * hz;
+// Bits z + 1 and z - 1 of a row's word i at its bit z.
+__device__ __forceinline__ uint64_t bits_up(const uint64_t* b, int64_t i, bool last) {
+  return (b[i] >> 1) | (last ? 0 : b[i + 1] << 63);
+}
+__device__ __forceinline__ uint64_t bits_down(const uint64_t* b, int64_t i, bool first) {
+  return (b[i] << 1) | (first ? 0 : b[i - 1] >> 63);
 }
 
-__global__ void mc_faces_kernel(McArgs a, const uint8_t* cases, const uint32_t* foff, const uint32_t* vid,
-                                int32_t* faces) {
-  const int64_t ncx = a.nx - 1, ncy = a.ny - 1, ncz = a.nz - 1;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncx * ncy * ncz) return;
-  const int cs = cases[c];
-  const int nt = a.T->ntri[cs];
-  if (nt == 0) return;
-  const int64_t z = c % ncz, y = (c / ncz) % ncy, x = c / (ncz * ncy);
-  int32_t* o = faces + 3 * (int64_t)foff[c];
-  for (int t = 0; t < nt; ++t)
-    for (int k = 0; k < 3; ++k) o[3 * t + k] = (int32_t)vid[gedge(a, x, y, z, a.T->tri[cs][t][k])];
-}
-
-// Exclusive scan of n uint32 in chunks of 1024 (256 threads x 4), the chunk
-// totals scanned by one workgroup; *total receives the sum.
-__global__ __launch_bounds__(256) void scan_chunks_kernel(const uint32_t* in, uint32_t* out, int64_t n,
-                                                          uint32_t* sums) {
-  __shared__ uint32_t s[256];
-  const int64_t base = (int64_t)blockIdx.x * 1024 + 4 * threadIdx.x;
-  uint32_t v[4], acc = 0;
-  for (int k = 0; k < 4; ++k) {
-    v[k] = base + k < n ? in[base + k] : 0u;
-    acc += v[k];
+// Meshed cubes of a word: the mask at the far corner (+1, +1, +1), no NaN at any corner.
+__global__ __launch_bounds__(256) void mc_valid_kernel(McArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.words) return;
+  const uint32_t row = (uint32_t)i / (uint32_t)a.W, w = i - row * a.W, x = row / (uint32_t)a.ny, y = row - x * a.ny;
+  uint64_t ok = 0;
+  if (x + 1 < a.nx && y + 1 < a.ny) {
+    const bool last = w + 1 == a.W;
+    const int64_t left = a.nz - 1 - 64 * (int64_t)w;              // cubes of the row from this word on
+    ok = left >= 64 ? ~0ull : (left > 0 ? (1ull << left) - 1 : 0);
+    ok &= bits_up(a.msk, i + a.ny * a.W + a.W, last);
+    for (int k = 0; k < 4; ++k) {
+      const int64_t j = i + (k & 1) * a.ny * a.W + (k >> 1) * a.W;
+      ok &= ~(a.nan[j] | bits_up(a.nan, j, last));
+    }
   }
-  s[threadIdx.x] = acc;
+  a.valid[i] = ok;
+}
+
+// Case of the cube at bit z of the four rows' words lo (z) and hi (z + 1).
+__device__ __forceinline__ int mc_case(const uint64_t* lo, const uint64_t* hi, int z) {
+  int cs = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    cs |= (int)((lo[k] >> z) & 1) << k | (int)((hi[k] >> z) & 1) << (k + 4);
+  return cs;
+}
+
+// The four rows x + (k & 1), y + (k >> 1) of the cubes of word i (rows beyond
+// the lattice repeat the own one: such cubes are not meshed).
+__device__ __forceinline__ void mc_corner_words(const McArgs& a, int64_t i, int64_t x, int64_t y, bool last,
+                                                uint64_t* lo, uint64_t* hi) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t j = i + (((k & 1) && x + 1 < a.nx) ? a.ny * a.W : 0) + (((k >> 1) && y + 1 < a.ny) ? a.W : 0);
+    lo[k] = a.above[j];
+    hi[k] = bits_up(a.above, j, last);
+  }
+}
+
+__device__ __forceinline__ uint64_t mc_active(const uint64_t* lo, const uint64_t* hi, uint64_t valid) {
+  const uint64_t any = lo[0] | lo[1] | lo[2] | lo[3] | hi[0] | hi[1] | hi[2] | hi[3];
+  const uint64_t all = lo[0] & lo[1] & lo[2] & lo[3] & hi[0] & hi[1] & hi[2] & hi[3];
+  return valid & any & ~all;
+}
+
+// Inclusive sums over the block's 256 threads of a pair of counts.
+__device__ __forceinline__ uint2 block_scan(uint2 v, uint2* s) {
+  const int t = threadIdx.x, n = blockDim.x;
+  s[t] = v;
   __syncthreads();
-  for (int o = 1; o < 256; o <<= 1) {
-    const uint32_t t = threadIdx.x >= (unsigned)o ? s[threadIdx.x - o] : 0u;
+  for (int o = 1; o < n; o <<= 1) {
+    const uint2 u = t >= o ? s[t - o] : make_uint2(0, 0);
     __syncthreads();
-    s[threadIdx.x] += t;
+    v.x += u.x;
+    v.y += u.y;
+    s[t] = v;
     __syncthreads();
   }
-  uint32_t run = s[threadIdx.x] - acc;
-  for (int k = 0; k < 4; ++k) {
-    if (base + k < n) out[base + k] = run;
-    run += v[k];
-  }
-  if (threadIdx.x == 255) sums[blockIdx.x] = s[255];
+  return v;
 }
 
-__global__ __launch_bounds__(1024) void scan_sums_kernel(uint32_t* sums, int64_t nb, uint32_t* total) {
-  __shared__ uint32_t s[1024];
+// Used edges of each word, and the counts of the vertices and triangles
+// before it in its block.  An edge is used when its ends differ and one of
+// the (up to four) cubes around it is meshed.
+__global__ __launch_bounds__(MC_WORDS) void mc_count_kernel(McArgs a) {
+  __shared__ uint2 s[MC_WORDS];
+  const int64_t i = (int64_t)blockIdx.x * MC_WORDS + threadIdx.x;
+  uint2 n = make_uint2(0, 0);
+  if (i < a.words) {
+    const uint32_t row = (uint32_t)i / (uint32_t)a.W, w = i - row * a.W, x = row / (uint32_t)a.ny, y = row - x * a.ny;
+    const int64_t sx = a.ny * a.W, sy = a.W;
+    const bool first = w == 0, last = w + 1 == a.W;
+    uint64_t lo[4], hi[4];
+    mc_corner_words(a, i, x, y, last, lo, hi);
+    const uint64_t v00 = a.valid[i], v10 = x ? a.valid[i - sx] : 0, v01 = y ? a.valid[i - sy] : 0,
+                   v11 = x && y ? a.valid[i - sx - sy] : 0;
+    const uint64_t d00 = bits_down(a.valid, i, first), d10 = x ? bits_down(a.valid, i - sx, first) : 0,
+                   d01 = y ? bits_down(a.valid, i - sy, first) : 0;
+    const uint64_t e0 = (lo[0] ^ lo[1]) & (v00 | d00 | v01 | d01);
+    const uint64_t e1 = (lo[0] ^ lo[2]) & (v00 | d00 | v10 | d10);
+    const uint64_t e2 = (lo[0] ^ hi[0]) & (v00 | v10 | v01 | v11);
+    a.edge[0][i] = e0;
+    a.edge[1][i] = e1;
+    a.edge[2][i] = e2;
+    n.x = __popcll(e0) + __popcll(e1) + __popcll(e2);
+    for (uint64_t left = mc_active(lo, hi, v00); left; left &= left - 1)
+      n.y += a.T->ntri[mc_case(lo, hi, __ffsll((unsigned long long)left) - 1)];
+  }
+  const uint2 sum = block_scan(n, s);
+  if (i < a.words) {
+    a.vpre[i] = sum.x - n.x;
+    a.tpre[i] = sum.y - n.y;
+  }
+  if (threadIdx.x == MC_WORDS - 1) {
+    a.vsum[blockIdx.x] = sum.x;
+    a.tsum[blockIdx.x] = sum.y;
+  }
+}
+
+// Block sums to sums over the earlier blocks (one workgroup); the totals go
+// to device memory, for the writing pass, and to the caller's pinned pair.
+__global__ __launch_bounds__(1024) void mc_scan_kernel(McArgs a, int64_t nb, uint32_t* host) {
+  __shared__ uint2 s[1024];
   const int64_t per = (nb + 1023) / 1024;
-  const int64_t b0 = threadIdx.x * per;
-  uint32_t acc = 0;
-  for (int64_t i = b0; i < b0 + per && i < nb; ++i) acc += sums[i];
-  s[threadIdx.x] = acc;
+  const int64_t b0 = threadIdx.x * per, b1 = b0 + per < nb ? b0 + per : nb;
+  uint2 acc = make_uint2(0, 0);
+  for (int64_t i = b0; i < b1; ++i) { acc.x += a.vsum[i]; acc.y += a.tsum[i]; }
+  const uint2 sum = block_scan(acc, s);
+  uint2 run = make_uint2(sum.x - acc.x, sum.y - acc.y);
+  for (int64_t i = b0; i < b1; ++i) {
+    const uint32_t v = a.vsum[i], t = a.tsum[i];
+    a.vsum[i] = run.x;
+    a.tsum[i] = run.y;
+    run.x += v;
+    run.y += t;
+  }
+  if (threadIdx.x == 1023) {
+    a.total[0] = host[0] = sum.x;
+    a.total[1] = host[1] = sum.y;
+  }
+}
+
+// Vertex of the edge from point (row, z) along axis: vertices are numbered by point, then axis.
+__device__ __forceinline__ uint32_t mc_vertex(const McArgs& a, int64_t row, int64_t z, int axis) {
+  const int64_t i = row * a.W + (z >> 6);
+  const int b = (int)(z & 63);
+  const uint64_t e0 = a.edge[0][i], e1 = a.edge[1][i], e2 = a.edge[2][i], below = (1ull << b) - 1;
+  uint32_t id = a.vsum[i / MC_WORDS] + a.vpre[i] + __popcll(e0 & below) + __popcll(e1 & below) + __popcll(e2 & below);
+  if (axis > 0) id += (uint32_t)(e0 >> b) & 1u;
+  if (axis > 1) id += (uint32_t)(e1 >> b) & 1u;
+  return id;
+}
+
+// Writes the vertices and the triangles of MC_EMIT words.  Both are few (a
+// crossed word holds a handful) and reached through chains of dependent loads,
+// so a block first lists them in LDS, MC_LANES threads per word each at its 4
+// bits, and then gives every vertex and every triangle corner a thread of its
+// own: as one lane per point, almost all idle, this pass took 75 us of 132 at
+// 200^3, and takes 35 us now.  Writes nothing when the results exceed the
+// caller's buffers.
+constexpr int MC_EMIT = 16, MC_LANES = 16;
+static_assert(MC_WORDS % MC_EMIT == 0, "the words of a writing block lie in one counting block");
+__global__ __launch_bounds__(MC_EMIT * MC_LANES) void mc_emit_kernel(McArgs a, double ox, double oy, double oz,
+                                                                     double hx, double hy, double hz, double* verts,
+                                                                     int64_t max_verts, int32_t* faces,
+                                                                     int64_t max_faces) {
+  __shared__ uint32_t list[MC_EMIT * 64 * MC_MAX_TRI];   // vertices (at most 3 a point), then triangles
+  __shared__ uint32_t count[2];
+  if (a.total[0] > max_verts || a.total[1] > max_faces) return;
+  const uint32_t t = threadIdx.x, w0 = blockIdx.x * MC_EMIT, i = w0 + t / MC_LANES;
+  const int z0 = 4 * (int)(t % MC_LANES);
+  const bool live = i < a.words;
+  // the first vertex and triangle of the block's words (one counting block holds them all)
+  const uint32_t vbase = a.vsum[w0 / MC_WORDS] + a.vpre[w0], tbase = a.tsum[w0 / MC_WORDS] + a.tpre[w0];
+  if (t < 2) count[t] = 0;
   __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const uint32_t t = threadIdx.x >= (unsigned)o ? s[threadIdx.x - o] : 0u;
-    __syncthreads();
-    s[threadIdx.x] += t;
-    __syncthreads();
+  uint64_t e[3] = {0, 0, 0};
+  uint32_t n = 0;
+  if (live) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      e[u] = a.edge[u][i];
+      n += __popcll(e[u]);
+    }
+    uint32_t at = a.vpre[i] - a.vpre[w0];
+    if (z0 == 0 && n) atomicMax(&count[0], at + n);
+    const uint64_t below = (1ull << z0) - 1;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) at += __popcll(e[u] & below);
+#pragma unroll
+    for (int z = z0; z < z0 + 4; ++z)
+#pragma unroll
+      for (uint32_t u = 0; u < 3; ++u)
+        if ((e[u] >> z) & 1) list[at++] = (i - w0) << 8 | (uint32_t)z << 2 | u;
   }
-  uint32_t run = s[threadIdx.x] - acc;
-  for (int64_t i = b0; i < b0 + per && i < nb; ++i) {
-    const uint32_t v = sums[i];
-    sums[i] = run;
-    run += v;
+  __syncthreads();
+  const int64_t step[3] = {a.ny * a.nz, a.nz, 1};
+  for (uint32_t k = t; k < count[0]; k += MC_EMIT * MC_LANES) {
+    const uint32_t r = list[k], axis = r & 3, j = w0 + (r >> 8);
+    const uint32_t row = j / (uint32_t)a.W, z = (j - row * (uint32_t)a.W) * 64 + ((r >> 2) & 63);
+    const uint32_t x = row / (uint32_t)a.ny, y = row - x * (uint32_t)a.ny;
+    const int64_t p = row * a.nz + z;
+    const double v0 = a.f[p], v1 = a.f[p + (axis == 0 ? step[0] : (axis == 1 ? step[1] : step[2]))];
+    const double s = (a.level - v0) / (v1 - v0);
+    double P[3] = {(double)x, (double)y, (double)z};
+#pragma unroll
+    for (uint32_t u = 0; u < 3; ++u)
+      if (u == axis) P[u] += s;
+    double* o = verts + 3 * (int64_t)(vbase + k);
+    o[0] = ox + P[0] * hx;
+    o[1] = oy + P[1] * hy;
+    o[2] = oz + P[2] * hz;
   }
-  if (threadIdx.x == 1023) *total = s[1023];
-}
-
-__global__ void scan_add_kernel(uint32_t* out, int64_t n, const uint32_t* sums) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] += sums[i / 1024];
-}
-
-void exclusive_scan(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* sums, uint32_t* total, hipStream_t st) {
-  const int64_t nb = std::max<int64_t>(gk_ceil_div(n, 1024), 1);
-  hipLaunchKernelGGL(scan_chunks_kernel, dim3((unsigned)nb), dim3(256), 0, st, in, out, n, sums);
-  hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, st, sums, nb, total);
-  hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)gk_ceil_div(n, 256)), dim3(256), 0, st, out, n, sums);
+  __syncthreads();
+  int cs[4] = {0, 0, 0, 0};
+  uint32_t nt = 0;
+  if (live) {
+    const uint32_t row = i / (uint32_t)a.W, w = i - row * (uint32_t)a.W;
+    const uint32_t x = row / (uint32_t)a.ny, y = row - x * (uint32_t)a.ny;
+    uint64_t lo[4], hi[4];
+    mc_corner_words(a, i, x, y, w + 1 == a.W, lo, hi);
+    const uint64_t act = mc_active(lo, hi, a.valid[i]);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if ((act >> (z0 + b)) & 1) {
+        cs[b] = mc_case(lo, hi, z0 + b);
+        nt += a.T->ntri[cs[b]];
+      }
+  }
+  uint32_t sum = nt;                     // of the word's threads up to this one
+#pragma unroll
+  for (int o = 1; o < MC_LANES; o <<= 1) {
+    const uint32_t v = __shfl_up(sum, o, MC_LANES);
+    if ((int)(t % MC_LANES) >= o) sum += v;
+  }
+  if (live) {
+    uint32_t at = a.tpre[i] - a.tpre[w0] + sum - nt;
+    if (nt) atomicMax(&count[1], at + nt);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (cs[b])
+        for (uint32_t q = 0; q < a.T->ntri[cs[b]]; ++q)
+          list[at++] = (i - w0) << 17 | (uint32_t)(z0 + b) << 11 | (uint32_t)cs[b] << 3 | q;
+  }
+  __syncthreads();
+  for (uint32_t k = t; k < 3 * count[1]; k += MC_EMIT * MC_LANES) {
+    const uint32_t r = list[k / 3], j = w0 + (r >> 17);
+    const int le = a.T->tri[(r >> 3) & 255][r & 7][k % 3], axis = le >> 2, q = le & 3;
+    // the edge's start from the cube's corner: q's bits go to the other axes in order
+    const int dx = axis == 0 ? 0 : q & 1, dy = axis == 1 ? 0 : (axis == 0 ? q & 1 : q >> 1),
+              dz = axis == 2 ? 0 : q >> 1;
+    const uint32_t row = j / (uint32_t)a.W, z = (j - row * (uint32_t)a.W) * 64 + ((r >> 11) & 63);
+    faces[3 * (int64_t)tbase + k] = (int32_t)mc_vertex(a, row + dx * a.ny + dy, z + dz, axis);
+  }
 }
 
 }  // namespace
@@ -280,15 +434,14 @@ extern "C" int gk_marching_cubes(gk_handle h, const double* field, const int64_t
   *n_faces = 0;
   if (nx < 2 || ny < 2 || nz < 2) return GK_OK;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nc = (nx - 1) * (ny - 1) * (nz - 1);
-  const int64_t ne = 3 * np_;
-  // workspace: tables | eflag ne | vid ne | cases nc | ntri nc | foff nc | sums | totals
+  const int64_t W = gk_ceil_div(nz, 64), words = nx * ny * W, nb = gk_ceil_div(words, MC_WORDS);
+  // workspace: tables | totals | 7 word arrays | 2 counts per word | 2 sums per block
   size_t need = 0;
   auto take = [&](size_t bytes) { size_t o = need; need += gk_round_up(bytes, 256); return o; };
-  const size_t o_T = take(sizeof(McTables)), o_ef = take(ne * 4), o_vid = take(ne * 4), o_cs = take(nc),
-               o_nt = take(nc * 4), o_fo = take(nc * 4),
-               o_sum = take((size_t)(std::max(gk_ceil_div(ne, 1024), gk_ceil_div(nc, 1024)) + 1) * 4),
-               o_tot = take(16);
+  const size_t o_T = take(sizeof(McTables)), o_tot = take(16);
+  size_t o_w[7], o_n[4];
+  for (size_t& o : o_w) o = take(words * 8);
+  for (int k = 0; k < 4; ++k) o_n[k] = take((k < 2 ? words : nb) * 4);
   void* p = nullptr;
   GK_TRY(gk_workspace(h, WS_MESH, need, &p));
   char* b = static_cast<char*>(p);
@@ -297,31 +450,32 @@ extern "C" int gk_marching_cubes(gk_handle h, const double* field, const int64_t
     GK_HIP(hipMemcpyAsync(b + o_T, &host, sizeof(McTables), hipMemcpyHostToDevice, st));
     h->mesh_tables = b + o_T;
   }
-  McArgs a{field, mask, nx, ny, nz, level, reinterpret_cast<const McTables*>(b + o_T)};
-  uint32_t* ef = reinterpret_cast<uint32_t*>(b + o_ef);
-  uint32_t* vid = reinterpret_cast<uint32_t*>(b + o_vid);
-  uint8_t* cs = reinterpret_cast<uint8_t*>(b + o_cs);
-  uint32_t* nt = reinterpret_cast<uint32_t*>(b + o_nt);
-  uint32_t* fo = reinterpret_cast<uint32_t*>(b + o_fo);
-  uint32_t* sums = reinterpret_cast<uint32_t*>(b + o_sum);
-  uint32_t* tot = reinterpret_cast<uint32_t*>(b + o_tot);
-  GK_HIP(hipMemsetAsync(ef, 0, ne * 4, st));
-  hipLaunchKernelGGL(mc_classify_kernel, dim3((unsigned)gk_ceil_div(nc, 256)), dim3(256), 0, st, a, cs, nt, ef);
-  exclusive_scan(ef, vid, ne, sums, tot, st);
-  exclusive_scan(nt, fo, nc, sums, tot + 1, st);
-  uint32_t counts[2] = {0, 0};
-  GK_HIP(hipMemcpyAsync(counts, tot, sizeof(counts), hipMemcpyDeviceToHost, st));
+  if (!h->mesh_counts) GK_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->mesh_counts), 64, hipHostMallocDefault));
+  McArgs a{};
+  a.f = field; a.mask = mask;
+  a.nx = nx; a.ny = ny; a.nz = nz; a.W = W; a.words = words;
+  a.level = level;
+  a.T = reinterpret_cast<const McTables*>(b + o_T);
+  uint64_t** wp[7] = {&a.above, &a.nan, &a.msk, &a.valid, &a.edge[0], &a.edge[1], &a.edge[2]};
+  for (int k = 0; k < 7; ++k) *wp[k] = reinterpret_cast<uint64_t*>(b + o_w[k]);
+  uint32_t** np[4] = {&a.vpre, &a.tpre, &a.vsum, &a.tsum};
+  for (int k = 0; k < 4; ++k) *np[k] = reinterpret_cast<uint32_t*>(b + o_n[k]);
+  a.total = reinterpret_cast<uint32_t*>(b + o_tot);
+  hipLaunchKernelGGL(mc_bits_kernel, dim3((unsigned)gk_ceil_div(words, 4 * MC_PER_WAVE)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(mc_valid_kernel, dim3((unsigned)gk_ceil_div(words, 256)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(mc_count_kernel, dim3((unsigned)nb), dim3(MC_WORDS), 0, st, a);
+  hipLaunchKernelGGL(mc_scan_kernel, dim3(1), dim3(1024), 0, st, a, nb, h->mesh_counts);
+  if (verts && faces)
+    hipLaunchKernelGGL(mc_emit_kernel, dim3((unsigned)gk_ceil_div(words, MC_EMIT)), dim3(MC_EMIT * MC_LANES), 0, st, a, origin[0],
+                       origin[1], origin[2], spacing[0], spacing[1], spacing[2], verts, max_verts, faces, max_faces);
+  GK_HIP(hipGetLastError());
   GK_HIP(hipStreamSynchronize(st));
+  const uint32_t counts[2] = {h->mesh_counts[0], h->mesh_counts[1]};
   *n_verts = counts[0];
   *n_faces = counts[1];
   if (!verts || !faces) return GK_OK;
   GK_REQUIRE(counts[0] <= max_verts && counts[1] <= max_faces, GK_ERR_ARG,
              "gk_marching_cubes: %u vertices / %u faces exceed the output capacity (%lld / %lld)", counts[0],
              counts[1], (long long)max_verts, (long long)max_faces);
-  hipLaunchKernelGGL(mc_vertices_kernel, dim3((unsigned)gk_ceil_div(ne, 256)), dim3(256), 0, st, a, ef, vid,
-                     origin[0], origin[1], origin[2], spacing[0], spacing[1], spacing[2], verts);
-  hipLaunchKernelGGL(mc_faces_kernel, dim3((unsigned)gk_ceil_div(nc, 256)), dim3(256), 0, st, a, cs, fo, vid, faces);
-  GK_HIP(hipGetLastError());
-  GK_HIP(hipStreamSynchronize(st));
   return GK_OK;
 }
