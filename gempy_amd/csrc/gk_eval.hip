@@ -114,6 +114,100 @@ template <> struct Tiny<float> { static constexpr float v = 1e-30f; };
 __device__ __forceinline__ double gk_rsq_raw(double t) { return __builtin_amdgcn_rsq(t); }
 __device__ __forceinline__ float gk_rsq_raw(float t) { return __builtin_amdgcn_rsqf(t); }
 
+// Sums of one LDS tile's sources over a z-run of PPT lattice points (x0, y0,
+// z0 + q hz).  What bounds them is the issue of FP64 (FP32) vector
+// instructions, so everything that depends on the source or the run alone is
+// kept out of the pair: the source weight goes into the polynomial, the
+// Newton step of rho = sqrt(t) rides on it (see above), t never reaches 0.
+// Without mask and gradient 9 instructions and an rsq per interface pair; the
+// gradient adds 8 (12 on orientations).  With a clamp, a full Newton step and
+// unweighted polynomials per pair instead, field and gradient of 1.2e6 points
+// and 1,900 sources took 2.44 ms against 2.21, the masked field of 1.2e6 points
+// and 6,000 sources 4.82 against 4.28.
+template <typename T, bool GRAD, bool MASKED, int PPT>
+__device__ __forceinline__ void lattice_pts_tile(const V4<T>* s4, int nk, T x0, T y0, T z0, T hz, T (&part)[PPT],
+                                                 T (&gpart)[PPT][3]) {
+  T wsum = T(0);
+#pragma unroll 2
+  for (int k = 0; k < nk; ++k) {
+    const V4<T> s = s4[k];
+    const T dx = x0 - s.x, dy = y0 - s.y;
+    const T dxy = fma(dx, dx, fma(dy, dy, Tiny<T>::v));
+    const T c3 = T(0.375) * s.w, c2 = T(-1.75) * s.w, c1 = T(4.375) * s.w, c0 = T(-7.0) * s.w;
+    T d3 = T(0), d2 = T(0), d1 = T(0), d0 = T(0);
+    if (GRAD) { d3 = T(2.625) * s.w; d2 = T(-8.75) * s.w; d1 = T(13.125) * s.w; d0 = T(-14.0) * s.w; }
+    const T e0 = z0 - s.z;
+    if (!MASKED && !GRAD) wsum += s.w;
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+      const T e = fma(T(q), hz, e0);
+      const T t = fma(e, e, dxy);
+      const T y = gk_rsq_raw(t);
+      const T r = t * y;
+      const T h3 = fma(-r, y, T(3));
+      T u = fma(c3, t, c2);
+      u = fma(u, t, c1);
+      const T v = fma(r * u, h3, c0);
+      if (MASKED || GRAD) {                // with gradient the same sums with and without mask
+        const T c = fma(v, t, s.w);
+        part[q] += !MASKED || t < T(1) ? c : T(0) * s.w;
+      } else {
+        part[q] = fma(v, t, part[q]);
+      }
+      if (GRAD) {
+        T g = fma(d3, t, d2);
+        g = fma(g, t, d1);
+        T wd = fma(r * g, h3, d0);
+        if (MASKED) wd = t < T(1) ? wd : T(0) * s.w;
+        gpart[q][0] = fma(wd, dx, gpart[q][0]);
+        gpart[q][1] = fma(wd, dy, gpart[q][1]);
+        gpart[q][2] = fma(wd, e, gpart[q][2]);
+      }
+    }
+  }
+  if (!MASKED && !GRAD) {
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) part[q] += wsum;
+  }
+}
+
+template <typename T, bool GRAD, bool MASKED, int PPT>
+__device__ __forceinline__ void lattice_ori_tile(const V8<T>* s8, int nk, T x0, T y0, T z0, T hz, T (&part)[PPT],
+                                                 T (&gpart)[PPT][3]) {
+  // the derivative polynomial's constants held in registers (as literals
+  // the compiler would rebuild them inside the loop)
+  T d3 = T(2.625), d2 = T(-8.75), d1 = T(13.125), d0 = T(-14.0);     // d1..d3 halved
+  asm volatile("" : "+v"(d3), "+v"(d2), "+v"(d1), "+v"(d0));
+#pragma unroll 2
+  for (int k = 0; k < nk; ++k) {
+    const V8<T> s = s8[k];
+    const T dx = s.x - x0, dy = s.y - y0;          // q - x
+    const T dxy = fma(dx, dx, fma(dy, dy, Tiny<T>::v));
+    const T base_dot = fma(s.wx, dx, s.wy * dy);
+    const T e0 = z0 - s.z;                         // x - q (z)
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+      const T e = fma(T(q), hz, e0);
+      const T t = fma(e, e, dxy);
+      const T y = gk_rsq_raw(t);
+      const T r = t * y;
+      const T h3 = fma(-r, y, T(3));
+      T p = fma(r * fma(fma(d3, t, d2), t, d1), h3, d0);
+      if (MASKED) p = t < T(1) ? p : T(0);
+      const T dot = fma(-s.wz, e, base_dot);
+      part[q] = fma(dot, p, part[q]);
+      if (GRAD) {
+        const T om = T(1) - t;
+        T hw = (d1 * dot) * (om * om) * (y * h3);  // 26.25 (1-t)^2 / rho, 1/rho = y (3 - r y) / 2
+        if (MASKED) hw = t < T(1) ? hw : T(0) * dot;
+        gpart[q][0] = fma(-s.wx, p, fma(-hw, dx, gpart[q][0]));
+        gpart[q][1] = fma(-s.wy, p, fma(-hw, dy, gpart[q][1]));
+        gpart[q][2] = fma(-s.wz, p, fma(hw, e, gpart[q][2]));
+      }
+    }
+  }
+}
+
 // SCALAR false (explicit points with gradient): the gradient only; the
 // scalar output then holds the drift terms alone.
 template <typename T, bool LATTICE, bool GRAD, bool MASKED, int PPT, bool SCALAR = true>
@@ -201,58 +295,12 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
       s4[tid] = v;
     }
     __syncthreads();
-    if constexpr (LATTICE && !GRAD && !MASKED) {
-      T wsum = T(0);
+    if constexpr (LATTICE) {
+      lattice_pts_tile<T, GRAD, MASKED, PPT>(s4, nk, x0, y0, z0, hz, part, gpart);
+    } else {             // explicit points: no clamp per pair, Newton step folded as on the lattice
 #pragma unroll 2
       for (int k = 0; k < nk; ++k) {
         const V4<T> s = s4[k];
-        const T dx = x0 - s.x, dy = y0 - s.y;
-        const T dxy = fma(dx, dx, fma(dy, dy, Tiny<T>::v));
-        const T c3 = T(0.375) * s.w, c2 = T(-1.75) * s.w, c1 = T(4.375) * s.w, c0 = T(-7.0) * s.w;
-        const T e0 = z0 - s.z;
-        wsum += s.w;
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-          const T e = fma(T(q), hz, e0);
-          const T t = fma(e, e, dxy);
-          const T y = gk_rsq_raw(t);
-          const T r = t * y;
-          const T h3 = fma(-r, y, T(3));
-          T u = fma(c3, t, c2);
-          u = fma(u, t, c1);
-          const T v = fma(r * u, h3, c0);
-          part[q] = fma(v, t, part[q]);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < PPT; ++q) part[q] += wsum;
-    } else {
-#pragma unroll 2
-    for (int k = 0; k < nk; ++k) {
-      const V4<T> s = s4[k];
-      if (LATTICE) {
-        const T dx = x0 - s.x, dy = y0 - s.y;
-        const T dxy = fma(dx, dx, dy * dy);
-        T e = z0 - s.z;
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-          const T t = fma(e, e, dxy);
-          const T y = gk_rsqrt(t);
-          const T rho = t * y;
-          T c = gk_cov_poly(t, rho);
-          if (MASKED) c = t < T(1) ? c : T(0);
-          part[q] = fma(s.w, c, part[q]);
-          if (GRAD) {
-            T dp = gk_dcov_poly(t, rho);
-            if (MASKED) dp = t < T(1) ? dp : T(0);
-            const T wd = s.w * dp;
-            gpart[q][0] = fma(wd, dx, gpart[q][0]);
-            gpart[q][1] = fma(wd, dy, gpart[q][1]);
-            gpart[q][2] = fma(wd, e, gpart[q][2]);
-          }
-          e += hz;
-        }
-      } else {           // explicit points: no clamp per pair, Newton step folded as on the lattice
 #pragma unroll
         for (int q = 0; q < PPT; ++q) {
           const T dx = px[q] - s.x, dy = py[q] - s.y, dz = pz[q] - s.z;
@@ -273,7 +321,6 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
           }
         }
       }
-    }
     }
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
@@ -298,60 +345,12 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
       s_src[tid] = v;
     }
     __syncthreads();
-    if constexpr (LATTICE && !GRAD && !MASKED) {
-      // the derivative polynomial's constants held in registers (as literals
-      // the compiler would rebuild them inside the loop)
-      T d3 = T(2.625), d2 = T(-8.75), d1 = T(13.125), d0 = T(-14.0);     // d1..d3 halved
-      asm volatile("" : "+v"(d3), "+v"(d2), "+v"(d1), "+v"(d0));
+    if constexpr (LATTICE) {
+      lattice_ori_tile<T, GRAD, MASKED, PPT>(s_src, nk, x0, y0, z0, hz, part, gpart);
+    } else {             // explicit points (see the interface-source loop)
 #pragma unroll 2
       for (int k = 0; k < nk; ++k) {
         const V8<T> s = s_src[k];
-        const T dx = s.x - x0, dy = s.y - y0;          // q - x
-        const T dxy = fma(dx, dx, fma(dy, dy, Tiny<T>::v));
-        const T base_dot = fma(s.wx, dx, s.wy * dy);
-        const T e0 = z0 - s.z;                         // x - q (z)
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-          const T e = fma(T(q), hz, e0);
-          const T t = fma(e, e, dxy);
-          const T y = gk_rsq_raw(t);
-          const T r = t * y;
-          const T h3 = fma(-r, y, T(3));
-          const T p = fma(r * fma(fma(d3, t, d2), t, d1), h3, d0);
-          const T dot = fma(-s.wz, e, base_dot);
-          part[q] = fma(dot, p, part[q]);
-        }
-      }
-    } else {
-#pragma unroll 2
-    for (int k = 0; k < nk; ++k) {
-      const V8<T> s = s_src[k];
-      if (LATTICE) {
-        const T dx = s.x - x0, dy = s.y - y0;          // q - x
-        const T dxy = fma(dx, dx, dy * dy);
-        const T base_dot = fma(s.wx, dx, s.wy * dy);
-        T e = z0 - s.z;                                // x - q (z)
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-          const T t = fma(e, e, dxy);
-          const T y = gk_rsqrt(t);
-          const T rho = t * y;
-          T p = gk_dcov_poly(t, rho);
-          if (MASKED) p = t < T(1) ? p : T(0);
-          const T dot = fma(-s.wz, e, base_dot);
-          part[q] = fma(dot, p, part[q]);
-          if (GRAD) {
-            const T om = T(1) - t;
-            T dd = T(26.25) * om * om * y;
-            if (MASKED) dd = t < T(1) ? dd : T(0);
-            const T hw = dot * dd;
-            gpart[q][0] -= fma(s.wx, p, hw * dx);
-            gpart[q][1] -= fma(s.wy, p, hw * dy);
-            gpart[q][2] -= fma(s.wz, p, -hw * e);
-          }
-          e += hz;
-        }
-      } else {           // explicit points (see the interface-source loop)
 #pragma unroll
         for (int q = 0; q < PPT; ++q) {
           const T dx = s.x - px[q], dy = s.y - py[q], dz = s.z - pz[q];   // q - x
@@ -374,7 +373,6 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
           }
         }
       }
-    }
     }
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
