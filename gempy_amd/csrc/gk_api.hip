@@ -105,29 +105,35 @@ extern "C" int gk_assemble_drift_impl(const gk_system* sys, double* U, hipStream
 
 // Bounding box of all sources (orientation, rest and reference points), read
 // back once per evaluation to decide whether the r < a mask can be dropped.
-__global__ void source_box_kernel(gk_system sys, double* box) {
-  __shared__ double lo[3][256], hi[3][256];
-  const int t = threadIdx.x;
+// One workgroup: a chain of dependent rounds, so as few as its 1024 threads
+// allow, and within the waves by shuffles (25,000 points: 39 us with 256
+// threads and a tree in LDS, 12 us).
+__global__ __launch_bounds__(1024) void source_box_kernel(gk_system sys, double* box) {
+  __shared__ double lo[3][16], hi[3][16];
+  const int t = threadIdx.x, wave = t >> 6;
   double l[3] = {1e300, 1e300, 1e300}, u[3] = {-1e300, -1e300, -1e300};
   const int64_t n = sys.n_ori + sys.n_rest + sys.n_surf;
-  for (int64_t i = t; i < n; i += 256) {
+#pragma unroll 4
+  for (int64_t i = t; i < n; i += 1024) {
     const double* p = i < sys.n_ori ? sys.ori_xyz + 3 * i
                       : (i < sys.n_ori + sys.n_rest ? sys.rest_xyz + 3 * (i - sys.n_ori)
                                                     : sys.ref_xyz + 3 * (i - sys.n_ori - sys.n_rest));
     for (int k = 0; k < 3; ++k) { l[k] = fmin(l[k], p[k]); u[k] = fmax(u[k], p[k]); }
   }
-  for (int k = 0; k < 3; ++k) { lo[k][t] = l[k]; hi[k][t] = u[k]; }
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w)
-      for (int k = 0; k < 3; ++k) {
-        lo[k][t] = fmin(lo[k][t], lo[k][t + w]);
-        hi[k][t] = fmax(hi[k][t], hi[k][t + w]);
-      }
-    __syncthreads();
+  for (int k = 0; k < 3; ++k) {
+    for (int o = 32; o > 0; o >>= 1) {
+      l[k] = fmin(l[k], __shfl_xor(l[k], o));
+      u[k] = fmax(u[k], __shfl_xor(u[k], o));
+    }
+    if ((t & 63) == 0) { lo[k][wave] = l[k]; hi[k][wave] = u[k]; }
   }
-  if (t == 0)
-    for (int k = 0; k < 3; ++k) { box[k] = lo[k][0]; box[3 + k] = hi[k][0]; }
+  __syncthreads();
+  if (t < 3) {
+    double a = lo[t][0], b = hi[t][0];
+    for (int w = 1; w < 16; ++w) { a = fmin(a, lo[t][w]); b = fmax(b, hi[t][w]); }
+    box[t] = a;
+    box[3 + t] = b;
+  }
 }
 
 extern "C" int gk_eval(gk_handle h, const gk_system* sys, const double* weights, gk_eval_desc* desc,
@@ -139,7 +145,7 @@ extern "C" int gk_eval(gk_handle h, const gk_system* sys, const double* weights,
   if (desc && desc->kind == GK_POINTS_LATTICE && sys && sys->n_ori + sys->n_rest + sys->n_surf > 0) {
     void* ws = nullptr;
     GK_TRY(gk_workspace(h, WS_SMALL, 256, &ws));
-    hipLaunchKernelGGL(source_box_kernel, dim3(1), dim3(256), 0, st, *sys, static_cast<double*>(ws));
+    hipLaunchKernelGGL(source_box_kernel, dim3(1), dim3(1024), 0, st, *sys, static_cast<double*>(ws));
     GK_HIP(hipMemcpyAsync(box, ws, sizeof(box), hipMemcpyDeviceToHost, st));
     GK_HIP(hipStreamSynchronize(st));
     pbox = box;
@@ -170,7 +176,7 @@ extern "C" int gk_source_box(gk_handle h, const gk_system* sys, double* box, gk_
   hipStream_t st = (hipStream_t)stream;
   void* ws = nullptr;
   GK_TRY(gk_workspace(h, WS_SMALL, 256, &ws));
-  hipLaunchKernelGGL(source_box_kernel, dim3(1), dim3(256), 0, st, *sys, static_cast<double*>(ws));
+  hipLaunchKernelGGL(source_box_kernel, dim3(1), dim3(1024), 0, st, *sys, static_cast<double*>(ws));
   GK_HIP(hipMemcpyAsync(box, ws, 6 * sizeof(double), hipMemcpyDeviceToHost, st));
   GK_HIP(hipStreamSynchronize(st));
   return GK_OK;

@@ -248,8 +248,9 @@ int gk_eval(gk_handle h, const gk_system* sys, const double* weights, gk_eval_de
  * GK_EVAL_SCRATCH_BYTES per GPU instead of the handle's growable workspace:
  * systems whose packed sources (8 n_surf + 32 (n_rest + n_surf) + 64 n_ori
  * bytes, FP64) exceed it are rejected with GK_ERR_ARG; explicit point sets
- * use fewer source splits when their partials do not fit.  Results equal
- * gk_eval's whenever the same split is used.  Every call on one GPU shares
+ * use fewer source splits when their partials do not fit; lattices are summed
+ * pair by pair, where gk_eval takes large ones in blocks.  Results equal
+ * gk_eval's whenever the same split is used, and within rounding otherwise.  Every call on one GPU shares
  * that array: calls that overlap on one GPU (other streams, other threads)
  * race and must be serialised by the caller. */
 #define GK_EVAL_SCRATCH_BYTES (32u << 20)

@@ -1,0 +1,105 @@
+"""Lattice evaluations that run in blocks (far sources through interpolation
+nodes, sources beyond the range left out) against the plain sum over all
+sources at the same points in extended precision on a sample, and against the
+explicit-point path, which has no blocks, at every point.
+
+Tolerances: sqrt(n) terms of size |w| max(1, |k|) with a few roundings each
+(2^-53 or 2^-24; the kernels reach 3 for orientations), 8 standard deviations;
+the drift adds its own rounding."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # res, points, orientations, range, precision, gradient
+    ((101, 97, 103), 2000, 400, 1732.05, "f64", False),      # ragged blocks, nodes
+    ((130, 64, 90), 3000, 30, 1732.05, "f64", False),
+    ((128, 128, 128), 600, 200, 1732.05, "f64", False),
+    ((200, 3, 200), 6000, 1500, 1732.05, "f64", False),      # a thin slab
+    ((1, 300, 301), 9000, 2000, 1732.05, "f64", False),      # one plane: never in blocks
+    ((100, 100, 100), 3000, 600, 1732.05, "f32", False),
+    ((61, 157, 73), 5000, 1000, 1732.05, "f32", False),
+    ((96, 97, 98), 3000, 700, 450.0, "f64", False),          # most sources beyond
+    ((96, 97, 98), 3000, 700, 1300.0, "f64", False),         # mask and nodes
+    ((96, 97, 98), 2000, 500, 450.0, "f64", True),
+    ((96, 97, 98), 3000, 700, 300.0, "f32", False),
+    ((96, 97, 98), 2000, 500, 450.0, "f32", True),
+    ((80, 81, 300), 2000, 600, 60.0, "f64", False),          # nearly all beyond
+]
+
+
+def _setup(points, oris, rng_, seed=3):
+    from gempy_amd import synthetic
+    from gempy_amd.data import KernelOptions
+    from gempy_amd.engine import DeviceStack
+    m = synthetic.config3(seed=seed, n_points=points, n_ori=oris, n_surfaces=4, resolution=(8, 8, 8))
+    ds = DeviceStack(m.stacks[0], KernelOptions(range=rng_, c_o=rng_ * rng_ / 42.0, uni_degree=1), [500.0] * 3)
+    w = torch.randn(ds.N, dtype=torch.float64, generator=torch.Generator().manual_seed(seed))
+    return ds, w.cuda()
+
+
+def _prec(p):
+    from gempy_amd import _lib
+    return _lib.GK_F64 if p == "f64" else _lib.GK_F32
+
+
+def _bound(points, oris, rng_, precision, gradient=False):
+    eps = 2.0 ** -53 if precision == "f64" else 2.0 ** -24
+    c_o = rng_ * rng_ / 42.0
+    # weights: 4 c_o per point; 2 c_o / a (times 3) per orientation; rounding of the terms and of their partial
+    # sums (sqrt(256) of them per tile); positions in FP32 move the terms by 14 eps of their size
+    size = np.sqrt(points) * 4 * c_o * 16 + np.sqrt(3 * oris) * 2 * c_o / rng_ * 3 * 16
+    if gradient:
+        size = (np.sqrt(points) * 4 * c_o * 14 + np.sqrt(3 * oris) * 2 * c_o / rng_ * 40) * 16 / rng_
+    return 8 * eps * size + 2.0 ** -50 * 1000.0
+
+
+@pytest.mark.parametrize("res,points,oris,rng_,prec,gradient", CASES)
+def test_matches_explicit_points(gpu, res, points, oris, rng_, prec, gradient):
+    from gempy_amd import synthetic
+    from gempy_amd.data import RegularGrid
+    ds, w = _setup(points, oris, rng_)
+    g = RegularGrid(synthetic.EXTENT, res)
+    S, G, _ = ds.evaluate_lattice(g, w, _prec(prec), gradient)
+    S2, G2, _ = ds.evaluate_points(torch.tensor(g.values(), device="cuda"), w, _prec("f64"), gradient)
+    err, tol = float((S - S2).abs().max()), _bound(points, oris, rng_, prec)
+    print(f"[gpu-case] blocks {res} {prec} range {rng_}: {err:.2e} (bound {tol:.2e})", flush=True)
+    assert err <= tol
+    if gradient:
+        assert float((G - G2).abs().max()) <= _bound(points, oris, rng_, prec, True)
+
+
+@pytest.mark.parametrize("box", [(2000.0, 2600.0, -50.0, 300.0, 400.0, 500.0), (0.0, 1000.0, 0.0, 1000.0, 499.0, 500.0)])
+def test_other_boxes(gpu, box):
+    """A grid beside its sources (range kept above every distance) and a flat one."""
+    from gempy_amd.data import RegularGrid
+    ds, w = _setup(3000, 600, 4000.0)
+    g = RegularGrid(box, (90, 91, 92))
+    S, _, _ = ds.evaluate_lattice(g, w)
+    S2, _, _ = ds.evaluate_points(torch.tensor(g.values(), device="cuda"), w)
+    assert float((S - S2).abs().max()) <= 4 * _bound(3000, 600, 4000.0, "f64")
+
+
+def test_ids_and_fault_drift(gpu):
+    from gempy_amd import synthetic
+    from gempy_amd.data import RegularGrid
+    ds, w = _setup(2500, 500, 1732.05)
+    g = RegularGrid(synthetic.EXTENT, (101, 99, 97))
+    thr = [3e6, 0.0, -3e6]
+    S, _, ids = ds.evaluate_lattice(g, w, thresholds=thr)
+    want = 1 + sum((S < t).int() for t in thr)
+    assert bool((ids == want).all())
+
+
+@pytest.mark.parametrize("rng_", [1732.05, 450.0])
+def test_weight_that_is_not_finite(gpu, rng_):
+    """A NaN weight reaches every point, wherever the source lies, as in the plain sum."""
+    from gempy_amd import synthetic
+    from gempy_amd.data import RegularGrid
+    ds, w = _setup(3000, 600, rng_)
+    g = RegularGrid(synthetic.EXTENT, (100, 101, 102))
+    w[3 * 600 + 17] = float("nan")
+    S, _, _ = ds.evaluate_lattice(g, w)
+    assert bool(torch.isnan(S).all())
