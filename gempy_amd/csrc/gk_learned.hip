@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void knn_kernel(gk_system sys, int64_t n, int3
 }
 
 #ifndef GK_LI_GRID
-#define GK_LI_GRID 128          // workgroups of the FP32 form's local-inverse kernel
+#define GK_LI_GRID 256          // workgroups of the FP32 form's local-inverse kernel
 #endif
 
 // ------------------------------------------------------- grid neighbours
@@ -168,62 +168,100 @@ __global__ void knn_scatter_kernel(gk_system sys, int64_t n, const int32_t* cell
   spos[slot] = make_float4(x[0], x[1], x[2], __int_as_float((int)p));
 }
 
+// Ascending order of 64 keys over a wave's lanes (bitonic); half: the keys are
+// already bitonic.
+__device__ __forceinline__ uint64_t wave_sort(uint64_t key, int lane, bool half) {
+  for (int k = half ? 64 : 2; k <= 64; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      const uint64_t other = __shfl_xor((unsigned long long)key, j);
+      const bool low = (lane & j) == 0, up = (lane & k) == 0;     // k == 64: ascending throughout
+      key = (low == up) == (key < other) ? key : other;
+    }
+  return key;
+}
+
+// A wave per query.  Distances and indices form one key, (bits of d, index),
+// whose order is theirs; lane l holds the l-th smallest key so far, a batch of
+// 64 candidates that holds a key below the K-th is sorted and merged in.  The
+// cells of a shell's row lie one after the other in spos, so a lane takes a
+// run of cells and the candidates of 64 runs spread over the lanes by their
+// prefix sums.  One thread per query walked its cells alone and carried the
+// sorted list in registers: with a few thousand points a handful of waves on a
+// chip of a thousand, 1.8 ms for 2,790 points; 20 us now.
 template <int K>
 __global__ __launch_bounds__(256) void knn_grid_kernel(gk_system sys, int64_t n, KnnGrid g, const int32_t* start,
                                                        const float4* spos, int32_t* idx, float* hk) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  static_assert(K <= 64, "one list entry per lane");
+  __shared__ int32_t s_pre[4][64], s_beg[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t p = (int64_t)blockIdx.x * 4 + wave;
   if (p >= n) return;
+  int32_t *pre = s_pre[wave], *beg = s_beg[wave];
   float x[3];
   norm_point(sys, p, 1.0 / sys.range, x);
   const int cx = cell_coord(x[0], g.lo[0], g.inv_c, g.n[0]), cy = cell_coord(x[1], g.lo[1], g.inv_c, g.n[1]),
             cz = cell_coord(x[2], g.lo[2], g.inv_c, g.n[2]);
-  float bd[K];
-  int32_t bi[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) { bd[j] = 3.4e38f; bi[j] = 0x7fffffff; }
+  constexpr uint64_t NONE = (uint64_t)0x7f7fffff << 32 | 0x7fffffff;     // no neighbour: FLT_MAX, no index
+  uint64_t best = NONE, worst = NONE;
   const int rmax = max(g.n[0], max(g.n[1], g.n[2]));
   for (int r = 0; r <= rmax; ++r) {
-    for (int dz = -r; dz <= r; ++dz) {
-      const int z = cz + dz;
-      if (z < 0 || z >= g.n[2]) continue;
-      for (int dy = -r; dy <= r; ++dy) {
-        const int y = cy + dy;
-        if (y < 0 || y >= g.n[1]) continue;
-        const bool inner = abs(dz) < r && abs(dy) < r;
-        for (int dx = -r; dx <= r; dx += (inner ? 2 * r : 1)) {   // only the shell of the cube
-          const int xx = cx + dx;
-          if (r > 0 && inner && dx != -r && dx != r) continue;
-          if (xx < 0 || xx >= g.n[0]) continue;
-          const int c = (z * g.n[1] + y) * g.n[0] + xx;
-          for (int s = start[c], e = start[c + 1]; s < e; ++s) {
-            const float4 q = spos[s];
-            const float ddx = q.x - x[0], ddy = q.y - x[1], ddz = q.z - x[2];
-            float d = fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx));
-            int32_t id = __float_as_int(q.w);
-            if (d < bd[K - 1] || (d == bd[K - 1] && id < bi[K - 1])) {
-#pragma unroll
-              for (int t = 0; t < K; ++t) {
-                if (d < bd[t] || (d == bd[t] && id < bi[t])) {
-                  const float td = bd[t];
-                  const int32_t ti = bi[t];
-                  bd[t] = d; bi[t] = id;
-                  d = td; id = ti;
-                }
-              }
-            }
-          }
-          if (r == 0) break;
+    // rows (z, y) of the cube of radius r inside the grid; an inner row gives
+    // the cell at either end, an outer one all its cells
+    const int z0 = max(cz - r, 0), z1 = min(cz + r, g.n[2] - 1), y0 = max(cy - r, 0), y1 = min(cy + r, g.n[1] - 1);
+    const int ny = y1 - y0 + 1, segs = 2 * (z1 - z0 + 1) * ny;
+    for (int base = 0; base < segs; base += 64) {
+      const int sg = base + lane;
+      int32_t b = 0, e = 0;
+      if (sg < segs) {
+        const int z = z0 + (sg >> 1) / ny, y = y0 + (sg >> 1) % ny;
+        const bool inner = abs(z - cz) < r && abs(y - cy) < r;
+        const int c0 = (z * g.n[1] + y) * g.n[0];
+        int xa = max(cx - r, 0), xb = min(cx + r, g.n[0] - 1);
+        if (inner) {
+          xa = xb = (sg & 1) ? cx + r : cx - r;
+          if (xa < 0 || xa >= g.n[0]) xb = xa - 1;
+        } else if (sg & 1) {
+          xb = xa - 1;
         }
+        if (xa <= xb) { b = start[c0 + xa]; e = start[c0 + xb + 1]; }
+      }
+      int32_t sum = e - b;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int32_t v = __shfl_up(sum, o);
+        if (lane >= o) sum += v;
+      }
+      __builtin_amdgcn_wave_barrier();
+      pre[lane] = sum - (e - b);
+      beg[lane] = b;
+      __builtin_amdgcn_wave_barrier();
+      const int32_t total = __shfl(sum, 63);
+      for (int32_t at = 0; at < total; at += 64) {
+        const int32_t c = at + lane;
+        uint64_t key = NONE;
+        if (c < total) {
+          int lo = 0;                    // the last run that starts at or before c
+          for (int o = 32; o > 0; o >>= 1)
+            if (pre[lo + o] <= c) lo += o;
+          const float4 q = spos[beg[lo] + c - pre[lo]];
+          const float ddx = q.x - x[0], ddy = q.y - x[1], ddz = q.z - x[2];
+          const float d = fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx));
+          key = (uint64_t)__float_as_uint(d) << 32 | (uint32_t)__float_as_int(q.w);
+        }
+        if (!__any(key < worst)) continue;
+        key = wave_sort(key, lane, false);
+        // the smaller half of two ascending lists, one reversed, is bitonic
+        const uint64_t rev = __shfl((unsigned long long)key, 63 - lane);
+        best = wave_sort(best < rev ? best : rev, lane, true);
+        worst = __shfl((unsigned long long)best, K - 1);
       }
     }
     // every point within r cell sizes of the query has been seen (a margin
     // for the rounding of the cell coordinates)
     const float reach = ((float)r - 1e-3f) * g.c;
-    if (bi[K - 1] != 0x7fffffff && bd[K - 1] <= reach * reach) break;
+    if (worst != NONE && __uint_as_float((uint32_t)(worst >> 32)) <= reach * reach) break;
   }
-#pragma unroll
-  for (int j = 0; j < K; ++j) idx[p * K + j] = bi[j];
-  hk[p] = sqrtf(bd[K - 1]);
+  if (lane < K) idx[p * K + lane] = (int32_t)(uint32_t)best;
+  if (lane == 0) hk[p] = sqrtf(__uint_as_float((uint32_t)(worst >> 32)));
 }
 
 // ------------------------------------------------------------------ features
@@ -281,111 +319,126 @@ __global__ __launch_bounds__(256) void local_blocks_kernel(Geo G, int64_t nq, co
 // identity) is symmetric positive definite; its unknowns are ordered with p's
 // own three last, so with H_loc = L L^T the wanted columns H_loc^-1 e_s are
 // L^-T z with z = L^-1 e_s nonzero only in its last three entries (the inverse
-// of L's last 3x3 block).  Cholesky in LDS (LD^3/6 multiply-adds, a third of a
-// Gauss-Jordan elimination's), then one wave solves L^T x = z for the three
-// columns with broadcasts instead of barriers.
+// of L's last 3x3 block).  A rest point has one unknown of its three slot rows;
+// the others are identity rows, which decouple exactly, so the matrix is
+// factored on the real unknowns only (the three rows of p itself are always
+// kept, last).
+// A wave per point, the lower triangle packed in LDS: column by column, lane l
+// rows k + l and k + 64 + l, each a dot product of two rows (no writes but the
+// column, no barriers); then L^T x = z for the three columns with broadcasts.
+// What bounds it is the chain of columns, so points side by side are what
+// helps: a workgroup of 256 threads per point with three barriers a column
+// took 1.28 ms for 2,790 points, two waves with a point each in the same LDS
+// 0.84 ms, and 0.47 ms on 256 workgroups (74 KB of LDS each, which leaves room
+// for one of the factorization's).
+constexpr int LI_WAVES = 2;
 template <int K>
-__global__ __launch_bounds__(256) void local_inverse_kernel(Geo G, int64_t n, const int32_t* idx,
-                                                            const double* dscale, float* Y) {
+__global__ __launch_bounds__(64 * LI_WAVES) void local_inverse_kernel(Geo G, int64_t n, const int32_t* idx,
+                                                                      const double* dscale, float* Y) {
   constexpr int LD = 3 * K;
-  __shared__ double A[LD][LD + 1];
-  __shared__ int64_t un[LD];
-  __shared__ int orig[LD];                // compact row -> slot row (3 slot + component)
-  __shared__ int self, nc;
-  const int tid = threadIdx.x;
+  static_assert(K <= 64 && LD <= 128, "a lane per slot, two rows per lane");
+  __shared__ double s_A[LI_WAVES][LD * (LD + 1) / 2];
+  __shared__ int32_t s_un[LI_WAVES][LD], s_orig[LI_WAVES][LD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double* A = s_A[wave];
+  int32_t *un = s_un[wave], *orig = s_orig[wave];        // of each compact row: its unknown, its slot row
+  auto at = [](int r, int c) { return r * (r + 1) / 2 + c; };
   // a fixed grid walks the points: the kernel holds at most gridDim.x CUs'
   // worth of LDS, so a factorization running beside it keeps the rest
-  for (int64_t p = blockIdx.x; p < n; p += gridDim.x) {
-  __syncthreads();
-  if (tid == 0) {
-    self = 0;
-    for (int j = 0; j < K; ++j)
-      if (idx[p * K + j] == p) { self = j; break; }
-  }
-  __syncthreads();
-  // slot s < K - 1: neighbour s (s + 1 past self); slot K - 1: p itself.
-  // A rest point has one unknown of its three slot rows; the others are
-  // identity rows, which decouple exactly, so the matrix is factored on the
-  // real unknowns only (the three rows of p itself are always kept, last).
-  if (tid < LD) {
-    const int sl = tid / 3, d = tid % 3;
-    const int j = sl == K - 1 ? self : (sl < self ? sl : sl + 1);
-    un[tid] = unknown_of(G.s, idx[p * K + j], d);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int c = 0;
-    for (int r = 0; r < LD; ++r)
-      if (un[r] >= 0 || r >= LD - 3) orig[c++] = r;
-    nc = c;
-  }
-  __syncthreads();
-  const int m_all = nc;
-  for (int e = tid; e < m_all * m_all; e += 256) {
-    const int r = e / m_all, c = e % m_all;
-    if (c > r) continue;
-    const int64_t ur = un[orig[r]], uc = un[orig[c]];
-    A[r][c] = (ur < 0 || uc < 0) ? (r == c ? 1.0 : 0.0) : entry(G, ur, uc) * dscale[ur] * dscale[uc];
-  }
-  __syncthreads();
-  for (int k = 0; k < m_all; ++k) {
-    if (tid == 0) A[k][k] = sqrt(A[k][k]);
-    __syncthreads();
-    const double ip = 1.0 / A[k][k];
-    for (int r = k + 1 + tid; r < m_all; r += 256) A[r][k] *= ip;
-    __syncthreads();
-    // trailing lower triangle: rows k+1+i (16 thread groups), columns k+1+t <= row
-    const int m = m_all - k - 1;
-    for (int i = tid >> 4; i < m; i += 16) {
-      const double ark = A[k + 1 + i][k];
-      for (int t = tid & 15; t <= i; t += 16) A[k + 1 + i][k + 1 + t] -= ark * A[k + 1 + t][k];
+  for (int64_t p = (int64_t)blockIdx.x * LI_WAVES + wave; p < n; p += (int64_t)gridDim.x * LI_WAVES) {
+    // slot s < K - 1: neighbour s (s + 1 past self); slot K - 1: p itself
+    const uint64_t own = __ballot(lane < K && idx[p * K + (lane < K ? lane : 0)] == p);
+    const int self = own ? __ffsll((unsigned long long)own) - 1 : 0;
+    const int slot_j = lane == K - 1 ? self : (lane < self ? lane : lane + 1);   // neighbour of slot `lane`
+    const int64_t q = lane < K ? idx[p * K + slot_j] : 0;
+    const int rows = lane >= K ? 0 : (lane == K - 1 || q < G.s.n_ori ? 3 : 1);
+    int end = rows;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(end, o);
+      if (lane >= o) end += v;
     }
-    __syncthreads();
-  }
-  if (tid < 64) {
+    const int m_all = __shfl(end, K - 1);
+    __builtin_amdgcn_wave_barrier();
+    for (int d = 0; d < rows; ++d) {
+      un[end - rows + d] = (int32_t)unknown_of(G.s, q, d);
+      orig[end - rows + d] = 3 * lane + d;
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int cells = m_all * (m_all + 1) / 2;
+    for (int e = lane; e < cells; e += 64) {
+      int r = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
+      while (at(r + 1, 0) <= e) ++r;
+      while (at(r, 0) > e) --r;
+      const int c = e - at(r, 0);
+      const int64_t ur = un[r], uc = un[c];
+      A[e] = (ur < 0 || uc < 0) ? (r == c ? 1.0 : 0.0) : entry(G, ur, uc) * dscale[ur] * dscale[uc];
+    }
+    __builtin_amdgcn_wave_barrier();
+    for (int k = 0; k < m_all; ++k) {
+      const int r0 = k + lane, r1 = r0 + 64;
+      const double* Ak = A + at(k, 0);
+      const double *A0 = A + at(min(r0, m_all - 1), 0), *A1 = A + at(min(r1, m_all - 1), 0);
+      double v0 = A0[k], v1 = A1[k];
+      if (m_all - k > 64) {
+#pragma unroll 4
+        for (int j = 0; j < k; ++j) {
+          const double b = Ak[j];
+          v0 = fma(-A0[j], b, v0);
+          v1 = fma(-A1[j], b, v1);
+        }
+      } else {
+#pragma unroll 8
+        for (int j = 0; j < k; ++j) v0 = fma(-A0[j], Ak[j], v0);
+      }
+      const double piv = sqrt(__shfl(v0, 0)), ip = 1.0 / piv;
+      __builtin_amdgcn_wave_barrier();
+      if (r0 < m_all) A[at(r0, k)] = lane == 0 ? piv : v0 * ip;
+      if (r1 < m_all) A[at(r1, k)] = v1 * ip;
+      __builtin_amdgcn_wave_barrier();
+    }
     // z = L^-1 e_{n-3+q}: only z[n-3 .. n-1] are nonzero (forward substitution
     // on L's last 3x3 block), then x = L^-T z; lane l owns rows l, l + 64
     constexpr int RPL = (LD + 63) / 64;
     double x[RPL][3];
     const int b0 = m_all - 3;
-    const double l00 = A[b0][b0], l10 = A[b0 + 1][b0], l11 = A[b0 + 1][b0 + 1];
-    const double l20 = A[b0 + 2][b0], l21 = A[b0 + 2][b0 + 1], l22 = A[b0 + 2][b0 + 2];
+    const double l00 = A[at(b0, b0)], l10 = A[at(b0 + 1, b0)], l11 = A[at(b0 + 1, b0 + 1)];
+    const double l20 = A[at(b0 + 2, b0)], l21 = A[at(b0 + 2, b0 + 1)], l22 = A[at(b0 + 2, b0 + 2)];
     double z[3][3];                      // z[q][t]: column q, entry b0 + t
-    for (int q = 0; q < 3; ++q) {
-      const double e0 = q == 0, e1 = q == 1, e2 = q == 2;
-      z[q][0] = e0 / l00;
-      z[q][1] = (e1 - l10 * z[q][0]) / l11;
-      z[q][2] = (e2 - l20 * z[q][0] - l21 * z[q][1]) / l22;
+#pragma unroll
+    for (int q3 = 0; q3 < 3; ++q3) {
+      const double e0 = q3 == 0, e1 = q3 == 1, e2 = q3 == 2;
+      z[q3][0] = e0 / l00;
+      z[q3][1] = (e1 - l10 * z[q3][0]) / l11;
+      z[q3][2] = (e2 - l20 * z[q3][0] - l21 * z[q3][1]) / l22;
     }
 #pragma unroll
     for (int u = 0; u < RPL; ++u) {
-      const int r = tid + 64 * u;
+      const int t = lane + 64 * u - b0;
 #pragma unroll
-      for (int q = 0; q < 3; ++q) x[u][q] = r >= b0 && r < m_all ? z[q][r - b0] : 0.0;
+      for (int q3 = 0; q3 < 3; ++q3) x[u][q3] = t == 0 ? z[q3][0] : (t == 1 ? z[q3][1] : (t == 2 ? z[q3][2] : 0.0));
     }
     for (int k = m_all - 1; k >= 0; --k) {
-      const double ikk = 1.0 / A[k][k];
+      const double ikk = 1.0 / A[at(k, k)];
       const int owner = k & 63, uo = k >> 6;
       double xk[3];
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
+      for (int q3 = 0; q3 < 3; ++q3) {
         double v = 0.0;
 #pragma unroll
         for (int u = 0; u < RPL; ++u)
-          if (u == uo) v = x[u][q];
-        v = __shfl(v, owner) * ikk;          // x_k = (z_k - sum_{i>k} L_ik x_i) / L_kk
-        xk[q] = v;
+          if (u == uo) v = x[u][q3];
+        xk[q3] = __shfl(v, owner) * ikk;     // x_k = (z_k - sum_{i>k} L_ik x_i) / L_kk
       }
 #pragma unroll
       for (int u = 0; u < RPL; ++u) {
-        const int r = tid + 64 * u;
+        const int r = lane + 64 * u;
         if (r == k) {
 #pragma unroll
-          for (int q = 0; q < 3; ++q) x[u][q] = xk[q];
+          for (int q3 = 0; q3 < 3; ++q3) x[u][q3] = xk[q3];
         } else if (r < k) {
-          const double lkr = A[k][r];
+          const double lkr = A[at(k, r)];
 #pragma unroll
-          for (int q = 0; q < 3; ++q) x[u][q] -= lkr * xk[q];
+          for (int q3 = 0; q3 < 3; ++q3) x[u][q3] -= lkr * xk[q3];
         }
       }
     }
@@ -393,23 +446,19 @@ __global__ __launch_bounds__(256) void local_inverse_kernel(Geo G, int64_t n, co
     // the rows of identity unknowns (not factored) hold 0
 #pragma unroll
     for (int u = 0; u < RPL; ++u) {
-      const int row = tid + 64 * u;
+      const int row = lane + 64 * u;
       if (row >= m_all) continue;
-      const int orow = orig[row];
-      const int sl = orow / 3, c = orow % 3;
+      const int sl = orig[row] / 3, c = orig[row] % 3;
       const int j = sl == K - 1 ? self : (sl < self ? sl : sl + 1);
 #pragma unroll
-      for (int q = 0; q < 3; ++q) Y[((int64_t)p * K + j) * 9 + 3 * q + c] = (float)x[u][q];
+      for (int q3 = 0; q3 < 3; ++q3) Y[((int64_t)p * K + j) * 9 + 3 * q3 + c] = (float)x[u][q3];
     }
-  }
-  // zeros for the slot rows left out (identity unknowns of neighbours)
-  for (int row = tid; row < LD - 3; row += 256) {
-    if (un[row] >= 0) continue;
-    const int sl = row / 3, c = row % 3;
-    const int j = sl < self ? sl : sl + 1;
+    if (rows == 1)
 #pragma unroll
-    for (int q = 0; q < 3; ++q) Y[((int64_t)p * K + j) * 9 + 3 * q + c] = 0.0f;
-  }
+      for (int c = 1; c < 3; ++c)
+#pragma unroll
+        for (int q3 = 0; q3 < 3; ++q3) Y[((int64_t)p * K + slot_j) * 9 + 3 * q3 + c] = 0.0f;
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -665,7 +714,7 @@ extern "C" int gk_knn_local(gk_handle h, const gk_system* sys, const double* box
   hipLaunchKernelGGL(knn_cells_kernel, dim3(nb), dim3(256), 0, st, *sys, n, g, cell, count);
   hipLaunchKernelGGL(knn_scan_kernel, dim3(1), dim3(1024), 0, st, count, nc, start);
   hipLaunchKernelGGL(knn_scatter_kernel, dim3(nb), dim3(256), 0, st, *sys, n, cell, start, fill, spos);
-  hipLaunchKernelGGL(knn_grid_kernel<GK_LOCAL_K>, dim3(nb), dim3(256), 0, st, *sys, n, g, start, spos, idx, hk);
+  hipLaunchKernelGGL(knn_grid_kernel<GK_LOCAL_K>, dim3((unsigned)gk_ceil_div(n, 4)), dim3(256), 0, st, *sys, n, g, start, spos, idx, hk);
   GK_HIP(hipGetLastError());
   return GK_OK;
 }
@@ -683,7 +732,8 @@ extern "C" int gk_local_inverse_local(gk_handle h, const gk_system* sys, const i
   const int64_t n = sys->n_ori + sys->n_rest;
   if (n == 0) return GK_OK;
   // a fixed grid (the work spreads over the factorization it runs beside)
-  hipLaunchKernelGGL(local_inverse_kernel<GK_LOCAL_K>, dim3((unsigned)std::min<int64_t>(n, GK_LI_GRID)), dim3(256), 0,
+  hipLaunchKernelGGL(local_inverse_kernel<GK_LOCAL_K>,
+                     dim3((unsigned)std::min<int64_t>(gk_ceil_div(n, LI_WAVES), GK_LI_GRID)), dim3(64 * LI_WAVES), 0,
                      (hipStream_t)stream, make_geo(sys), n, idx, dscale, Y);
   GK_HIP(hipGetLastError());
   return GK_OK;
@@ -729,8 +779,8 @@ extern "C" int gk_spai_local_inverse(gk_handle h, const gk_system* sys, const in
   GK_REQUIRE(h && sys && idx && dscale && Y, GK_ERR_ARG, "gk_spai_local_inverse: bad arguments");
   const int64_t n = sys->n_ori + sys->n_rest;
   if (n == 0) return GK_OK;
-  hipLaunchKernelGGL(local_inverse_kernel<K>, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream, make_geo(sys), n,
-                     idx, dscale, Y);
+  hipLaunchKernelGGL(local_inverse_kernel<K>, dim3((unsigned)gk_ceil_div(n, LI_WAVES)), dim3(64 * LI_WAVES), 0,
+                     (hipStream_t)stream, make_geo(sys), n, idx, dscale, Y);
   GK_HIP(hipGetLastError());
   return GK_OK;
 }
