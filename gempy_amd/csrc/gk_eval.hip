@@ -908,59 +908,126 @@ __global__ __launch_bounds__(FIN_PTS * FIN_LANES) void eval_finalize_kernel(Eval
 // with weight -i_res c_o W_s (W_s = sum of w_i over the surface): the
 // rest-minus-reference differencing of the interface covariance collapses
 // into per-surface reference sources.
-__global__ __launch_bounds__(1024) void surface_sums_kernel(const double* wI, const int32_t* surf, int64_t R,
-                                                             double* W) {
-  __shared__ double red[16];
-  const int s = blockIdx.x;
-  double acc = 0.0;
-  for (int64_t i = threadIdx.x; i < R; i += 1024)
-    if (surf[i] == s) acc += wI[i];
+// One launch prepares everything an evaluation reads, the workgroups taking
+// roles one after the other: a surface each (its sum of weights and its
+// reference source), 1,024 rest points, 1,024 orientations; for the operator
+// product also the data points' positions and the partial sums of its drift
+// and fault rows, which depend on x alone.  These were four to six launches
+// one after the other, each of them shorter than the gap between two: a
+// product of 1,800 data took 49 us and takes 40 now, of 25,000 data 447 and
+// 430.
+//
+// Drift and fault rows: workgroup (l, c) adds chunk c of row l's terms (the
+// orientations and rest points split into DRIFT_CHUNKS ranges) into
+// part[l DRIFT_CHUNKS + c]; matvec_combine_kernel adds the chunks in order.
+constexpr int DRIFT_CHUNKS = 16, PREP = 1024;
+
+__device__ __forceinline__ double block_sum(double acc, double* red) {   // PREP threads; valid in thread 0
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < 16; ++w) t += red[w];
-    W[s] = t;
+  double t = 0.0;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < PREP / 64; ++w) t += red[w];
+  return t;
+}
+
+__device__ __forceinline__ double drift_row_chunk(const gk_system& sys, const double* x, int l, int c) {
+  const int64_t no = sys.n_ori, R = sys.n_rest, NG = 3 * no;
+  const int L = sys.uni_degree == 0 ? 0 : (sys.uni_degree == 1 ? 3 : 9);
+  const int64_t g0 = no * c / DRIFT_CHUNKS, g1 = no * (c + 1) / DRIFT_CHUNKS;
+  const int64_t r0 = R * c / DRIFT_CHUNKS, r1 = R * (c + 1) / DRIFT_CHUNKS;
+  double acc = 0.0;
+  if (l < L) {
+    for (int64_t g = g0 + threadIdx.x; g < g1; g += PREP) {
+      const double* q = sys.ori_xyz + 3 * g;
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        double df;
+        if (l < 3) df = (l == u) ? 1.0 : 0.0;
+        else if (l < 6) df = (l - 3 == u) ? 2.0 * q[u] : 0.0;
+        else if (l == 6) df = (u == 0) ? q[1] : (u == 1 ? q[0] : 0.0);
+        else if (l == 7) df = (u == 0) ? q[2] : (u == 2 ? q[0] : 0.0);
+        else df = (u == 1) ? q[2] : (u == 2 ? q[1] : 0.0);
+        acc += df * x[u * no + g];
+      }
+    }
+    for (int64_t r = r0 + threadIdx.x; r < r1; r += PREP) {
+      const double* p = sys.rest_xyz + 3 * r;
+      const double* p0 = sys.ref_xyz + 3 * sys.rest_surf[r];
+      double f1, f0;
+      if (l < 3) { f1 = p[l]; f0 = p0[l]; }
+      else if (l < 6) { f1 = p[l - 3] * p[l - 3]; f0 = p0[l - 3] * p0[l - 3]; }
+      else if (l == 6) { f1 = p[0] * p[1]; f0 = p0[0] * p0[1]; }
+      else if (l == 7) { f1 = p[0] * p[2]; f0 = p0[0] * p0[2]; }
+      else { f1 = p[1] * p[2]; f0 = p0[1] * p0[2]; }
+      acc += sys.gi_res * (f1 - f0) * x[NG + r];
+    }
+  } else {
+    for (int64_t r = r0 + threadIdx.x; r < r1; r += PREP)
+      acc += sys.gi_res * sys.fault_rest[r * sys.n_fault + (l - L)] * x[NG + r];
   }
+  return acc;
 }
 
+// xyz, drift (nullable): the operator product's.  drift_rows of them.
 template <typename T>
-__global__ void prep_pts_kernel(gk_system sys, const double* w, const double* W, V4<T>* out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t R = sys.n_rest, S = sys.n_surf;
-  if (i >= R + S) return;
+__global__ __launch_bounds__(PREP) void prep_kernel(gk_system sys, const double* w, V4<T>* pts, V8<T>* ori, double* xyz,
+                                                    double* drift, int drift_rows) {
+  __shared__ double red[PREP / 64];
+  const int64_t R = sys.n_rest, S = sys.n_surf, no = sys.n_ori;
   const double inv_a = 1.0 / sys.range;
-  const double* p;
-  double wt;
-  if (i < R) { p = sys.rest_xyz + 3 * i; wt = sys.i_res * sys.c_o * w[3 * sys.n_ori + i]; }
-  else { p = sys.ref_xyz + 3 * (i - R); wt = -sys.i_res * sys.c_o * W[i - R]; }
-  V4<T> v;
-  v.x = (T)((p[0] - sys.center[0]) * inv_a);
-  v.y = (T)((p[1] - sys.center[1]) * inv_a);
-  v.z = (T)((p[2] - sys.center[2]) * inv_a);
-  v.w = (T)wt;
-  out[i] = v;
-}
-
-template <typename T>
-__global__ void prep_ori_kernel(gk_system sys, const double* w, V8<T>* out) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = sys.n_ori;
-  if (g >= n) return;
-  const double inv_a = 1.0 / sys.range;
-  const double f = sys.gi_res * sys.c_o * inv_a;
-  const double* q = sys.ori_xyz + 3 * g;
-  V8<T> v;
-  v.x = (T)((q[0] - sys.center[0]) * inv_a);
-  v.y = (T)((q[1] - sys.center[1]) * inv_a);
-  v.z = (T)((q[2] - sys.center[2]) * inv_a);
-  v.pad0 = T(0);
-  v.wx = (T)(f * w[g]);
-  v.wy = (T)(f * w[n + g]);
-  v.wz = (T)(f * w[2 * n + g]);
-  v.pad1 = T(0);
-  out[g] = v;
+  auto put = [&](int64_t i, const double* p, double wt) {
+    V4<T> v;
+    v.x = (T)((p[0] - sys.center[0]) * inv_a);
+    v.y = (T)((p[1] - sys.center[1]) * inv_a);
+    v.z = (T)((p[2] - sys.center[2]) * inv_a);
+    v.w = (T)wt;
+    pts[i] = v;
+    if (xyz) { xyz[3 * i] = p[0]; xyz[3 * i + 1] = p[1]; xyz[3 * i + 2] = p[2]; }
+  };
+  int64_t b = blockIdx.x;
+  if (b < S) {                           // a surface
+    double acc = 0.0;
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i < R; i += PREP) {
+      const double wi = w[3 * no + i];
+      acc += sys.rest_surf[i] == b ? wi : 0.0;
+    }
+    const double W = block_sum(acc, red);
+    if (threadIdx.x == 0) put(R + b, sys.ref_xyz + 3 * b, -sys.i_res * sys.c_o * W);
+    return;
+  }
+  b -= S;
+  const int64_t nr = (R + PREP - 1) / PREP, nq = (no + PREP - 1) / PREP;
+  if (b < nr) {
+    const int64_t i = b * PREP + threadIdx.x;
+    if (i < R) put(i, sys.rest_xyz + 3 * i, sys.i_res * sys.c_o * w[3 * no + i]);
+    return;
+  }
+  b -= nr;
+  if (b < nq) {
+    const int64_t g = b * PREP + threadIdx.x;
+    if (g >= no) return;
+    const double f = sys.gi_res * sys.c_o * inv_a;
+    const double* q = sys.ori_xyz + 3 * g;
+    V8<T> v;
+    v.x = (T)((q[0] - sys.center[0]) * inv_a);
+    v.y = (T)((q[1] - sys.center[1]) * inv_a);
+    v.z = (T)((q[2] - sys.center[2]) * inv_a);
+    v.pad0 = T(0);
+    v.wx = (T)(f * w[g]);
+    v.wy = (T)(f * w[no + g]);
+    v.wz = (T)(f * w[2 * no + g]);
+    v.pad1 = T(0);
+    ori[g] = v;
+    return;
+  }
+  b -= nq;
+  if (b < (int64_t)drift_rows * DRIFT_CHUNKS) {
+    const double t = block_sum(drift_row_chunk(sys, w, (int)(b / DRIFT_CHUNKS), (int)(b % DRIFT_CHUNKS)), red);
+    if (threadIdx.x == 0) drift[b] = t;
+  }
 }
 
 int n_drift_of(int deg) { return deg == 0 ? 0 : (deg == 1 ? 3 : 9); }
@@ -1007,43 +1074,28 @@ void dispatch_eval(const EvalArgs& a, bool lattice, bool grad, bool masked, hipS
 
 }  // namespace
 
-// Prepare the packed sources for `weights` in the handle workspace.
-// Layout: [W_s (n_surf doubles, 256-B aligned) | pts V4<T> (R+S) | ori V8<T> (n_ori)].
-static int prepare_sources(gk_handle h, const gk_system* sys, const double* weights, int precision,
-                           hipStream_t st, const void** pts, const void** ori, void* ws, bool launch = true) {
-  const int64_t R = sys->n_rest, S = sys->n_surf, no = sys->n_ori;
+// Where the packed sources lie in a workspace: [pts V4<T> (R+S) | ori V8<T> (n_ori)].
+static void source_layout(const gk_system* sys, int precision, void* ws, void** pts, void** ori) {
   const size_t tsz = precision == GK_F64 ? 8 : 4;
-  char* base = static_cast<char*>(ws);
-  double* W = reinterpret_cast<double*>(base);
-  size_t off = gk_round_up(S * 8, 256);
-  void* p4 = base + off;
-  off += gk_round_up((R + S) * 4 * tsz, 256);
-  void* p8 = base + off;
-  (void)h;
-  *pts = p4;
-  *ori = p8;
-  if (!launch) return GK_OK;             // sources already prepared for these weights
-  if (S > 0)
-    hipLaunchKernelGGL(surface_sums_kernel, dim3((unsigned)S), dim3(1024), 0, st,
-                       weights + 3 * no, sys->rest_surf, R, W);
-  if (R + S > 0) {
-    unsigned nb = (unsigned)gk_ceil_div(R + S, 256);
-    if (precision == GK_F64)
-      hipLaunchKernelGGL(prep_pts_kernel<double>, dim3(nb), dim3(256), 0, st, *sys, weights, W,
-                         reinterpret_cast<V4<double>*>(p4));
-    else
-      hipLaunchKernelGGL(prep_pts_kernel<float>, dim3(nb), dim3(256), 0, st, *sys, weights, W,
-                         reinterpret_cast<V4<float>*>(p4));
-  }
-  if (no > 0) {
-    unsigned nb = (unsigned)gk_ceil_div(no, 256);
-    if (precision == GK_F64)
-      hipLaunchKernelGGL(prep_ori_kernel<double>, dim3(nb), dim3(256), 0, st, *sys, weights,
-                         reinterpret_cast<V8<double>*>(p8));
-    else
-      hipLaunchKernelGGL(prep_ori_kernel<float>, dim3(nb), dim3(256), 0, st, *sys, weights,
-                         reinterpret_cast<V8<float>*>(p8));
-  }
+  *pts = ws;
+  *ori = static_cast<char*>(ws) + gk_round_up((sys->n_rest + sys->n_surf) * 4 * tsz, 256);
+}
+
+// Prepare the packed sources for `weights` in the workspace ws; xyz, drift,
+// drift_rows: see prep_kernel.
+static int prepare_sources(const gk_system* sys, const double* weights, int precision, hipStream_t st, void* ws,
+                           double* xyz = nullptr, double* drift = nullptr, int drift_rows = 0) {
+  const int64_t nb = sys->n_surf + gk_ceil_div(sys->n_rest, PREP) + gk_ceil_div(sys->n_ori, PREP) +
+                     (int64_t)drift_rows * DRIFT_CHUNKS;
+  void *p4, *p8;
+  source_layout(sys, precision, ws, &p4, &p8);
+  if (nb == 0) return GK_OK;
+  if (precision == GK_F64)
+    hipLaunchKernelGGL(prep_kernel<double>, dim3((unsigned)nb), dim3(PREP), 0, st, *sys, weights,
+                       static_cast<V4<double>*>(p4), static_cast<V8<double>*>(p8), xyz, drift, drift_rows);
+  else
+    hipLaunchKernelGGL(prep_kernel<float>, dim3((unsigned)nb), dim3(PREP), 0, st, *sys, weights,
+                       static_cast<V4<float>*>(p4), static_cast<V8<float>*>(p8), xyz, drift, drift_rows);
   GK_HIP(hipGetLastError());
   return GK_OK;
 }
@@ -1340,7 +1392,11 @@ static int eval_impl(gk_handle h, const gk_system* sys, const double* weights, g
   } else {
     GK_TRY(gk_workspace(h, WS_EVAL_SRC, sources_bytes(sys), &ws));
   }
-  GK_TRY(prepare_sources(h, sys, weights, d->precision, st, &a.pts, &a.ori, ws, !reuse_sources));
+  void *pts = nullptr, *ori = nullptr;
+  source_layout(sys, d->precision, ws, &pts, &ori);
+  a.pts = pts;
+  a.ori = ori;
+  if (!reuse_sources) GK_TRY(prepare_sources(sys, weights, d->precision, st, ws));
   bool masked = true;
   if (!force_mask && src_box) {
     // explicit points: only callers whose points lie inside the source box
@@ -1369,98 +1425,36 @@ static int eval_impl(gk_handle h, const gk_system* sys, const double* weights, g
 
 // ------------------------------------------------------------------ matvec
 namespace {
-// y rows from the evaluated field at the data points.
-__global__ void matvec_combine_kernel(gk_system sys, const double* x, const double* s_data,
-                                      const double* g_ori, double* y) {
+// y rows from the evaluated field at the data points (the fault drift enters
+// the interface rows here); the last workgroup adds the chunks of the drift
+// and fault rows.
+__global__ void matvec_combine_kernel(gk_system sys, const double* x, const double* s_data, const double* g_ori,
+                                      const double* drift, int drift_rows, double* y) {
+  const int64_t no = sys.n_ori, R = sys.n_rest, NG = 3 * no;
+  if (drift_rows > 0 && blockIdx.x + 1 == gridDim.x) {
+    const int l = threadIdx.x;
+    if (l >= drift_rows) return;
+    double t = 0.0;
+    for (int c = 0; c < DRIFT_CHUNKS; ++c) t += drift[l * DRIFT_CHUNKS + c];
+    y[NG + R + l] = t;
+    return;
+  }
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t no = sys.n_ori, R = sys.n_rest;
-  const int64_t NG = 3 * no;
   if (i < NG) {
     const int64_t u = i / no, g = i % no;
     y[i] = g_ori[3 * g + u] / sys.gi_res + sys.ori_nugget[g] * x[i];
   } else if (i < NG + R) {
     const int64_t r = i - NG;
     double v = s_data[r] - s_data[R + sys.rest_surf[r]] + sys.rest_nugget[r] * x[i];
+    if (sys.n_fault > 0) {
+      const int L = sys.uni_degree == 0 ? 0 : (sys.uni_degree == 1 ? 3 : 9);
+      double t = 0.0;
+      for (int f = 0; f < sys.n_fault; ++f)
+        t += sys.gi_res * sys.fault_rest[r * sys.n_fault + f] * x[NG + R + L + f];
+      v += t;
+    }
     y[i] = v;
   }
-}
-
-// Drift / fault rows: deterministic block reductions, one block per row.
-// Drift rows: y[NG+R+l] = sum over the orientation and interface unknowns of
-// the drift function's derivative / difference times x (one workgroup per row).
-// Drift and fault rows: block (l, c) adds chunk c of row l's terms (the
-// orientations and rest points split into DRIFT_CHUNKS ranges) into
-// part[l DRIFT_CHUNKS + c]; matvec_drift_sum_kernel adds the chunks in order.
-constexpr int DRIFT_CHUNKS = 16;
-__global__ __launch_bounds__(256) void matvec_drift_rows_kernel(gk_system sys, const double* x, double* part) {
-  __shared__ double red[4];
-  const int l = blockIdx.x, c = blockIdx.y;  // row 0..L+F-1, chunk
-  const int64_t no = sys.n_ori, R = sys.n_rest, NG = 3 * no;
-  const int L = sys.uni_degree == 0 ? 0 : (sys.uni_degree == 1 ? 3 : 9);
-  const int64_t g0 = no * c / DRIFT_CHUNKS, g1 = no * (c + 1) / DRIFT_CHUNKS;
-  const int64_t r0 = R * c / DRIFT_CHUNKS, r1 = R * (c + 1) / DRIFT_CHUNKS;
-  double acc = 0.0;
-  if (l < L) {
-    for (int64_t g = g0 + threadIdx.x; g < g1; g += 256) {
-      const double* q = sys.ori_xyz + 3 * g;
-#pragma unroll
-      for (int u = 0; u < 3; ++u) {
-        double df;
-        if (l < 3) df = (l == u) ? 1.0 : 0.0;
-        else if (l < 6) df = (l - 3 == u) ? 2.0 * q[u] : 0.0;
-        else if (l == 6) df = (u == 0) ? q[1] : (u == 1 ? q[0] : 0.0);
-        else if (l == 7) df = (u == 0) ? q[2] : (u == 2 ? q[0] : 0.0);
-        else df = (u == 1) ? q[2] : (u == 2 ? q[1] : 0.0);
-        acc += df * x[u * no + g];
-      }
-    }
-    for (int64_t r = r0 + threadIdx.x; r < r1; r += 256) {
-      const double* p = sys.rest_xyz + 3 * r;
-      const double* p0 = sys.ref_xyz + 3 * sys.rest_surf[r];
-      double f1, f0;
-      if (l < 3) { f1 = p[l]; f0 = p0[l]; }
-      else if (l < 6) { f1 = p[l - 3] * p[l - 3]; f0 = p0[l - 3] * p0[l - 3]; }
-      else if (l == 6) { f1 = p[0] * p[1]; f0 = p0[0] * p0[1]; }
-      else if (l == 7) { f1 = p[0] * p[2]; f0 = p0[0] * p0[2]; }
-      else { f1 = p[1] * p[2]; f0 = p0[1] * p0[2]; }
-      acc += sys.gi_res * (f1 - f0) * x[NG + r];
-    }
-  } else {
-    for (int64_t r = r0 + threadIdx.x; r < r1; r += 256)
-      acc += sys.gi_res * sys.fault_rest[r * sys.n_fault + (l - L)] * x[NG + r];
-  }
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) part[l * DRIFT_CHUNKS + c] = (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-__global__ void matvec_drift_sum_kernel(const double* part, int rows, double* y) {
-  const int l = threadIdx.x;
-  if (l >= rows) return;
-  double t = 0.0;
-  for (int c = 0; c < DRIFT_CHUNKS; ++c) t += part[l * DRIFT_CHUNKS + c];
-  y[l] = t;
-}
-
-// Fault-drift contribution to the interface rows (not part of the field eval).
-__global__ void matvec_fault_rows_kernel(gk_system sys, const double* x, double* y) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= sys.n_rest) return;
-  const int L = sys.uni_degree == 0 ? 0 : (sys.uni_degree == 1 ? 3 : 9);
-  const int64_t NG = 3 * sys.n_ori, R = sys.n_rest;
-  double v = 0.0;
-  for (int f = 0; f < sys.n_fault; ++f)
-    v += sys.gi_res * sys.fault_rest[r * sys.n_fault + f] * x[NG + R + L + f];
-  y[NG + r] += v;
-}
-
-__global__ void gather_data_points_kernel(gk_system sys, double* pts) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t R = sys.n_rest, S = sys.n_surf;
-  if (i >= R + S) return;
-  const double* p = i < R ? sys.rest_xyz + 3 * i : sys.ref_xyz + 3 * (i - R);
-  pts[3 * i] = p[0]; pts[3 * i + 1] = p[1]; pts[3 * i + 2] = p[2];
 }
 }  // namespace
 
@@ -1473,9 +1467,11 @@ extern "C" int gk_matvec_impl(gk_handle h, const gk_system* sys, int32_t precisi
   double* s_ori = s_data + (R + S);
   double* g_ori = s_ori + no;
   double* d_part = g_ori + 3 * no;          // drift / fault row chunks
-  if (R + S > 0)
-    hipLaunchKernelGGL(gather_data_points_kernel, dim3((unsigned)gk_ceil_div(R + S, 256)), dim3(256),
-                       0, st, *sys, pts);
+  GK_TRY(check_system(sys));
+  const int drift_rows = n_drift_of(sys->uni_degree) + sys->n_fault;
+  void* ws = nullptr;
+  GK_TRY(gk_workspace(h, WS_EVAL_SRC, sources_bytes(sys), &ws));
+  GK_TRY(prepare_sources(sys, x, precision, st, ws, pts, d_part, drift_rows));
   gk_system nofault = *sys;
   nofault.n_fault = 0;  // fault drift enters the interface rows separately
   if (R + S > 0) {
@@ -1485,7 +1481,7 @@ extern "C" int gk_matvec_impl(gk_handle h, const gk_system* sys, int32_t precisi
     d.n_points = R + S;
     d.xyz = pts;
     d.scalar = s_data;
-    GK_TRY(gk_eval_impl(h, &nofault, x, &d, st, src_box == nullptr, src_box, false));
+    GK_TRY(gk_eval_impl(h, &nofault, x, &d, st, src_box == nullptr, src_box, true));
   }
   if (no > 0) {
     gk_eval_desc d{};
@@ -1495,21 +1491,12 @@ extern "C" int gk_matvec_impl(gk_handle h, const gk_system* sys, int32_t precisi
     d.xyz = sys->ori_xyz;
     d.scalar = s_ori;             // drift terms only: the rows take the gradient
     d.gradient = g_ori;
-    GK_TRY(eval_impl(h, &nofault, x, &d, st, src_box == nullptr, src_box, R + S > 0, nullptr, 0, true));
+    GK_TRY(eval_impl(h, &nofault, x, &d, st, src_box == nullptr, src_box, true, nullptr, 0, true));
   }
-  const int64_t NG = 3 * no;
-  if (NG + R > 0)
-    hipLaunchKernelGGL(matvec_combine_kernel, dim3((unsigned)gk_ceil_div(NG + R, 256)), dim3(256), 0,
-                       st, *sys, x, s_data, g_ori, y);
-  if (sys->n_fault > 0 && R > 0)
-    hipLaunchKernelGGL(matvec_fault_rows_kernel, dim3((unsigned)gk_ceil_div(R, 256)), dim3(256), 0,
-                       st, *sys, x, y);
-  const int L = n_drift_of(sys->uni_degree);
-  if (L + sys->n_fault > 0) {
-    hipLaunchKernelGGL(matvec_drift_rows_kernel, dim3(L + sys->n_fault, DRIFT_CHUNKS), dim3(256), 0, st, *sys, x,
-                       d_part);
-    hipLaunchKernelGGL(matvec_drift_sum_kernel, dim3(1), dim3(32), 0, st, d_part, L + sys->n_fault, y + NG + R);
-  }
+  const int64_t nb = gk_ceil_div(3 * no + R, 256) + (drift_rows > 0 ? 1 : 0);
+  if (nb > 0)
+    hipLaunchKernelGGL(matvec_combine_kernel, dim3((unsigned)nb), dim3(256), 0, st, *sys, x, s_data, g_ori, d_part,
+                       drift_rows, y);
   GK_HIP(hipGetLastError());
   return GK_OK;
 }
@@ -1840,8 +1827,9 @@ int gk_hessian_system(gk_handle h, const gk_system* sys, const double* weights, 
   GK_REQUIRE(part_cap >= (size_t)std::max<int64_t>(n, 1) * 48, GK_ERR_ARG, "hessian: partial buffer too small");
   void* ws = nullptr;
   GK_TRY(gk_workspace(h, WS_EVAL_SRC, sources_bytes(sys), &ws));
-  const void *pts = nullptr, *ori = nullptr;
-  GK_TRY(prepare_sources(h, sys, weights, GK_F64, st, &pts, &ori, ws, true));
+  void *pts = nullptr, *ori = nullptr;
+  source_layout(sys, GK_F64, ws, &pts, &ori);
+  GK_TRY(prepare_sources(sys, weights, GK_F64, st, ws));
   HessArgs a{};
   a.pts = static_cast<const V4<double>*>(pts);
   a.n_pts = sys->n_rest + sys->n_surf;
