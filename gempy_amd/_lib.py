@@ -123,6 +123,8 @@ SIGNATURES = {
                                     P]),
     "gk_octree_points": (C.c_int, [P, C.POINTER(C.c_double), C.POINTER(C.c_int64), P, C.c_int64, C.c_int32,
                                    P, P]),
+    "gk_octree_probes": (C.c_int, [P, C.POINTER(C.c_double), C.POINTER(C.c_int64), P, C.c_int64, P, P,
+                                   C.POINTER(C.c_int64), P]),
     "gk_octree_refine": (C.c_int, [P, C.c_int32, P, C.c_int64, P, C.POINTER(C.c_int64), P, P,
                                    C.POINTER(C.c_int64), P]),
     "gk_test_trsv_set_error": (C.c_int, [P, C.c_int32, P]),

@@ -217,31 +217,45 @@ def compute_octree(m: _Model, levels: int) -> List[OctreeLevel]:
         n = int(vox.numel())
         cres = (C.c_int64 * 3)(*res)
         last = lvl == levels - 1
+        # where the active voxels fill a good part of the level (its corner
+        # lattice has at most 16 points a voxel) they share most corners: each
+        # is evaluated once; else probes with repeats, without a table per corner
+        corners = (res[0] + 1) * (res[1] + 1) * (res[2] + 1)
+        shared = not last and corners <= 16 * n and max(9 * n, corners) < 2 ** 31 - 1
         npts = n if last else 9 * n
         pts = torch.empty((max(npts, 1), 3), dtype=torch.float64, device="cuda")
-        _lib.check("gk_octree_points", lib.gk_octree_points(handle(0), ext, cres, _ptr(vox), n, int(last),
-                                                            _ptr(pts), _stream()))
+        if shared:
+            probe = torch.empty(9 * n, dtype=torch.int32, device="cuda")
+            count = C.c_int64(0)
+            _lib.check("gk_octree_probes", lib.gk_octree_probes(handle(0), ext, cres, _ptr(vox), n, _ptr(pts),
+                                                                _ptr(probe), C.byref(count), _stream()))
+            npts = count.value
+        else:
+            _lib.check("gk_octree_points", lib.gk_octree_points(handle(0), ext, cres, _ptr(vox), n, int(last),
+                                                                _ptr(pts), _stream()))
+        centre = slice(0, n) if last or shared else slice(0, None, 9)
         pts = pts[:npts]
         per: list = []
         lith, faults, scal = m.at_points(pts, keep_scalar=True, per_stack=per)
-        step = 1 if last else 9                 # voxel centres: every 9th probe point
         outs = [StackSolution(weights=sol.weights, scalar_field_at_surface_points=sol.scalar_field_at_surface_points,
-                              thresholds=sol.thresholds, scalar_field=S[0::step], ids_block=ids[0::step],
+                              thresholds=sol.thresholds, scalar_field=S[centre], ids_block=ids[centre],
                               solver_info=sol.solver_info, sigmoid_slope=sol.sigmoid_slope,
-                              mask=None if msk is None else msk[0::step])
+                              mask=None if msk is None else msk[centre])
                 for sol, (S, ids, msk) in zip(m.sols, per)]
         if last:
             out.append(OctreeLevel(tuple(res), vox, lith, scal[-1] if scal else None, None, outs))
             break
         fields = torch.stack([lith] + faults).contiguous() if lith is not None else torch.stack(faults)
+        if shared:
+            fields = fields.index_select(1, probe)
         refine = torch.empty(max(n, 1), dtype=torch.uint8, device="cuda")
         children = torch.empty(max(8 * n, 1), dtype=torch.int64, device="cuda")
         nch = C.c_int64(0)
         _lib.check("gk_octree_refine", lib.gk_octree_refine(handle(0), fields.shape[0], _ptr(fields), n, _ptr(vox),
                                                             cres, _ptr(refine), _ptr(children), C.byref(nch),
                                                             _stream()))
-        centre_scalar = scal[-1][0::9] if scal else None
-        out.append(OctreeLevel(tuple(res), vox, lith[0::9] if lith is not None else None, centre_scalar,
+        centre_scalar = scal[-1][centre] if scal else None
+        out.append(OctreeLevel(tuple(res), vox, lith[centre] if lith is not None else None, centre_scalar,
                                refine[:n].bool(), outs))
         vox = children[:nch.value].clone()
         res = [2 * r for r in res]

@@ -50,6 +50,7 @@ enum gk_ws_slot {
   WS_MESH,           // case tables, edge flags and scans of the isosurface extraction
   WS_LANCZOS,        // Lanczos basis of the condition-number estimate
   WS_KNN,            // cells and sorted points of the grid neighbour search
+  WS_OCTREE,         // corner flags and ranks of an octree level's probes
   WS_COUNT
 };
 // Independent sets of tables, flags and buffers of the sync-free triangular
