@@ -17,7 +17,7 @@
 //
 // The field is read once: a first pass packs every z row into words of 64
 // points (above the level, NaN, masked), and everything that follows works on
-// those words - 3/64 of a byte per point and flag - until the crossed edges
+// those words - an eighth of a byte per point and flag - until the crossed edges
 // and the cubes with triangles, few and known, are written.  What it is bound
 // by is that one read (8 bytes a point, 9 with a mask).  Per-point flags, edge
 // ids and cube cases in memory with scans over them moved about 500 bytes a
