@@ -62,6 +62,11 @@ struct EvalArgs {
   // carries the same work.
   int32_t nsplit;
   int64_t cost_chunk;
+  // explicit points, mask asked for: 1 for each of n_out groups of sources
+  // with one outside the sphere of half the range around the centre (null:
+  // not known)
+  const int32_t* src_out;
+  int32_t n_out;
   double* part_s;
   double* part_g;
 };
@@ -250,6 +255,74 @@ __device__ __forceinline__ void lattice_ori_tile(const V8<T>* s8, int nk, T x0, 
   }
 }
 
+// Sums of one LDS tile's sources at PPT explicit points: no clamp per pair,
+// Newton step folded as on the lattice.  kc: the halved constants of C (3/4,
+// -7/2, 35/4) and C'/r (21/4, -35/2, 105/4), held in registers.
+template <typename T, bool GRAD, bool MASKED, int PPT, bool SCALAR>
+__device__ __forceinline__ void points_pts_tile(const V4<T>* s4, int nk, const T (&kc)[6], const T (&px)[PPT],
+                                                const T (&py)[PPT], const T (&pz)[PPT], T (&part)[PPT],
+                                                T (&gpart)[PPT][3]) {
+#pragma unroll 2
+  for (int k = 0; k < nk; ++k) {
+    const V4<T> s = s4[k];
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+      const T dx = px[q] - s.x, dy = py[q] - s.y, dz = pz[q] - s.z;
+      const T t = fma(dz, dz, fma(dy, dy, fma(dx, dx, Tiny<T>::v)));
+      const T y = gk_rsq_raw(t);
+      const T r = t * y;
+      const T h3 = fma(-r, y, T(3));
+      T c = fma(fma(r * fma(fma(kc[0], t, kc[1]), t, kc[2]), h3, T(-7)), t, T(1));
+      if (MASKED) c = t < T(1) ? c : T(0);
+      if (SCALAR) part[q] = fma(s.w, c, part[q]);
+      if (GRAD) {
+        T dp = fma(r * fma(fma(kc[3], t, kc[4]), t, kc[5]), h3, T(-14));
+        if (MASKED) dp = t < T(1) ? dp : T(0);
+        const T wd = s.w * dp;
+        gpart[q][0] = fma(wd, dx, gpart[q][0]);
+        gpart[q][1] = fma(wd, dy, gpart[q][1]);
+        gpart[q][2] = fma(wd, dz, gpart[q][2]);
+      }
+    }
+  }
+}
+
+template <typename T, bool GRAD, bool MASKED, int PPT, bool SCALAR>
+__device__ __forceinline__ void points_ori_tile(const V8<T>* s8, int nk, const T (&kc)[6], const T (&px)[PPT],
+                                                const T (&py)[PPT], const T (&pz)[PPT], T (&part)[PPT],
+                                                T (&gpart)[PPT][3]) {
+#pragma unroll 2
+  for (int k = 0; k < nk; ++k) {
+    const V8<T> s = s8[k];
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+      const T dx = s.x - px[q], dy = s.y - py[q], dz = s.z - pz[q];   // q - x
+      const T t = fma(dz, dz, fma(dy, dy, fma(dx, dx, Tiny<T>::v)));
+      const T y = gk_rsq_raw(t);
+      const T r = t * y;
+      const T h3 = fma(-r, y, T(3));
+      T p = fma(r * fma(fma(kc[3], t, kc[4]), t, kc[5]), h3, T(-14));
+      if (MASKED) p = t < T(1) ? p : T(0);
+      const T dot = fma(s.wz, dz, fma(s.wy, dy, s.wx * dx));
+      if (SCALAR) part[q] = fma(dot, p, part[q]);
+      if (GRAD) {
+        const T om = T(1) - t;
+        T dd = T(13.125) * om * om * (y * h3);     // 26.25 (1-t)^2 / rho, 1/rho = y (3 - r y) / 2
+        if (MASKED) dd = t < T(1) ? dd : T(0);
+        const T hw = dot * dd;
+        gpart[q][0] -= fma(s.wx, p, hw * dx);
+        gpart[q][1] -= fma(s.wy, p, hw * dy);
+        gpart[q][2] -= fma(s.wz, p, hw * dz);
+      }
+    }
+  }
+}
+
+// Square of half the range (range units) less the rounding of both ends of a pair.
+template <typename T> __host__ __device__ constexpr double half_range2() {
+  return 0.25 * (1.0 - (sizeof(T) == 4 ? 1e-5 : 1e-9));
+}
+
 // SCALAR false (explicit points with gradient): the gradient only; the
 // scalar output then holds the drift terms alone.
 template <typename T, bool LATTICE, bool GRAD, bool MASKED, int PPT, bool SCALAR = true>
@@ -305,8 +378,22 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
     gpart[q][0] = gpart[q][1] = gpart[q][2] = T(0);
   }
 
-  // halved polynomial constants for the explicit-point loops, held in
-  // registers: C: 3/4, -7/2, 35/4; C'/r: 21/4, -35/2, 105/4 (all halved)
+  // Explicit points come without a box.  Where every source and every point
+  // of the wave lies within half the range of the centre no pair is beyond it,
+  // and the same sums go without the mask: the preparing launch leaves a flag
+  // per group of sources, the wave looks at its own points.  Scalar at 20,000
+  // points of 25,000 sources 370 us with the mask, 310 without; a product of
+  // 25,000 data 431 and 391, 100,000 points of 6,000 sources 390 and 351.
+  bool inside = false;
+  if constexpr (!LATTICE && MASKED) {
+    bool out = a.src_out == nullptr;
+    for (int i = tid & 63; !out && i < a.n_out; i += 64) out = a.src_out[i] != 0;
+#pragma unroll
+    for (int q = 0; q < PPT; ++q)
+      out = out || !((double)fma(pz[q], pz[q], fma(py[q], py[q], px[q] * px[q])) <= half_range2<T>());
+    inside = !__any(out);
+  }
+
   T kc[6] = {T(0.375), T(-1.75), T(4.375), T(2.625), T(-8.75), T(13.125)};
   if constexpr (!LATTICE) asm volatile("" : "+v"(kc[0]), "+v"(kc[1]), "+v"(kc[2]), "+v"(kc[3]), "+v"(kc[4]), "+v"(kc[5]));
 
@@ -338,30 +425,10 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
     __syncthreads();
     if constexpr (LATTICE) {
       lattice_pts_tile<T, GRAD, MASKED, PPT>(s4, nk, x0, y0, SpacedRun<T>{z0, hz}, part, gpart);
-    } else {             // explicit points: no clamp per pair, Newton step folded as on the lattice
-#pragma unroll 2
-      for (int k = 0; k < nk; ++k) {
-        const V4<T> s = s4[k];
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-          const T dx = px[q] - s.x, dy = py[q] - s.y, dz = pz[q] - s.z;
-          const T t = fma(dz, dz, fma(dy, dy, fma(dx, dx, Tiny<T>::v)));
-          const T y = gk_rsq_raw(t);
-          const T r = t * y;
-          const T h3 = fma(-r, y, T(3));
-          T c = fma(fma(r * fma(fma(kc[0], t, kc[1]), t, kc[2]), h3, T(-7)), t, T(1));
-          if (MASKED) c = t < T(1) ? c : T(0);
-          if (SCALAR) part[q] = fma(s.w, c, part[q]);
-          if (GRAD) {
-            T dp = fma(r * fma(fma(kc[3], t, kc[4]), t, kc[5]), h3, T(-14));
-            if (MASKED) dp = t < T(1) ? dp : T(0);
-            const T wd = s.w * dp;
-            gpart[q][0] = fma(wd, dx, gpart[q][0]);
-            gpart[q][1] = fma(wd, dy, gpart[q][1]);
-            gpart[q][2] = fma(wd, dz, gpart[q][2]);
-          }
-        }
-      }
+    } else if (MASKED && !inside) {
+      points_pts_tile<T, GRAD, true, PPT, SCALAR>(s4, nk, kc, px, py, pz, part, gpart);
+    } else {
+      points_pts_tile<T, GRAD, false, PPT, SCALAR>(s4, nk, kc, px, py, pz, part, gpart);
     }
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
@@ -388,32 +455,10 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
     __syncthreads();
     if constexpr (LATTICE) {
       lattice_ori_tile<T, GRAD, MASKED, PPT>(s_src, nk, x0, y0, SpacedRun<T>{z0, hz}, part, gpart);
-    } else {             // explicit points (see the interface-source loop)
-#pragma unroll 2
-      for (int k = 0; k < nk; ++k) {
-        const V8<T> s = s_src[k];
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-          const T dx = s.x - px[q], dy = s.y - py[q], dz = s.z - pz[q];   // q - x
-          const T t = fma(dz, dz, fma(dy, dy, fma(dx, dx, Tiny<T>::v)));
-          const T y = gk_rsq_raw(t);
-          const T r = t * y;
-          const T h3 = fma(-r, y, T(3));
-          T p = fma(r * fma(fma(kc[3], t, kc[4]), t, kc[5]), h3, T(-14));
-          if (MASKED) p = t < T(1) ? p : T(0);
-          const T dot = fma(s.wz, dz, fma(s.wy, dy, s.wx * dx));
-          if (SCALAR) part[q] = fma(dot, p, part[q]);
-          if (GRAD) {
-            const T om = T(1) - t;
-            T dd = T(13.125) * om * om * (y * h3);     // 26.25 (1-t)^2 / rho, 1/rho = y (3 - r y) / 2
-            if (MASKED) dd = t < T(1) ? dd : T(0);
-            const T hw = dot * dd;
-            gpart[q][0] -= fma(s.wx, p, hw * dx);
-            gpart[q][1] -= fma(s.wy, p, hw * dy);
-            gpart[q][2] -= fma(s.wz, p, hw * dz);
-          }
-        }
-      }
+    } else if (MASKED && !inside) {
+      points_ori_tile<T, GRAD, true, PPT, SCALAR>(s_src, nk, kc, px, py, pz, part, gpart);
+    } else {
+      points_ori_tile<T, GRAD, false, PPT, SCALAR>(s_src, nk, kc, px, py, pz, part, gpart);
     }
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
@@ -971,12 +1016,15 @@ __device__ __forceinline__ double drift_row_chunk(const gk_system& sys, const do
 }
 
 // xyz, drift (nullable): the operator product's.  drift_rows of them.
+// out (nullable): per workgroup of sources, whether one of them lies outside
+// the sphere of half the range around the centre (or is no number).
 template <typename T>
 __global__ __launch_bounds__(PREP) void prep_kernel(gk_system sys, const double* w, V4<T>* pts, V8<T>* ori, double* xyz,
-                                                    double* drift, int drift_rows) {
+                                                    double* drift, int drift_rows, int32_t* out) {
   __shared__ double red[PREP / 64];
   const int64_t R = sys.n_rest, S = sys.n_surf, no = sys.n_ori;
   const double inv_a = 1.0 / sys.range;
+  bool beyond = false;
   auto put = [&](int64_t i, const double* p, double wt) {
     V4<T> v;
     v.x = (T)((p[0] - sys.center[0]) * inv_a);
@@ -984,6 +1032,7 @@ __global__ __launch_bounds__(PREP) void prep_kernel(gk_system sys, const double*
     v.z = (T)((p[2] - sys.center[2]) * inv_a);
     v.w = (T)wt;
     pts[i] = v;
+    beyond = !((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z <= half_range2<T>());
     if (xyz) { xyz[3 * i] = p[0]; xyz[3 * i + 1] = p[1]; xyz[3 * i + 2] = p[2]; }
   };
   int64_t b = blockIdx.x;
@@ -995,7 +1044,10 @@ __global__ __launch_bounds__(PREP) void prep_kernel(gk_system sys, const double*
       acc += sys.rest_surf[i] == b ? wi : 0.0;
     }
     const double W = block_sum(acc, red);
-    if (threadIdx.x == 0) put(R + b, sys.ref_xyz + 3 * b, -sys.i_res * sys.c_o * W);
+    if (threadIdx.x == 0) {
+      put(R + b, sys.ref_xyz + 3 * b, -sys.i_res * sys.c_o * W);
+      if (out) out[blockIdx.x] = beyond;
+    }
     return;
   }
   b -= S;
@@ -1003,24 +1055,30 @@ __global__ __launch_bounds__(PREP) void prep_kernel(gk_system sys, const double*
   if (b < nr) {
     const int64_t i = b * PREP + threadIdx.x;
     if (i < R) put(i, sys.rest_xyz + 3 * i, sys.i_res * sys.c_o * w[3 * no + i]);
+    const bool any = __syncthreads_or(beyond);
+    if (out && threadIdx.x == 0) out[blockIdx.x] = any;
     return;
   }
   b -= nr;
   if (b < nq) {
     const int64_t g = b * PREP + threadIdx.x;
-    if (g >= no) return;
-    const double f = sys.gi_res * sys.c_o * inv_a;
-    const double* q = sys.ori_xyz + 3 * g;
-    V8<T> v;
-    v.x = (T)((q[0] - sys.center[0]) * inv_a);
-    v.y = (T)((q[1] - sys.center[1]) * inv_a);
-    v.z = (T)((q[2] - sys.center[2]) * inv_a);
-    v.pad0 = T(0);
-    v.wx = (T)(f * w[g]);
-    v.wy = (T)(f * w[no + g]);
-    v.wz = (T)(f * w[2 * no + g]);
-    v.pad1 = T(0);
-    ori[g] = v;
+    if (g < no) {
+      const double f = sys.gi_res * sys.c_o * inv_a;
+      const double* q = sys.ori_xyz + 3 * g;
+      V8<T> v;
+      v.x = (T)((q[0] - sys.center[0]) * inv_a);
+      v.y = (T)((q[1] - sys.center[1]) * inv_a);
+      v.z = (T)((q[2] - sys.center[2]) * inv_a);
+      v.pad0 = T(0);
+      v.wx = (T)(f * w[g]);
+      v.wy = (T)(f * w[no + g]);
+      v.wz = (T)(f * w[2 * no + g]);
+      v.pad1 = T(0);
+      ori[g] = v;
+      beyond = !((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z <= half_range2<T>());
+    }
+    const bool any = __syncthreads_or(beyond);
+    if (out && threadIdx.x == 0) out[blockIdx.x] = any;
     return;
   }
   b -= nq;
@@ -1074,6 +1132,24 @@ void dispatch_eval(const EvalArgs& a, bool lattice, bool grad, bool masked, hipS
 
 }  // namespace
 
+// Workgroups of prep_kernel that hold sources.
+static int64_t source_groups(const gk_system* sys) {
+  return sys->n_surf + gk_ceil_div(sys->n_rest, PREP) + gk_ceil_div(sys->n_ori, PREP);
+}
+
+static size_t sources_bytes(const gk_system* sys) {
+  const int64_t R = sys->n_rest, S = sys->n_surf, no = sys->n_ori;
+  return gk_round_up(S * 8, 256) + gk_round_up((R + S) * 32, 256) + gk_round_up(no * 64, 256) + 256;
+}
+
+// The handle's workspace of packed sources, with the groups' flags behind them.
+static int source_workspace(gk_handle h, const gk_system* sys, void** ws, int32_t** out) {
+  const size_t at = gk_round_up(sources_bytes(sys), 256);
+  GK_TRY(gk_workspace(h, WS_EVAL_SRC, at + source_groups(sys) * sizeof(int32_t) + 256, ws));
+  *out = reinterpret_cast<int32_t*>(static_cast<char*>(*ws) + at);
+  return GK_OK;
+}
+
 // Where the packed sources lie in a workspace: [pts V4<T> (R+S) | ori V8<T> (n_ori)].
 static void source_layout(const gk_system* sys, int precision, void* ws, void** pts, void** ori) {
   const size_t tsz = precision == GK_F64 ? 8 : 4;
@@ -1084,25 +1160,19 @@ static void source_layout(const gk_system* sys, int precision, void* ws, void** 
 // Prepare the packed sources for `weights` in the workspace ws; xyz, drift,
 // drift_rows: see prep_kernel.
 static int prepare_sources(const gk_system* sys, const double* weights, int precision, hipStream_t st, void* ws,
-                           double* xyz = nullptr, double* drift = nullptr, int drift_rows = 0) {
-  const int64_t nb = sys->n_surf + gk_ceil_div(sys->n_rest, PREP) + gk_ceil_div(sys->n_ori, PREP) +
-                     (int64_t)drift_rows * DRIFT_CHUNKS;
+                           int32_t* out, double* xyz = nullptr, double* drift = nullptr, int drift_rows = 0) {
+  const int64_t nb = source_groups(sys) + (int64_t)drift_rows * DRIFT_CHUNKS;
   void *p4, *p8;
   source_layout(sys, precision, ws, &p4, &p8);
   if (nb == 0) return GK_OK;
   if (precision == GK_F64)
     hipLaunchKernelGGL(prep_kernel<double>, dim3((unsigned)nb), dim3(PREP), 0, st, *sys, weights,
-                       static_cast<V4<double>*>(p4), static_cast<V8<double>*>(p8), xyz, drift, drift_rows);
+                       static_cast<V4<double>*>(p4), static_cast<V8<double>*>(p8), xyz, drift, drift_rows, out);
   else
     hipLaunchKernelGGL(prep_kernel<float>, dim3((unsigned)nb), dim3(PREP), 0, st, *sys, weights,
-                       static_cast<V4<float>*>(p4), static_cast<V8<float>*>(p8), xyz, drift, drift_rows);
+                       static_cast<V4<float>*>(p4), static_cast<V8<float>*>(p8), xyz, drift, drift_rows, out);
   GK_HIP(hipGetLastError());
   return GK_OK;
-}
-
-static size_t sources_bytes(const gk_system* sys) {
-  const int64_t R = sys->n_rest, S = sys->n_surf, no = sys->n_ori;
-  return gk_round_up(S * 8, 256) + gk_round_up((R + S) * 32, 256) + gk_round_up(no * 64, 256) + 256;
 }
 
 static int check_system(const gk_system* sys) {
@@ -1379,6 +1449,7 @@ static int eval_impl(gk_handle h, const gk_system* sys, const double* weights, g
   for (int k = 0; k < d->n_thresholds; ++k) a.thr[k] = d->thresholds[k];
 
   void* ws = nullptr;
+  int32_t* out = nullptr;
   char* part = nullptr;
   size_t part_bytes = 0;
   if (ext) {
@@ -1390,13 +1461,15 @@ static int eval_impl(gk_handle h, const gk_system* sys, const double* weights, g
     part = ext + need;
     part_bytes = ext_bytes - need;
   } else {
-    GK_TRY(gk_workspace(h, WS_EVAL_SRC, sources_bytes(sys), &ws));
+    GK_TRY(source_workspace(h, sys, &ws, &out));
   }
+  a.src_out = out;
+  a.n_out = (int32_t)source_groups(sys);
   void *pts = nullptr, *ori = nullptr;
   source_layout(sys, d->precision, ws, &pts, &ori);
   a.pts = pts;
   a.ori = ori;
-  if (!reuse_sources) GK_TRY(prepare_sources(sys, weights, d->precision, st, ws));
+  if (!reuse_sources) GK_TRY(prepare_sources(sys, weights, d->precision, st, ws, out));
   bool masked = true;
   if (!force_mask && src_box) {
     // explicit points: only callers whose points lie inside the source box
@@ -1470,8 +1543,9 @@ extern "C" int gk_matvec_impl(gk_handle h, const gk_system* sys, int32_t precisi
   GK_TRY(check_system(sys));
   const int drift_rows = n_drift_of(sys->uni_degree) + sys->n_fault;
   void* ws = nullptr;
-  GK_TRY(gk_workspace(h, WS_EVAL_SRC, sources_bytes(sys), &ws));
-  GK_TRY(prepare_sources(sys, x, precision, st, ws, pts, d_part, drift_rows));
+  int32_t* out = nullptr;
+  GK_TRY(source_workspace(h, sys, &ws, &out));
+  GK_TRY(prepare_sources(sys, x, precision, st, ws, out, pts, d_part, drift_rows));
   gk_system nofault = *sys;
   nofault.n_fault = 0;  // fault drift enters the interface rows separately
   if (R + S > 0) {
@@ -1829,7 +1903,7 @@ int gk_hessian_system(gk_handle h, const gk_system* sys, const double* weights, 
   GK_TRY(gk_workspace(h, WS_EVAL_SRC, sources_bytes(sys), &ws));
   void *pts = nullptr, *ori = nullptr;
   source_layout(sys, GK_F64, ws, &pts, &ori);
-  GK_TRY(prepare_sources(sys, weights, GK_F64, st, ws));
+  GK_TRY(prepare_sources(sys, weights, GK_F64, st, ws, nullptr));
   HessArgs a{};
   a.pts = static_cast<const V4<double>*>(pts);
   a.n_pts = sys->n_rest + sys->n_surf;
