@@ -382,7 +382,7 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
   // of the wave lies within half the range of the centre no pair is beyond it,
   // and the same sums go without the mask: the preparing launch leaves a flag
   // per group of sources, the wave looks at its own points.  Scalar at 20,000
-  // points of 25,000 sources 370 us with the mask, 297 without; a product of
+  // points of 25,000 sources 370 us with the mask, 339 without; a product of
   // 25,000 data 431 and 391, 100,000 points of 6,000 sources 390 and 351.
   bool inside = false;
   if constexpr (!LATTICE && MASKED) {
