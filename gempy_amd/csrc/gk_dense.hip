@@ -843,8 +843,11 @@ __global__ __launch_bounds__(1024) void getrf128_kernel(double* A, int64_t lda, 
 // panel buffers P[b] hold the 16 columns of panels s - 1, s and s + 1
 // column-major (P[b][t][i] = L[i][jb + t], columns 144 apart for the banks):
 // panel rows are loaded without per-row branches and the tiles read the panel
-// with consecutive addresses.  FP32 61 KB, FP64 122 KB (two triangles and two
-// panels would need 161 KB in FP64, more than a CU has).  Measured cycle by
+// with consecutive addresses.  The factored diagonal tile of panel s goes to a
+// buffer of its own, D(s, t, i) = L[jb + i][jb + t]: the three waves of the
+// next panel all read the tile not yet factored from P, at any time of phase
+// B, so wave 0 must not store there.  FP32 63 KB, FP64 126 KB (two triangles
+// and two panels would need 161 KB in FP64, more than a CU has).  Measured cycle by
 // cycle (FP64): with branches per element a tile took 2,100 cycles, the block
 // load 19,000 and the whole 73 us; with masked accesses, the pivot chain beside
 // the column updates and the tiles beside the next panel 48 us (FP32 42 -> 34).
@@ -854,12 +857,14 @@ struct BlkStore {
   static constexpr int PB = GK_POTRF_PB;
   T* S;
   static constexpr int PS = DB + 16;          // column stride of the panel buffers
-  static constexpr int TRI = DB * (DB + 1) / 2, IPV = TRI + 3 * PB * PS, SPARE = IPV + 2 * PB;
+  static constexpr int TRI = DB * (DB + 1) / 2, DIAG = TRI + 3 * PB * PS, IPV = DIAG + 2 * PB * PB,
+                       SPARE = IPV + 2 * PB;
   static constexpr int SIZE = SPARE + 64 + 2;
   __device__ static int pl(int i, int c) { return (int)__umul24(i, i + 1) / 2 + c; }
   __device__ static int po(int b, int t, int i) { return TRI + (b * PB + t) * PS + i; }
   __device__ T& V(int i, int c) { return S[pl(i, c)]; }
   __device__ T& P(int b, int t, int i) { return S[po(b, t, i)]; }
+  __device__ T& D(int s, int t, int i) { return S[DIAG + ((s & 1) * PB + t) * PB + i]; }
   __device__ T& ipv(int s, int j) { return S[IPV + (s & 1) * PB + j]; }     // 1 / pivot j of panel s
   __device__ int spare() const { return SPARE + (threadIdx.x & 63); }       // where masked stores go
   __device__ int* next() { return reinterpret_cast<int*>(&S[SPARE + 64]); }  // next tile of phase B
@@ -1000,7 +1005,12 @@ __device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ld
       }
       a[j] = lane == j ? piv : (lane > j ? aj : a[j]);
     }
-    if (r < DB && (lane >= PB || w == 0)) {
+    if (lane < PB) {
+      if (w == 0) {
+#pragma unroll
+        for (int c = 0; c < PB; ++c) B.D(s, c, lane) = a[c];
+      }
+    } else if (r < DB) {
 #pragma unroll
       for (int c = 0; c < PB; ++c) B.P(pb, c, r) = a[c];
     }
@@ -1013,7 +1023,7 @@ __device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ld
   // same order as a row-by-row substitution; the dependent chain is 16 steps,
   // not 120).
   auto x_rows = [&](int s, int coff) {
-    const int jb = s * PB, pb = s % 3, c = lane + coff;
+    const int jb = s * PB, c = lane + coff;
     T x[PB], ipv[PB];
     vt col[2][PB / VL];
 #pragma unroll
@@ -1026,14 +1036,14 @@ __device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ld
       const vt v = *reinterpret_cast<const vt*>(&B.ipv(s, r));
 #pragma unroll
       for (int u = 0; u < VL; ++u) ipv[r + u] = v[u];
-      col[0][r / VL] = *reinterpret_cast<const vt*>(&B.P(pb, 0, jb + r));
+      col[0][r / VL] = *reinterpret_cast<const vt*>(&B.D(s, 0, r));
     }
 #pragma unroll
     for (int k = 0; k < PB; ++k) {            // the next column is read beside step k
       if (k + 1 < PB) {
 #pragma unroll
         for (int r = (k + 2) / VL * VL; r < PB; r += VL)
-          col[(k + 1) & 1][r / VL] = *reinterpret_cast<const vt*>(&B.P(pb, k + 1, jb + r));
+          col[(k + 1) & 1][r / VL] = *reinterpret_cast<const vt*>(&B.D(s, k + 1, r));
       }
       x[k] *= ipv[k];
 #pragma unroll
@@ -1049,7 +1059,7 @@ __device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ld
     const int jb = s * PB, pb = s % 3;
     for (int e = t; e < PB * PB; e += nt) {
       const int r = e / PB, c = e % PB;
-      if (c <= r) A[(jb + r) * lda + jb + c] = B.P(pb, c, jb + r);
+      if (c <= r) A[(jb + r) * lda + jb + c] = B.D(s, c, r);
     }
     for (int e = t; e < (nlive - jb - PB) * (PB / VL); e += nt) {
       const int i = jb + PB + e / (PB / VL), c = e % (PB / VL) * VL;
@@ -1152,7 +1162,7 @@ __device__ void potrf_blocked(BlkStore<T> B, T* A, int64_t lda, T* X, int64_t ld
   }
 }
 
-// FP32: 61 KB of LDS, so the kernel fits on a CU beside a workgroup of the
+// FP32: 63 KB of LDS, so the kernel fits on a CU beside a workgroup of the
 // concurrent trailing update (the look-ahead factorization runs it on a
 // second stream).
 __global__ __launch_bounds__(GK_POTRF_NT) void potrf128b_f32_kernel(float* A, int64_t lda, float* X, int64_t ldx,
