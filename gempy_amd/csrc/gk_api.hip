@@ -69,6 +69,7 @@ extern "C" void gk_destroy(gk_handle h) {
   for (hipEvent_t& e : h->aux_ev)
     if (e) (void)hipEventDestroy(e);
   if (h->aux) (void)hipStreamDestroy(h->aux);
+  if (h->mesh_tables) (void)hipFree(h->mesh_tables);
   if (h->mesh_counts) (void)hipHostFree(h->mesh_counts);
   delete h;
 }

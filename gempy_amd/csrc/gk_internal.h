@@ -47,7 +47,7 @@ enum gk_ws_slot {
   WS_SMALL,          // small scratch (bounding boxes, counts)
   WS_TRSV,           // work tables, readiness flags and partial sums of the triangular solves
   WS_ASSEMBLE,       // reference-point tables of the assembly
-  WS_MESH,           // case tables, edge flags and scans of the isosurface extraction
+  WS_MESH,           // bit words and counts of the isosurface extraction
   WS_LANCZOS,        // Lanczos basis of the condition-number estimate
   WS_KNN,            // cells and sorted points of the grid neighbour search
   WS_OCTREE,         // corner flags and ranks of an octree level's probes
@@ -76,7 +76,7 @@ struct gk_context {
   hipEvent_t aux_ev[2] = {};
   // device address of gk_eval_noalloc's file-scope scratch array (this device's copy)
   char* eval_scratch = nullptr;
-  // where the marching-cubes case tables were last uploaded (inside WS_MESH)
+  // case tables of the isosurface extraction, uploaded by its first call
   void* mesh_tables = nullptr;
   // pinned pair of counts that the isosurface extraction's kernels write
   uint32_t* mesh_counts = nullptr;

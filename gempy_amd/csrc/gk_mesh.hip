@@ -435,27 +435,35 @@ extern "C" int gk_marching_cubes(gk_handle h, const double* field, const int64_t
   if (nx < 2 || ny < 2 || nz < 2) return GK_OK;
   hipStream_t st = (hipStream_t)stream;
   const int64_t W = gk_ceil_div(nz, 64), words = nx * ny * W, nb = gk_ceil_div(words, MC_WORDS);
-  // workspace: tables | totals | 7 word arrays | 2 counts per word | 2 sums per block
+  // workspace: totals | 7 word arrays | 2 counts per word | 2 sums per block
   size_t need = 0;
   auto take = [&](size_t bytes) { size_t o = need; need += gk_round_up(bytes, 256); return o; };
-  const size_t o_T = take(sizeof(McTables)), o_tot = take(16);
+  const size_t o_tot = take(16);
   size_t o_w[7], o_n[4];
   for (size_t& o : o_w) o = take(words * 8);
   for (int k = 0; k < 4; ++k) o_n[k] = take((k < 2 ? words : nb) * 4);
   void* p = nullptr;
   GK_TRY(gk_workspace(h, WS_MESH, need, &p));
   char* b = static_cast<char*>(p);
-  if (h->mesh_tables != b + o_T) {        // tables uploaded once per workspace
+  // The tables, once per handle, in memory of their own: a workspace that
+  // grows may come back at the same address without its contents.
+  if (!h->mesh_tables) {
     static const McTables host = build_tables();
-    GK_HIP(hipMemcpyAsync(b + o_T, &host, sizeof(McTables), hipMemcpyHostToDevice, st));
-    h->mesh_tables = b + o_T;
+    void* t = nullptr;
+    GK_HIP(hipMalloc(&t, sizeof(McTables)));
+    if (hipMemcpyAsync(t, &host, sizeof(McTables), hipMemcpyHostToDevice, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess) {
+      (void)hipFree(t);
+      GK_REQUIRE(false, GK_ERR_HIP, "gk_marching_cubes: the case tables could not be copied to the device");
+    }
+    h->mesh_tables = t;
   }
   if (!h->mesh_counts) GK_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->mesh_counts), 64, hipHostMallocDefault));
   McArgs a{};
   a.f = field; a.mask = mask;
   a.nx = nx; a.ny = ny; a.nz = nz; a.W = W; a.words = words;
   a.level = level;
-  a.T = reinterpret_cast<const McTables*>(b + o_T);
+  a.T = static_cast<const McTables*>(h->mesh_tables);
   uint64_t** wp[7] = {&a.above, &a.nan, &a.msk, &a.valid, &a.edge[0], &a.edge[1], &a.edge[2]};
   for (int k = 0; k < 7; ++k) *wp[k] = reinterpret_cast<uint64_t*>(b + o_w[k]);
   uint32_t** np[4] = {&a.vpre, &a.tpre, &a.vsum, &a.tsum};
