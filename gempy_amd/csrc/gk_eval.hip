@@ -685,6 +685,8 @@ __device__ __forceinline__ void add_exact(double& acc, double& err, double v) {
   err += (acc - (s - b)) + (v - b);
   acc = s;
 }
+// The sum; its error term is no number where the sum is infinite.
+__device__ __forceinline__ double exact_sum(double acc, double err) { return err == err ? acc + err : acc; }
 
 // Far sources of a block at its nodes: one wave per 64 runs of 8 nodes and per
 // part of the sources, so that a few hundred blocks still fill the chip.
@@ -740,7 +742,7 @@ __global__ __launch_bounds__(FAR_TS) void far_nodes_kernel(FarArgs f) {
   }
   double* o = f.nodes + ((int64_t)split * nb + b) * (N * N * N) + ((int64_t)ix * N + iy) * N + iz;
 #pragma unroll
-  for (int q = 0; q < FAR_RUN; ++q) o[q] = acc[q] + err[q];
+  for (int q = 0; q < FAR_RUN; ++q) o[q] = exact_sum(acc[q], err[q]);
 }
 
 // Node sums to the points, one axis after the other: a workgroup takes up to
@@ -874,7 +876,7 @@ __global__ __launch_bounds__(64 * NEAR_WAVES) void near_kernel(FarArgs f) {
     flush();
   }
 #pragma unroll
-  for (int q = 0; q < PPT; ++q) acc[q] += err[q];
+  for (int q = 0; q < PPT; ++q) acc[q] = exact_sum(acc[q], err[q]);
   __syncthreads();                     // the tiles give way to the sums
   double* sums = reinterpret_cast<double*>(lds);
   if (wave > 0) {
