@@ -554,15 +554,18 @@ enum { FAR_BEYOND = 0, FAR_NEAR = 1, FAR_FAR = 2 };
 
 // Group of a source at distance d (per axis, from the block's centre) of a
 // block with half widths h, in units of the range.  The margins of the range
-// tests cover FP32: the near sums test each pair themselves.
-__host__ __device__ inline int far_group(const float d[3], const float h[3], bool masked, bool nodes, float amin) {
+// tests cover FP32: the near sums test each pair themselves.  slack: what the
+// rounding of d, h and FP32 positions may add to the squared distance (it
+// counts where the block is many ranges wide or away from the centre).
+__host__ __device__ inline int far_group(const float d[3], const float h[3], bool masked, bool nodes, float amin,
+                                         float slack = 0.0f) {
   float g[3], dmin = 0.0f, dmax = 0.0f;
   for (int k = 0; k < 3; ++k) {
     g[k] = d[k] > h[k] ? d[k] - h[k] : 0.0f;
     dmin += g[k] * g[k];
     dmax += (d[k] + h[k]) * (d[k] + h[k]);
   }
-  if (masked && dmin >= 1.0001f) return FAR_BEYOND;
+  if (masked && dmin >= 1.0001f + slack) return FAR_BEYOND;
   if (!nodes || (masked && !(dmax < 0.9999f))) return FAR_NEAR;
   for (int k = 0; k < 3; ++k) {
     const float s2 = dmin - g[k] * g[k], u = d[k] + h[k], v = d[k] - h[k];
@@ -602,13 +605,16 @@ __device__ void far_sort(const FarArgs& f, const V* src, int64_t n, const double
   const int t = threadIdx.x, wave = t >> 6;
   const uint64_t below = (1ull << (t & 63)) - 1;
   int32_t nnear = 0, nfar = 0;
+  // 2^-24 each of d, of h (d < h + 2 where it matters) and, in FP32, of both
+  // positions, on every axis, twice for the square
+  const float slack = 1e-6f * (float)(fabs(c[0]) + fabs(c[1]) + fabs(c[2]) + h[0] + h[1] + h[2]);
   for (int64_t base = 0; base < n; base += 1024) {
     int g = FAR_BEYOND;
     if (base + t < n) {
       const V v = src[base + t];
       const float d[3] = {(float)fabs((double)v.x - c[0]), (float)fabs((double)v.y - c[1]),
                           (float)fabs((double)v.z - c[2])};
-      g = finite4(v) ? far_group(d, h, f.masked != 0, f.n > 0, f.amin) : FAR_NEAR;
+      g = finite4(v) ? far_group(d, h, f.masked != 0, f.n > 0, f.amin, slack) : FAR_NEAR;
     }
     const uint64_t mn = __ballot(g == FAR_NEAR), mf = __ballot(g == FAR_FAR);
     if ((t & 63) == 0) { w_near[wave] = __popcll(mn); w_far[wave] = __popcll(mf); }

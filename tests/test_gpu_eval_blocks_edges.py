@@ -34,3 +34,56 @@ def test_infinite_orientation_weight(gpu, weight, prec):
     S2, _, _ = ds.evaluate_points(torch.tensor(g.values(), device="cuda"), w, p)
     assert int(S2.isinf().sum()) > 0.99 * S2.numel()
     assert bool(((S == S2) | (S.isnan() & S2.isnan())).all())
+
+
+@pytest.mark.parametrize("prec,depth", [("f64", 0.01), ("f32", 0.05)])
+def test_blocks_many_ranges_wide(gpu, prec, depth):
+    """A lattice whose blocks are thousands of ranges wide, orientations just
+    within the range of its points: none is taken for beyond the range.  The
+    reference is the plain lattice sum with the same runs of points
+    (gk_eval_noalloc), so that both see the same rounded positions.
+
+    Bound: a point has some ten sources within the range, each a polynomial with
+    terms up to 14 times the packed weight 2, some ten roundings; in FP64 the
+    runs start at other points (4 and 8 long), so positions differ by two
+    roundings of 2.4e5, times 105 depth^2, the slope of C'/r."""
+    import ctypes as C
+    from gempy_amd import _lib
+    from gempy_amd.data import KernelOptions, RegularGrid, StackInput
+    from gempy_amd.engine import DeviceStack, _ptr, _stream
+    n, h, no = 96, 5000.123, 3000
+    g = RegularGrid((0.0, n * h) * 3, (n,) * 3)
+    r = np.random.default_rng(11)
+    ijk, axis, ang = r.integers(0, n, (no, 3)), r.integers(0, 3, no), r.uniform(0, np.pi / 2, no)
+    off = -(1.0 - depth * r.random(no))[:, None] * np.stack([np.cos(ang), np.sin(ang)], 1)
+    q = ijk.astype(float)
+    for a in range(3):                       # beside the three edges of the lattice at its origin, where blocks start
+        u, v, i = (a + 1) % 3, (a + 2) % 3, axis == a
+        q[i, u], q[i, v] = 0.0, 0.0
+    q = (q + 0.5) * h
+    for a in range(3):
+        u, v, i = (a + 1) % 3, (a + 2) % 3, axis == a
+        q[i, u] += off[i, 0]
+        q[i, v] += off[i, 1]
+    st = StackInput("wide", np.array([[0.0, 0, 0], [h, h, h]]), [2], np.zeros(2), q, np.ones((no, 3)), np.zeros(no))
+    ds = DeviceStack(st, KernelOptions(range=1.0, c_o=1.0, uni_degree=0), [n * h / 2] * 3)
+    w = torch.zeros(ds.N, dtype=torch.float64)
+    w[:3 * no] = 1.0
+    w = w.cuda()
+    out = []
+    for name in ("gk_eval", "gk_eval_noalloc"):
+        d = _lib.GkEvalDesc()
+        d.kind, d.precision = _lib.GK_POINTS_LATTICE, _lib.GK_F64 if prec == "f64" else _lib.GK_F32
+        for k in range(3):
+            d.origin[k], d.spacing[k], d.res[k] = g.origin[k], g.spacing[k], n
+        S = torch.full((g.n_points,), -1.0, dtype=torch.float64, device=gpu)
+        d.scalar = _ptr(S)
+        print(f"[gpu-case] wide blocks {prec} {name}", flush=True)
+        _lib.check(name, getattr(_lib.load(), name)(ds.h, C.byref(ds.sys), _ptr(w), C.byref(d), _stream()))
+        out.append(S)
+    eps = 2.0 ** -53 if prec == "f64" else 2.0 ** -24
+    bound = 24 * 2 * 14 * 10 * eps
+    if prec == "f64":
+        bound += 24 * 2 * 105 * depth ** 2 * 4 * 2.4e5 * eps
+    assert int((out[1].abs() > 8 * bound).sum()) > n
+    assert float((out[0] - out[1]).abs().max()) <= bound
