@@ -94,10 +94,14 @@ struct ProbeArgs {
   int64_t n, nc;                         // voxels, corners of the lattice
   uint8_t* flag;
   int32_t *rank, *sums;
-  int32_t* total;
+  int32_t* total;                        // number of corners; then whether a voxel lies outside the level
   double* xyz;
   int32_t* map;
 };
+
+__device__ __forceinline__ bool probe_voxel(const ProbeArgs& a, int64_t v) {
+  return v >= 0 && v < a.res[0] * a.res[1] * a.res[2];
+}
 
 __device__ __forceinline__ int64_t probe_corner(const ProbeArgs& a, int64_t v, int c, int64_t* at) {
   at[2] = v % a.res[2] + (c & 1);
@@ -109,7 +113,10 @@ __device__ __forceinline__ int64_t probe_corner(const ProbeArgs& a, int64_t v, i
 __global__ void probe_flags_kernel(ProbeArgs a) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t at[3];
-  if (t < 8 * a.n) a.flag[probe_corner(a, a.vox[t / 8], (int)(t % 8), at)] = 1;
+  if (t >= 8 * a.n) return;
+  const int64_t v = a.vox[t / 8];
+  if (probe_voxel(a, v)) a.flag[probe_corner(a, v, (int)(t % 8), at)] = 1;
+  else a.total[1] = 1;
 }
 
 // Ranks within blocks of 1,024 corners, and the blocks' totals.
@@ -160,6 +167,7 @@ __global__ void probe_points_kernel(ProbeArgs a) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= 9 * a.n) return;
   const int64_t i = t / 9, v = a.vox[i];
+  if (!probe_voxel(a, v)) return;
   const int k = (int)(t % 9);
   int64_t at[3], p = i;
   double f = 0.5;
@@ -193,30 +201,31 @@ extern "C" int gk_octree_probes(gk_handle h, const double* extent, const int64_t
   }
   a.vox = voxels;
   a.n = n;
+  GK_REQUIRE(n < (int64_t)INT32_MAX / 9 && (res[0] + 1.0) * (res[1] + 1.0) * (res[2] + 1.0) < (double)INT32_MAX,
+             GK_ERR_ARG, "gk_octree_probes: level too large");
   a.nc = (res[0] + 1) * (res[1] + 1) * (res[2] + 1);
-  GK_REQUIRE(9 * n < (int64_t)INT32_MAX && a.nc < (int64_t)INT32_MAX, GK_ERR_ARG, "gk_octree_probes: level too large");
   const int64_t nb = gk_ceil_div(a.nc, 1024);
-  const size_t o_rank = gk_round_up(a.nc, 256), o_sums = o_rank + gk_round_up(a.nc * 4, 256),
-               o_total = o_sums + gk_round_up(nb * 4, 256);
+  const size_t o_flag = 256, o_rank = o_flag + gk_round_up(a.nc, 256), o_sums = o_rank + gk_round_up(a.nc * 4, 256);
   void* ws = nullptr;
-  GK_TRY(gk_workspace(h, WS_OCTREE, o_total + 256, &ws));
+  GK_TRY(gk_workspace(h, WS_OCTREE, o_sums + gk_round_up(nb * 4, 256), &ws));
   char* b = static_cast<char*>(ws);
-  a.flag = reinterpret_cast<uint8_t*>(b);
+  a.total = reinterpret_cast<int32_t*>(b);
+  a.flag = reinterpret_cast<uint8_t*>(b + o_flag);
   a.rank = reinterpret_cast<int32_t*>(b + o_rank);
   a.sums = reinterpret_cast<int32_t*>(b + o_sums);
-  a.total = reinterpret_cast<int32_t*>(b + o_total);
   a.xyz = xyz;
   a.map = map;
-  GK_HIP(hipMemsetAsync(a.flag, 0, a.nc, st));
+  GK_HIP(hipMemsetAsync(b, 0, o_flag + a.nc, st));
   hipLaunchKernelGGL(probe_flags_kernel, dim3((unsigned)gk_ceil_div(8 * n, 256)), dim3(256), 0, st, a);
   hipLaunchKernelGGL(probe_rank_kernel, dim3((unsigned)nb), dim3(1024), 0, st, a);
   hipLaunchKernelGGL(probe_scan_kernel, dim3(1), dim3(1024), 0, st, a, nb);
   hipLaunchKernelGGL(probe_points_kernel, dim3((unsigned)gk_ceil_div(9 * n, 256)), dim3(256), 0, st, a);
-  int32_t total = 0;
-  GK_HIP(hipMemcpyAsync(&total, a.total, sizeof(total), hipMemcpyDeviceToHost, st));
+  int32_t total[2] = {0, 0};
+  GK_HIP(hipMemcpyAsync(total, a.total, sizeof(total), hipMemcpyDeviceToHost, st));
   GK_HIP(hipStreamSynchronize(st));
   GK_HIP(hipGetLastError());
-  *n_points = n + total;
+  GK_REQUIRE(total[1] == 0, GK_ERR_ARG, "gk_octree_probes: a voxel index lies outside the level");
+  *n_points = n + total[0];
   return GK_OK;
 }
 

@@ -341,8 +341,8 @@ int gk_octree_points(gk_handle h, const double* extent, const int64_t* res, cons
  * count (host, the call synchronises the stream). */
 /* The same probes without repeats: xyz receives the n centres and then every
  * corner of the voxels once, in lattice order (room for 9 n points), map[9 v + k]
- * (int32) the point of probe k of voxel v, *n_points their number.  Synchronizes
- * the stream. */
+ * (int32) the point of probe k of voxel v, *n_points their number.  Voxel
+ * indices outside the level are refused (GK_ERR_ARG).  Synchronizes the stream. */
 int gk_octree_probes(gk_handle h, const double* extent, const int64_t* res, const int64_t* voxels, int64_t n,
                      double* xyz, int32_t* map, int64_t* n_points, gk_stream stream);
 int gk_octree_refine(gk_handle h, int32_t n_fields, const int32_t* ids, int64_t n, const int64_t* voxels,
