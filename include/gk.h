@@ -335,16 +335,16 @@ int gk_gravity(gk_handle h, int64_t n_devices, int64_t n_kernel, const double* t
  * (xyz [n*9*3], centre first) or, with centres_only, the centres [n*3]. */
 int gk_octree_points(gk_handle h, const double* extent, const int64_t* res, const int64_t* voxels, int64_t n,
                      int32_t centres_only, double* xyz, gk_stream stream);
-/* ids [n_fields][n*9] (int32) at the probe points; refine[v] = 1 when any field
- * differs among voxel v's 9 points; children [8*n] receives the 8 children (at
- * resolution 2*res) of every refined voxel in voxel order; *n_children their
- * count (host, the call synchronises the stream). */
 /* The same probes without repeats: xyz receives the n centres and then every
  * corner of the voxels once, in lattice order (room for 9 n points), map[9 v + k]
  * (int32) the point of probe k of voxel v, *n_points their number.  Voxel
  * indices outside the level are refused (GK_ERR_ARG).  Synchronizes the stream. */
 int gk_octree_probes(gk_handle h, const double* extent, const int64_t* res, const int64_t* voxels, int64_t n,
                      double* xyz, int32_t* map, int64_t* n_points, gk_stream stream);
+/* ids [n_fields][n*9] (int32) at the probe points; refine[v] = 1 when any field
+ * differs among voxel v's 9 points; children [8*n] receives the 8 children (at
+ * resolution 2*res) of every refined voxel in voxel order; *n_children their
+ * count (host, the call synchronises the stream). */
 int gk_octree_refine(gk_handle h, int32_t n_fields, const int32_t* ids, int64_t n, const int64_t* voxels,
                      const int64_t* res, uint8_t* refine, int64_t* children, int64_t* n_children,
                      gk_stream stream);
