@@ -396,18 +396,31 @@ int gemm_launch(int64_t m, int64_t n, int64_t k, const T* A, int64_t lda, const 
     // latency-bound: a 128^3 product on one such tile took 24-30 us, eight
     // 16-deep stages of one global latency each.  Small tiles with 32-deep
     // stages, two of them in flight, spread them over the chip.
-    constexpr int64_t FEW = 512;          // 128 x 128 tiles: two per CU
+    //   m, n, k            128 x 128 tiles   small tiles
+    //   1024, 1024, 1024        165 us          53 us    (64 tiles)
+    //   16384, 256, 256          58             51       (256)
+    //   4352, 1024, 2048        558            385       (272)
+    // Where the large tiles fill their one or two rounds of the 256 CUs nearly
+    // to the end and the product is long, they are the faster ones:
+    //   2048, 2048, 2048        311            333       (256)
+    //   2816, 2816, 4096       1098           1245       (484)
+    //   2560, 2560, 2048 lower  309            320       (210)
+    //   3840, 3840, 256 lower    94            101       (465; 435 tiles, 3712: 93 and 90)
+    constexpr int64_t CUS = 256, FEW = 2 * CUS;
+    const int64_t rounds = gk_ceil_div(tiles * batch, CUS);
+    const bool full = 10 * tiles * batch >= (lower && rounds == 1 ? 8 : 9) * CUS * rounds && k >= (rounds == 1 ? 1024 : 256);
+    const bool few = k % 32 == 0 && tiles * batch < FEW && !full;
     if (k % 32 == 0 && row_tiles) {       // 16 rows x all 128 columns, 4 waves of 16 x 32
       gemm_dispatch<T, Tile<16, 1, 4, 128, 32, 2>, 2>(dim3((unsigned)(m / 16), (unsigned)batch), trans_b, false, st, m,
                                                       n, k, A, lda, B, ldb, alpha, beta, C, ldc, 1, m / 16, sA, sB, sC);
       launched = true;
-    } else if (k % 32 == 0 && lower && tiles * batch < FEW) {
+    } else if (few && lower) {
       const int64_t t64 = m / 64;
       gemm_dispatch<T, Tile<64, 2, 2, 64, 32, 2>, 2>(dim3((unsigned)(t64 * (t64 + 1) / 2), (unsigned)batch), trans_b,
                                                      true, st, m, n, k, A, lda, B, ldb, alpha, beta, C, ldc, t64,
                                                      t64 * (t64 + 1) / 2, sA, sB, sC);
       launched = true;
-    } else if (k % 32 == 0 && !lower && tiles * batch < FEW) {
+    } else if (few) {
       const int64_t t = (m / 32) * (n / 64);
       gemm_dispatch<T, Tile<32, 2, 2, 64, 32, 2>, 2>(dim3((unsigned)t, (unsigned)batch), trans_b, false, st, m, n, k,
                                                      A, lda, B, ldb, alpha, beta, C, ldc, n / 64, t, sA, sB, sC);
