@@ -15,13 +15,16 @@
 // loop is triangulated as a fan.  Triangles wind so that their normals
 // (right-hand rule) point towards increasing field values.
 //
-// The field is read once: a first pass packs every z row into words of 64
-// points (above the level, NaN, masked), and everything that follows works on
-// those words - an eighth of a byte per point and flag - until the crossed edges
-// and the cubes with triangles, few and known, are written.  What it is bound
+// The field is read once: a first pass packs the points, in memory order, into
+// words of 64 (above the level, NaN, masked), and everything that follows works
+// on those words - an eighth of a byte per point and flag - until the crossed
+// edges and the cubes with triangles, few and known, are written.  A neighbour
+// along an axis is the same bit of the words shifted by that axis' step; words
+// that began anew with every z row were mostly empty on lattices of few layers
+// (2000 x 2000 x 2: 1,500 us, 170 now).  What it is bound
 // by is that one read (8 bytes a point, 9 with a mask).  Per-point flags, edge
 // ids and cube cases in memory with scans over them moved about 500 bytes a
-// point: 200^3 cells with a mask took 400 us so and take 90 us now, of which the
+// point: 200^3 cells with a mask took 400 us so and take 83 us now, of which the
 // packing 26 us (72 MB, 2.8 TB/s) and the writing pass 35 us.
 #include <algorithm>
 #include <cmath>
@@ -135,12 +138,13 @@ McTables build_tables() {
 struct McArgs {
   const double* f;
   const uint8_t* mask;
-  int64_t nx, ny, nz, W, words;        // W words of 64 points per z row, words = nx ny W
+  int64_t nx, ny, nz, np, words;       // points, words of 64 points
+  int64_t sx, sy;                      // points from one to the next along x and y
   double level;
   const McTables* T;
-  uint64_t *above, *nan, *msk;         // bit z: value > level / NaN / mask set
-  uint64_t *valid;                     // bit z: cube (x, y, z) is meshed
-  uint64_t *edge[3];                   // bit z: a meshed cube uses the edge from (x, y, z) along the axis
+  uint64_t *above, *nan, *msk;         // bit of a point: value > level / NaN / mask set
+  uint64_t *valid;                     // the cube at the point is meshed
+  uint64_t *edge[3];                   // a meshed cube uses the edge from the point along the axis
   uint32_t *vpre, *tpre;               // vertices / triangles of the block's earlier words
   uint32_t *vsum, *tsum;               // vertices / triangles of each block of MC_WORDS words, then of the earlier ones
   uint32_t *total;                     // both, of all words
@@ -149,18 +153,17 @@ struct McArgs {
 constexpr int MC_WORDS = 256;          // words (threads) per counting block
 constexpr int MC_PER_WAVE = 8;         // words a wave packs: that many loads in flight
 
-// One wave per word: lane l looks at point z = 64 w + l of the row.
+// One wave per word: lane l looks at point 64 w + l.
 __global__ __launch_bounds__(256) void mc_bits_kernel(McArgs a) {
   const int lane = threadIdx.x & 63;
-  const uint32_t w0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * MC_PER_WAVE;   // the words of a lattice fit 32 bits
+  const uint32_t w0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * MC_PER_WAVE;   // the points of a lattice fit 32 bits
   double v[MC_PER_WAVE];
   uint8_t m[MC_PER_WAVE];
 #pragma unroll
   for (int i = 0; i < MC_PER_WAVE; ++i) {
-    const uint32_t w = w0 + i, row = w / (uint32_t)a.W, z = (w - row * (uint32_t)a.W) * 64 + lane;
-    const bool in = w < a.words && z < a.nz;
-    v[i] = in ? a.f[row * a.nz + z] : a.level;          // not above, and no cube reaches it
-    m[i] = in && a.mask ? a.mask[row * a.nz + z] : 1;
+    const int64_t p = (int64_t)(w0 + i) * 64 + lane;
+    v[i] = p < a.np ? a.f[p] : a.level;                 // not above, and no cube reaches it
+    m[i] = p < a.np && a.mask ? a.mask[p] : 1;
   }
 #pragma unroll
   for (int i = 0; i < MC_PER_WAVE; ++i) {
@@ -173,28 +176,40 @@ __global__ __launch_bounds__(256) void mc_bits_kernel(McArgs a) {
   }
 }
 
-// Bits z + 1 and z - 1 of a row's word i at its bit z.
-__device__ __forceinline__ uint64_t bits_up(const uint64_t* b, int64_t i, bool last) {
-  return (b[i] >> 1) | (last ? 0 : b[i + 1] << 63);
-}
-__device__ __forceinline__ uint64_t bits_down(const uint64_t* b, int64_t i, bool first) {
-  return (b[i] << 1) | (first ? 0 : b[i - 1] >> 63);
+// The bits of points 64 i + step + (0 .. 63) and of the points one further
+// along z; 0 before the lattice, of no use behind it.
+struct McPair { uint64_t at, up; };
+__device__ __forceinline__ McPair mc_pair(const McArgs& a, const uint64_t* b, int64_t i, int64_t step) {
+  const int64_t j = i + (step >> 6), last = a.words - 1;        // floor, also of a negative step
+  const int s = (int)(step & 63);                               // the same for all threads
+  const uint64_t w0 = j < 0 ? 0 : b[min(j, last)], w1 = j + 1 < 0 ? 0 : b[min(j + 1, last)];
+  McPair r;
+  r.at = w0 >> s | w1 << 1 << (63 - s);
+  r.up = r.at >> 1 | w1 >> s << 63;
+  return r;
 }
 
-// Meshed cubes of a word: the mask at the far corner (+1, +1, +1), no NaN at any corner.
+// Meshed cubes of a word: all corners on the lattice, the mask at the far
+// corner (+1, +1, +1), no NaN at any corner.
 __global__ __launch_bounds__(256) void mc_valid_kernel(McArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= a.words) return;
-  const uint32_t row = (uint32_t)i / (uint32_t)a.W, w = i - row * a.W, x = row / (uint32_t)a.ny, y = row - x * a.ny;
+  const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz, p = (uint32_t)i * 64, row = p / nz;
+  uint32_t z = p - row * nz, x = row / ny, y = row - x * ny;
   uint64_t ok = 0;
-  if (x + 1 < a.nx && y + 1 < a.ny) {
-    const bool last = w + 1 == a.W;
-    const int64_t left = a.nz - 1 - 64 * (int64_t)w;              // cubes of the row from this word on
-    ok = left >= 64 ? ~0ull : (left > 0 ? (1ull << left) - 1 : 0);
-    ok &= bits_up(a.msk, i + a.ny * a.W + a.W, last);
+  for (uint32_t at = 0; at < 64 && x + 1 < nx;) {       // the rows that reach into the word
+    const uint32_t len = min(nz - z, 64 - at), cubes = min(len, nz - 1 - z);
+    if (y + 1 < ny) ok |= (cubes < 64 ? (1ull << cubes) - 1 : ~0ull) << at;
+    at += len;
+    z = 0;
+    if (++y == ny) { y = 0; ++x; }
+  }
+  if (ok) {
+    ok &= mc_pair(a, a.msk, i, a.sx + a.sy).up;
+#pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int64_t j = i + (k & 1) * a.ny * a.W + (k >> 1) * a.W;
-      ok &= ~(a.nan[j] | bits_up(a.nan, j, last));
+      const McPair n = mc_pair(a, a.nan, i, (k & 1) * a.sx + (k >> 1) * a.sy);
+      ok &= ~(n.at | n.up);
     }
   }
   a.valid[i] = ok;
@@ -209,15 +224,14 @@ __device__ __forceinline__ int mc_case(const uint64_t* lo, const uint64_t* hi, i
   return cs;
 }
 
-// The four rows x + (k & 1), y + (k >> 1) of the cubes of word i (rows beyond
-// the lattice repeat the own one: such cubes are not meshed).
-__device__ __forceinline__ void mc_corner_words(const McArgs& a, int64_t i, int64_t x, int64_t y, bool last,
-                                                uint64_t* lo, uint64_t* hi) {
+// The points x + (k & 1), y + (k >> 1) of the cubes of word i, at z and z + 1
+// (what lies beyond a row's or the lattice's end belongs to no meshed cube).
+__device__ __forceinline__ void mc_corner_words(const McArgs& a, int64_t i, uint64_t* lo, uint64_t* hi) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int64_t j = i + (((k & 1) && x + 1 < a.nx) ? a.ny * a.W : 0) + (((k >> 1) && y + 1 < a.ny) ? a.W : 0);
-    lo[k] = a.above[j];
-    hi[k] = bits_up(a.above, j, last);
+    const McPair p = mc_pair(a, a.above, i, (k & 1) * a.sx + (k >> 1) * a.sy);
+    lo[k] = p.at;
+    hi[k] = p.up;
   }
 }
 
@@ -251,15 +265,13 @@ __global__ __launch_bounds__(MC_WORDS) void mc_count_kernel(McArgs a) {
   const int64_t i = (int64_t)blockIdx.x * MC_WORDS + threadIdx.x;
   uint2 n = make_uint2(0, 0);
   if (i < a.words) {
-    const uint32_t row = (uint32_t)i / (uint32_t)a.W, w = i - row * a.W, x = row / (uint32_t)a.ny, y = row - x * a.ny;
-    const int64_t sx = a.ny * a.W, sy = a.W;
-    const bool first = w == 0, last = w + 1 == a.W;
     uint64_t lo[4], hi[4];
-    mc_corner_words(a, i, x, y, last, lo, hi);
-    const uint64_t v00 = a.valid[i], v10 = x ? a.valid[i - sx] : 0, v01 = y ? a.valid[i - sy] : 0,
-                   v11 = x && y ? a.valid[i - sx - sy] : 0;
-    const uint64_t d00 = bits_down(a.valid, i, first), d10 = x ? bits_down(a.valid, i - sx, first) : 0,
-                   d01 = y ? bits_down(a.valid, i - sy, first) : 0;
+    mc_corner_words(a, i, lo, hi);
+    // cubes one back along x, y, both, and each of them one back along z (a
+    // step across a row's or the lattice's start meets a cube that is not meshed)
+    const McPair c00 = mc_pair(a, a.valid, i, -1), c10 = mc_pair(a, a.valid, i, -a.sx - 1),
+                 c01 = mc_pair(a, a.valid, i, -a.sy - 1), c11 = mc_pair(a, a.valid, i, -a.sx - a.sy - 1);
+    const uint64_t v00 = c00.up, v10 = c10.up, v01 = c01.up, v11 = c11.up, d00 = c00.at, d10 = c10.at, d01 = c01.at;
     const uint64_t e0 = (lo[0] ^ lo[1]) & (v00 | d00 | v01 | d01);
     const uint64_t e1 = (lo[0] ^ lo[2]) & (v00 | d00 | v10 | d10);
     const uint64_t e2 = (lo[0] ^ hi[0]) & (v00 | v10 | v01 | v11);
@@ -304,10 +316,10 @@ __global__ __launch_bounds__(1024) void mc_scan_kernel(McArgs a, int64_t nb, uin
   }
 }
 
-// Vertex of the edge from point (row, z) along axis: vertices are numbered by point, then axis.
-__device__ __forceinline__ uint32_t mc_vertex(const McArgs& a, int64_t row, int64_t z, int axis) {
-  const int64_t i = row * a.W + (z >> 6);
-  const int b = (int)(z & 63);
+// Vertex of the edge from point p along axis: vertices are numbered by point, then axis.
+__device__ __forceinline__ uint32_t mc_vertex(const McArgs& a, int64_t p, int axis) {
+  const int64_t i = p >> 6;
+  const int b = (int)(p & 63);
   const uint64_t e0 = a.edge[0][i], e1 = a.edge[1][i], e2 = a.edge[2][i], below = (1ull << b) - 1;
   uint32_t id = a.vsum[i / MC_WORDS] + a.vpre[i] + __popcll(e0 & below) + __popcll(e1 & below) + __popcll(e2 & below);
   if (axis > 0) id += (uint32_t)(e0 >> b) & 1u;
@@ -315,24 +327,27 @@ __device__ __forceinline__ uint32_t mc_vertex(const McArgs& a, int64_t row, int6
   return id;
 }
 
-// Writes the vertices and the triangles of MC_EMIT words.  Both are few (a
+// Writes the vertices and the triangles of EMIT words.  Both are few (a
 // crossed word holds a handful) and reached through chains of dependent loads,
-// so a block first lists them in LDS, MC_LANES threads per word each at its 4
-// bits, and then gives every vertex and every triangle corner a thread of its
-// own: as one lane per point, almost all idle, this pass took 75 us of 132 at
-// 200^3, and takes 35 us now.  Writes nothing when the results exceed the
-// caller's buffers.
-constexpr int MC_EMIT = 16, MC_LANES = 16;
-static_assert(MC_WORDS % MC_EMIT == 0, "the words of a writing block lie in one counting block");
-__global__ __launch_bounds__(MC_EMIT * MC_LANES) void mc_emit_kernel(McArgs a, double ox, double oy, double oz,
-                                                                     double hx, double hy, double hz, double* verts,
-                                                                     int64_t max_verts, int32_t* faces,
-                                                                     int64_t max_faces) {
-  __shared__ uint32_t list[MC_EMIT * 64 * MC_MAX_TRI];   // vertices (at most 3 a point), then triangles
+// so a block first lists them in LDS, LANES threads per word, and then gives
+// every vertex and every triangle corner a thread of its own: as one lane per
+// point, almost all idle, this pass took 75 us of 132 at 200^3, and takes 35 us
+// now.  Up to MC_SMALL words the blocks alone decide, and they take 2 words
+// (65^3 points, all of them crossed: the call 59 us, 70 with 16 words; 100^3,
+// one surface: 45 and 38).  Writes nothing when the results exceed the caller's
+// buffers.
+constexpr int MC_SMALL = 4800;
+template <int EMIT, int LANES>
+__global__ __launch_bounds__(EMIT * LANES) void mc_emit_kernel(McArgs a, double ox, double oy, double oz,
+                                                             double hx, double hy, double hz, double* verts,
+                                                             int64_t max_verts, int32_t* faces, int64_t max_faces) {
+  constexpr int BITS = 64 / LANES;                       // bits of a word per thread
+  static_assert(MC_WORDS % EMIT == 0, "the words of a writing block lie in one counting block");
+  __shared__ uint32_t list[EMIT * 64 * MC_MAX_TRI];      // vertices (at most 3 a point), then triangles
   __shared__ uint32_t count[2];
   if (a.total[0] > max_verts || a.total[1] > max_faces) return;
-  const uint32_t t = threadIdx.x, w0 = blockIdx.x * MC_EMIT, i = w0 + t / MC_LANES;
-  const int z0 = 4 * (int)(t % MC_LANES);
+  const uint32_t t = threadIdx.x, w0 = blockIdx.x * EMIT, i = w0 + t / LANES;
+  const int z0 = BITS * (int)(t % LANES);
   const bool live = i < a.words;
   // the first vertex and triangle of the block's words (one counting block holds them all)
   const uint32_t vbase = a.vsum[w0 / MC_WORDS] + a.vpre[w0], tbase = a.tsum[w0 / MC_WORDS] + a.tpre[w0];
@@ -352,19 +367,17 @@ __global__ __launch_bounds__(MC_EMIT * MC_LANES) void mc_emit_kernel(McArgs a, d
 #pragma unroll
     for (int u = 0; u < 3; ++u) at += __popcll(e[u] & below);
 #pragma unroll
-    for (int z = z0; z < z0 + 4; ++z)
+    for (int z = z0; z < z0 + BITS; ++z)
 #pragma unroll
       for (uint32_t u = 0; u < 3; ++u)
         if ((e[u] >> z) & 1) list[at++] = (i - w0) << 8 | (uint32_t)z << 2 | u;
   }
   __syncthreads();
-  const int64_t step[3] = {a.ny * a.nz, a.nz, 1};
-  for (uint32_t k = t; k < count[0]; k += MC_EMIT * MC_LANES) {
+  for (uint32_t k = t; k < count[0]; k += EMIT * LANES) {
     const uint32_t r = list[k], axis = r & 3, j = w0 + (r >> 8);
-    const uint32_t row = j / (uint32_t)a.W, z = (j - row * (uint32_t)a.W) * 64 + ((r >> 2) & 63);
+    const uint32_t p = j * 64 + ((r >> 2) & 63), row = p / (uint32_t)a.nz, z = p - row * (uint32_t)a.nz;
     const uint32_t x = row / (uint32_t)a.ny, y = row - x * (uint32_t)a.ny;
-    const int64_t p = row * a.nz + z;
-    const double v0 = a.f[p], v1 = a.f[p + (axis == 0 ? step[0] : (axis == 1 ? step[1] : step[2]))];
+    const double v0 = a.f[p], v1 = a.f[p + (axis == 0 ? a.sx : (axis == 1 ? a.sy : 1))];
     const double s = (a.level - v0) / (v1 - v0);
     double P[3] = {(double)x, (double)y, (double)z};
 #pragma unroll
@@ -376,16 +389,14 @@ __global__ __launch_bounds__(MC_EMIT * MC_LANES) void mc_emit_kernel(McArgs a, d
     o[2] = oz + P[2] * hz;
   }
   __syncthreads();
-  int cs[4] = {0, 0, 0, 0};
+  int cs[BITS] = {};
   uint32_t nt = 0;
   if (live) {
-    const uint32_t row = i / (uint32_t)a.W, w = i - row * (uint32_t)a.W;
-    const uint32_t x = row / (uint32_t)a.ny, y = row - x * (uint32_t)a.ny;
     uint64_t lo[4], hi[4];
-    mc_corner_words(a, i, x, y, w + 1 == a.W, lo, hi);
+    mc_corner_words(a, i, lo, hi);
     const uint64_t act = mc_active(lo, hi, a.valid[i]);
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < BITS; ++b)
       if ((act >> (z0 + b)) & 1) {
         cs[b] = mc_case(lo, hi, z0 + b);
         nt += a.T->ntri[cs[b]];
@@ -393,28 +404,28 @@ __global__ __launch_bounds__(MC_EMIT * MC_LANES) void mc_emit_kernel(McArgs a, d
   }
   uint32_t sum = nt;                     // of the word's threads up to this one
 #pragma unroll
-  for (int o = 1; o < MC_LANES; o <<= 1) {
-    const uint32_t v = __shfl_up(sum, o, MC_LANES);
-    if ((int)(t % MC_LANES) >= o) sum += v;
+  for (int o = 1; o < LANES; o <<= 1) {
+    const uint32_t v = __shfl_up(sum, o, LANES);
+    if ((int)(t % LANES) >= o) sum += v;
   }
   if (live) {
     uint32_t at = a.tpre[i] - a.tpre[w0] + sum - nt;
     if (nt) atomicMax(&count[1], at + nt);
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < BITS; ++b)
       if (cs[b])
         for (uint32_t q = 0; q < a.T->ntri[cs[b]]; ++q)
           list[at++] = (i - w0) << 17 | (uint32_t)(z0 + b) << 11 | (uint32_t)cs[b] << 3 | q;
   }
   __syncthreads();
-  for (uint32_t k = t; k < 3 * count[1]; k += MC_EMIT * MC_LANES) {
+  for (uint32_t k = t; k < 3 * count[1]; k += EMIT * LANES) {
     const uint32_t r = list[k / 3], j = w0 + (r >> 17);
     const int le = a.T->tri[(r >> 3) & 255][r & 7][k % 3], axis = le >> 2, q = le & 3;
     // the edge's start from the cube's corner: q's bits go to the other axes in order
     const int dx = axis == 0 ? 0 : q & 1, dy = axis == 1 ? 0 : (axis == 0 ? q & 1 : q >> 1),
               dz = axis == 2 ? 0 : q >> 1;
-    const uint32_t row = j / (uint32_t)a.W, z = (j - row * (uint32_t)a.W) * 64 + ((r >> 11) & 63);
-    faces[3 * (int64_t)tbase + k] = (int32_t)mc_vertex(a, row + dx * a.ny + dy, z + dz, axis);
+    const int64_t p = (int64_t)j * 64 + ((r >> 11) & 63) + dx * a.sx + dy * a.sy + dz;
+    faces[3 * (int64_t)tbase + k] = (int32_t)mc_vertex(a, p, axis);
   }
 }
 
@@ -434,7 +445,7 @@ extern "C" int gk_marching_cubes(gk_handle h, const double* field, const int64_t
   *n_faces = 0;
   if (nx < 2 || ny < 2 || nz < 2) return GK_OK;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t W = gk_ceil_div(nz, 64), words = nx * ny * W, nb = gk_ceil_div(words, MC_WORDS);
+  const int64_t words = gk_ceil_div(np_, 64), nb = gk_ceil_div(words, MC_WORDS);
   // workspace: totals | 7 word arrays | 2 counts per word | 2 sums per block
   size_t need = 0;
   auto take = [&](size_t bytes) { size_t o = need; need += gk_round_up(bytes, 256); return o; };
@@ -461,7 +472,8 @@ extern "C" int gk_marching_cubes(gk_handle h, const double* field, const int64_t
   if (!h->mesh_counts) GK_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->mesh_counts), 64, hipHostMallocDefault));
   McArgs a{};
   a.f = field; a.mask = mask;
-  a.nx = nx; a.ny = ny; a.nz = nz; a.W = W; a.words = words;
+  a.nx = nx; a.ny = ny; a.nz = nz; a.np = np_; a.words = words;
+  a.sx = ny * nz; a.sy = nz;
   a.level = level;
   a.T = static_cast<const McTables*>(h->mesh_tables);
   uint64_t** wp[7] = {&a.above, &a.nan, &a.msk, &a.valid, &a.edge[0], &a.edge[1], &a.edge[2]};
@@ -473,9 +485,14 @@ extern "C" int gk_marching_cubes(gk_handle h, const double* field, const int64_t
   hipLaunchKernelGGL(mc_valid_kernel, dim3((unsigned)gk_ceil_div(words, 256)), dim3(256), 0, st, a);
   hipLaunchKernelGGL(mc_count_kernel, dim3((unsigned)nb), dim3(MC_WORDS), 0, st, a);
   hipLaunchKernelGGL(mc_scan_kernel, dim3(1), dim3(1024), 0, st, a, nb, h->mesh_counts);
-  if (verts && faces)
-    hipLaunchKernelGGL(mc_emit_kernel, dim3((unsigned)gk_ceil_div(words, MC_EMIT)), dim3(MC_EMIT * MC_LANES), 0, st, a, origin[0],
-                       origin[1], origin[2], spacing[0], spacing[1], spacing[2], verts, max_verts, faces, max_faces);
+  if (verts && faces) {
+    auto emit = [&](auto kernel, int per, int threads) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)gk_ceil_div(words, per)), dim3(threads), 0, st, a, origin[0], origin[1],
+                         origin[2], spacing[0], spacing[1], spacing[2], verts, max_verts, faces, max_faces);
+    };
+    if (words <= MC_SMALL) emit(mc_emit_kernel<2, 64>, 2, 128);
+    else emit(mc_emit_kernel<16, 16>, 16, 256);
+  }
   GK_HIP(hipGetLastError());
   GK_HIP(hipStreamSynchronize(st));
   const uint32_t counts[2] = {h->mesh_counts[0], h->mesh_counts[1]};
