@@ -1269,26 +1269,22 @@ __global__ __launch_bounds__(256) void diag_apply_kernel(const T* Dk, T* b) {
 
 // Factor + invert one 256-wide diagonal block from two 128-wide halves.
 // Cholesky: L = [L11 0; L21 L22], L^-1 = [X11 0; -X22 L21 X11  X22].  L21 is
-// formed in T1; with copy_l21 false the caller copies it into A later (no
-// later step of the factorization reads it from A).  The upper-right quadrant
-// of Dinv is zeroed once per factorization by the caller.
-template <typename T>
-int diag256_chol(T* A, int64_t lda, int64_t n, int64_t k0, T* dinv, int32_t* dinfo, T* T1, T* T2, hipStream_t st,
-                 bool copy_l21 = true) {
-  T* A11 = A + k0 * lda + k0;
-  T* A21 = A + (k0 + DB) * lda + k0;
-  T* A22 = A21 + DB;
-  T* D = dinv + k0 * NB;                 // 256 x 256, ld NB
-  potrf128<T>(A11, lda, D, NB, dinfo, k0, n, st);
-  GK_TRY(gemm_launch<T>(DB, DB, DB, A21, lda, D, NB, true, T(1), T(0), T1, DB, false, st));        // L21
-  if (copy_l21)
-    hipLaunchKernelGGL(copy_block_kernel<T>, dim3(DB * DB / 256), dim3(256), 0, st, T1, (int64_t)DB, A21,
-                       lda, (int64_t)DB, (int64_t)DB);
-  GK_TRY(gemm_launch<T>(DB, DB, DB, T1, DB, T1, DB, true, T(-1), T(1), A22, lda, false, st));      // syrk
-  potrf128<T>(A22, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, n, st);
-  GK_TRY(gemm_launch<T>(DB, DB, DB, T1, DB, D, NB, false, T(1), T(0), T2, DB, false, st));         // L21 X11
-  GK_TRY(gemm_launch<T>(DB, DB, DB, D + DB * NB + DB, NB, T2, DB, false, T(-1), T(0), D + DB * NB, NB,
-                        false, st));
+// formed in T1; the caller copies it into A later (no later step of the
+// factorization reads it from A).  The upper-right quadrant of Dinv is zeroed
+// once per factorization by the caller.
+int diag256_chol32(float* A, int64_t lda, int64_t n, int64_t k0, float* dinv, int32_t* dinfo, float* T1, float* T2,
+                   hipStream_t st) {
+  float* A11 = A + k0 * lda + k0;
+  float* A21 = A + (k0 + DB) * lda + k0;
+  float* A22 = A21 + DB;
+  float* D = dinv + k0 * NB;             // 256 x 256, ld NB
+  potrf128<float>(A11, lda, D, NB, dinfo, k0, n, st);
+  GK_TRY(gemm_launch<float>(DB, DB, DB, A21, lda, D, NB, true, 1.0f, 0.0f, T1, DB, false, st));    // L21
+  GK_TRY(gemm_launch<float>(DB, DB, DB, T1, DB, T1, DB, true, -1.0f, 1.0f, A22, lda, false, st));  // syrk
+  potrf128<float>(A22, lda, D + DB * NB + DB, NB, dinfo, k0 + DB, n, st);
+  GK_TRY(gemm_launch<float>(DB, DB, DB, T1, DB, D, NB, false, 1.0f, 0.0f, T2, DB, false, st));     // L21 X11
+  GK_TRY(gemm_launch<float>(DB, DB, DB, D + DB * NB + DB, NB, T2, DB, false, -1.0f, 0.0f, D + DB * NB, NB,
+                            false, st));
   return GK_OK;
 }
 
@@ -1478,7 +1474,7 @@ struct CholRec {
 static int chol32_panel(float* A, int64_t lda, int64_t n, int64_t kb, float* dinv, int32_t* dinfo, float* W, float* Tb,
                         hipStream_t s, _Float16* P = nullptr) {
   const int64_t k0 = kb * NB, rem = lda - k0 - NB;
-  GK_TRY(diag256_chol<float>(A, lda, n, k0, dinv, dinfo, Tb, Tb + DB * DB, s, false));
+  GK_TRY(diag256_chol32(A, lda, n, k0, dinv, dinfo, Tb, Tb + DB * DB, s));
   if (rem > 0) {
     GK_TRY(gemm_launch<float>(rem, NB, NB, A + (k0 + NB) * lda + k0, lda, dinv + k0 * NB, NB, true, 1.0f, 0.0f, W,
                               NB, false, s));
@@ -1571,13 +1567,14 @@ static int cholesky_impl(gk_handle h, T* A, int64_t n, int64_t lda, T* dinv, int
   split16 = split16 && sizeof(T) == 4;
   void* ws = nullptr;
   const size_t split_bytes = split16 ? 4 * 2 * (size_t)lda * NB * sizeof(_Float16) : 0;
-  GK_TRY(gk_workspace(h, WS_FACTOR, 256 + (2 * (size_t)lda * NB + 2 * DB * DB) * sizeof(T) + split_bytes, &ws));
+  // FP64: one panel buffer; FP32: two (look-ahead) and two 128 x 128 blocks
+  const size_t panels = sizeof(T) == 8 ? (size_t)lda * NB : 2 * (size_t)lda * NB + 2 * DB * DB;
+  GK_TRY(gk_workspace(h, WS_FACTOR, 256 + panels * sizeof(T) + split_bytes, &ws));
   int32_t* dinfo = static_cast<int32_t*>(ws);
   int32_t* tile_ctr = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + 64);   // 8 XCD tile counters
-  T* W = reinterpret_cast<T*>(static_cast<char*>(ws) + 256);       // two panel buffers (FP32 look-ahead)
-  T* Tb = W + 2 * (size_t)lda * NB;
+  T* W = reinterpret_cast<T*>(static_cast<char*>(ws) + 256);
   // four tiled split panels of lda x NB x 2 halves
-  _Float16* Hs = split16 ? reinterpret_cast<_Float16*>(Tb + 2 * DB * DB) : nullptr;
+  _Float16* Hs = split16 ? reinterpret_cast<_Float16*>(W + panels) : nullptr;
   GK_HIP(hipMemsetAsync(ws, 0, 256, st));                              // info word and tile counters
   GK_HIP(hipMemsetAsync(dinv, 0, (size_t)lda * NB * sizeof(T), st));   // Dinv plane: upper-right quadrants stay 0
   if (n < lda) {
@@ -1612,6 +1609,7 @@ static int cholesky_impl(gk_handle h, T* A, int64_t n, int64_t lda, T* dinv, int
       hipEvent_t* ev;
       GK_TRY(gk_side_stream(h, &s2, &ev));
       T* Wb[2] = {W, W + (size_t)lda * NB};
+      T* Tb = W + 2 * (size_t)lda * NB;
       _Float16* Hb[4];
       for (int b = 0; b < 4; ++b) Hb[b] = Hs ? Hs + 2 * b * (size_t)lda * NB : nullptr;
       auto sp = [&](int64_t kb) { return Hb[kb % 4]; };

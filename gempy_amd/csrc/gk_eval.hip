@@ -1147,7 +1147,7 @@ static int64_t source_groups(const gk_system* sys) {
 
 static size_t sources_bytes(const gk_system* sys) {
   const int64_t R = sys->n_rest, S = sys->n_surf, no = sys->n_ori;
-  return gk_round_up(S * 8, 256) + gk_round_up((R + S) * 32, 256) + gk_round_up(no * 64, 256) + 256;
+  return gk_round_up((R + S) * 32, 256) + gk_round_up(no * 64, 256) + 256;
 }
 
 // The handle's workspace of packed sources, with the groups' flags behind them.
@@ -1461,7 +1461,8 @@ static int eval_impl(gk_handle h, const gk_system* sys, const double* weights, g
   char* part = nullptr;
   size_t part_bytes = 0;
   if (ext) {
-    const size_t need = gk_round_up(sources_bytes(sys), 256);
+    // 8 bytes a surface more than the sources take: the limit that gk.h states
+    const size_t need = sources_bytes(sys) + gk_round_up(sys->n_surf * 8, 256);
     GK_REQUIRE(need <= ext_bytes, GK_ERR_ARG,
                "gk_eval_noalloc: the system's packed sources need %zu bytes, the scratch array holds %zu "
                "(GK_EVAL_SCRATCH_BYTES)", need, ext_bytes);

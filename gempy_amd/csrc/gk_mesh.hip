@@ -37,7 +37,6 @@ constexpr int MC_MAX_TRI = 5;    // triangles per cube case, at most (the constr
 
 struct McTables {
   uint8_t ntri[256];
-  uint16_t edges[256];                 // bit e: local edge e crosses
   int8_t tri[256][MC_MAX_TRI][3];      // local edges of each triangle
 };
 
@@ -85,7 +84,6 @@ McTables build_tables() {
   for (int cs = 0; cs < 256; ++cs) {
     int next[12];
     for (int& e : next) e = -1;
-    uint16_t used = 0;
     for (int f = 0; f < 6; ++f) {
       int cross[4], dir[4], nc = 0;     // crossing edges in boundary order, +1 entering the "above" run
       for (int i = 0; i < 4; ++i) {
@@ -105,13 +103,11 @@ McTables build_tables() {
           const int k = (i + j) % nc;
           if (dir[k] == -1) {
             next[cross[i]] = cross[k];
-            used |= (uint16_t)((1u << cross[i]) | (1u << cross[k]));
             break;
           }
         }
       }
     }
-    T.edges[cs] = used;
     int nt = 0;
     bool seen[12] = {};
     for (int s = 0; s < 12; ++s) {
