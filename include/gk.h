@@ -239,6 +239,9 @@ int gk_adjoint_full(gk_handle h, const gk_system* sys, const double* w, int64_t 
                     double* lam_out, gk_stream stream);
 
 /* ---- (c) evaluation: scalar field, gradient, ids ------------------------ */
+/* Lattices worth 0.2 ms of pairs or more may be evaluated in blocks, whose lists
+ * and node sums take up to 288 MiB of device memory; the handle keeps it until
+ * gk_destroy.  Where it cannot be allocated the pairs are summed one by one. */
 int gk_eval(gk_handle h, const gk_system* sys, const double* weights, gk_eval_desc* desc,
             gk_stream stream);
 /* gk_eval without any device allocation, for callers that cannot allocate
@@ -250,9 +253,9 @@ int gk_eval(gk_handle h, const gk_system* sys, const double* weights, gk_eval_de
  * bytes, FP64) exceed it are rejected with GK_ERR_ARG; explicit point sets
  * use fewer source splits when their partials do not fit; lattices are summed
  * pair by pair, where gk_eval takes large ones in blocks.  Results equal
- * gk_eval's whenever the same split is used, and within rounding otherwise.  Every call on one GPU shares
- * that array: calls that overlap on one GPU (other streams, other threads)
- * race and must be serialised by the caller. */
+ * gk_eval's whenever the same split is used, and within rounding otherwise.
+ * Every call on one GPU shares that array: calls that overlap on one GPU (other
+ * streams, other threads) race and must be serialised by the caller. */
 #define GK_EVAL_SCRATCH_BYTES (32u << 20)
 int gk_eval_noalloc(gk_handle h, const gk_system* sys, const double* weights, gk_eval_desc* desc,
                     gk_stream stream);
