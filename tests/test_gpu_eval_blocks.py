@@ -103,3 +103,44 @@ def test_weight_that_is_not_finite(gpu, rng_):
     w[3 * 600 + 17] = float("nan")
     S, _, _ = ds.evaluate_lattice(g, w)
     assert bool(torch.isnan(S).all())
+
+
+def _extended(ds, w, X):
+    """The field at X in extended precision, term by term."""
+    ld = np.longdouble
+    st, k, no = ds.stack, ds.kopts, ds.stack.n_orientations
+    a, c, w = ld(k.range), ld(k.c_o), np.asarray(w, dtype=ld)
+    W = np.zeros(len(st.sp_xyz), dtype=ld)
+    W[ds.rest_idx] = w[3 * no:3 * no + len(ds.rest_idx)]
+    at = 0
+    for n in st.counts:
+        W[at] = -W[at + 1:at + n].sum()
+        at += n
+    out = np.zeros(len(X), dtype=ld)
+    for i, x in enumerate(np.asarray(X, dtype=ld)):
+        r = np.sqrt((((x - st.sp_xyz.astype(ld)) / a) ** 2).sum(1))
+        C = 1 - 7 * r ** 2 + ld(35) / 4 * r ** 3 - ld(7) / 2 * r ** 5 + ld(3) / 4 * r ** 7
+        d = (st.ori_xyz.astype(ld) - x) / a
+        r2 = np.sqrt((d ** 2).sum(1))
+        P = -14 + ld(105) / 4 * r2 - ld(35) / 2 * r2 ** 3 + ld(21) / 4 * r2 ** 5
+        dot = (d * w[:3 * no].reshape(3, no).T).sum(1)
+        out[i] = (ld(k.i_res) * c * (W * np.where(r < 1, C, 0)).sum() +
+                  ld(k.gi_res) * c / a * (dot * np.where(r2 < 1, P, 0)).sum() +
+                  ld(k.gi_res) * (w[3 * no + len(ds.rest_idx):] * x).sum())
+    return out
+
+
+@pytest.mark.parametrize("res,points,oris,rng_,prec", [
+    ((101, 97, 103), 2000, 400, 1732.05, "f64"), ((96, 97, 98), 3000, 700, 1300.0, "f64"),
+    ((96, 97, 98), 3000, 700, 450.0, "f64"), ((100, 100, 100), 3000, 600, 1732.05, "f32")])
+def test_matches_extended_precision(gpu, res, points, oris, rng_, prec):
+    """Half of the bound that two such sums are compared with above."""
+    from gempy_amd import synthetic
+    from gempy_amd.data import RegularGrid
+    ds, w = _setup(points, oris, rng_)
+    g = RegularGrid(synthetic.EXTENT, res)
+    S, _, _ = ds.evaluate_lattice(g, w, _prec(prec))
+    at = np.random.default_rng(7).integers(0, g.n_points, 48)
+    err = np.abs(S.cpu().numpy()[at].astype(np.longdouble) - _extended(ds, w.cpu().numpy(), g.values()[at])).max()
+    print(f"[gpu-case] blocks {res} {prec} range {rng_}: {float(err):.2e} off extended precision", flush=True)
+    assert err <= _bound(points, oris, rng_, prec) / 2

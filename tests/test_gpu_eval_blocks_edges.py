@@ -87,3 +87,65 @@ def test_blocks_many_ranges_wide(gpu, prec, depth):
         bound += 24 * 2 * 105 * depth ** 2 * 4 * 2.4e5 * eps
     assert int((out[1].abs() > 8 * bound).sum()) > n
     assert float((out[0] - out[1]).abs().max()) <= bound
+
+
+def _bound(points, oris, range_, prec, gradient=False):
+    """As in test_gpu_eval_blocks.py."""
+    from test_gpu_eval_blocks import _bound as b
+    return b(points, oris, range_, prec, gradient)
+
+
+@pytest.mark.parametrize("prec,ny", [("f64", 24), ("f32", 16)])
+def test_slab(gpu, prec, ny):
+    from gempy_amd import _lib, synthetic
+    from gempy_amd.data import RegularGrid
+    ds, w = _ds(3000, 600, 1732.05)
+    g = RegularGrid(synthetic.EXTENT, (150, ny, 170))
+    S, _, _ = ds.evaluate_lattice(g, w, _lib.GK_F64 if prec == "f64" else _lib.GK_F32)
+    S2, _, _ = ds.evaluate_points(torch.tensor(g.values(), device="cuda"), w)
+    assert float((S - S2).abs().max()) <= _bound(3000, 600, 1732.05, prec)
+
+
+@pytest.mark.parametrize("range_,gradient", [(1732.05, False), (450.0, True)])
+def test_negative_spacing(gpu, range_, gradient):
+    """Axes that run downwards: the same field, reversed."""
+    from gempy_amd.data import RegularGrid
+    n = (3000, 600) if not gradient else (2000, 500)
+    ds, w = _ds(*n, range_)
+    g = RegularGrid((1000.0, 0.0, 0.0, 1000.0, 1000.0, 0.0), (100, 101, 102))
+    S, G, _ = ds.evaluate_lattice(g, w, gradient=gradient)
+    S2, G2, _ = ds.evaluate_points(torch.tensor(g.values(), device="cuda"), w, gradient=gradient)
+    assert float((S - S2).abs().max()) <= _bound(*n, range_, "f64")
+    if gradient:
+        assert float((G - G2).abs().max()) <= _bound(*n, range_, "f64", True)
+
+
+@pytest.mark.parametrize("degree", [0, 2])
+@pytest.mark.parametrize("faults", [0, 2])
+def test_drift_and_fault_columns(gpu, degree, faults):
+    """Drift of degree 0 and 2 and fault columns, on a ragged lattice, with ids.
+    The drift's terms reach 2 x 10^6 times weights up to 5: 16 roundings of their
+    sum more than the pairs have."""
+    from gempy_amd import synthetic
+    from gempy_amd.data import KernelOptions, RegularGrid
+    from gempy_amd.engine import DeviceStack
+    m = synthetic.config3(seed=5, n_points=2500, n_ori=500, n_surfaces=4, resolution=(8, 8, 8)).stacks[0]
+    step = np.stack([np.where(m.sp_xyz[:, 0] > 400.0, 2.0, 1.0), np.where(m.sp_xyz[:, 1] > 300.0, 1.0, 2.0)], 1)
+    ds = DeviceStack(m, KernelOptions(range=1732.05, c_o=1732.05 ** 2 / 42.0, uni_degree=degree), [500.0] * 3,
+                     fault_sp=step[:, :faults] if faults else None)
+    assert ds.n_fault == faults
+    w = torch.randn(ds.N, dtype=torch.float64, generator=torch.Generator().manual_seed(9)).cuda()
+    g = RegularGrid(synthetic.EXTENT, (101, 99, 97))
+    X = torch.tensor(g.values(), device="cuda")
+    fv = None
+    if faults:
+        fv = torch.stack([(X[:, 0] > 400.0).double() + 1.0, (X[:, 1] <= 300.0).double() + 1.0], 1).contiguous()
+    thr = [3e6, 0.0, -3e6]
+    S, _, ids = ds.evaluate_lattice(g, w, thresholds=thr, fault_values=fv)
+    S2, _, _ = ds.evaluate_points(X, w, fault_values=fv)
+    drift = 16 * 2.0 ** -53 * 2 * 5 * 6e6 if degree == 2 else 0.0
+    assert float((S - S2).abs().max()) <= _bound(2500, 500, 1732.05, "f64") + drift
+    assert bool((ids == 1 + sum((S < t).int() for t in thr)).all())
+    if faults:                                # the columns do reach the field
+        S0, _, _ = ds.evaluate_lattice(g, w, fault_values=torch.zeros_like(fv))
+        assert float((S - S0).abs().min()) > 0.0
