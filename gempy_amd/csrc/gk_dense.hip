@@ -903,8 +903,9 @@ __device__ __forceinline__ double lane_value(double v, int l) {
 // step(), so that the caller can place other work between them.  FP32: the
 // hardware reciprocal square root (within 1 ulp), the factor being an FP32
 // preconditioner.  FP64: the hardware seed (2^-24), one Newton step (2^-47),
-// then one residual step each for the root and the reciprocal, which leaves
-// both within 1 ulp: a chain of 9 operations where the IEEE square root and
+// then one residual step each for the root (correctly rounded in a simulation)
+// and the reciprocal (within 1.5 ulp of 1 / sqrt(d), as a division by the
+// rounded root is): a chain of 9 operations where the IEEE square root and
 // division take several times that.
 template <typename T> struct PivotChain;
 template <> struct PivotChain<float> {

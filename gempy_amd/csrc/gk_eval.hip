@@ -142,8 +142,9 @@ template <typename T, int PPT> struct TableRun {
 // exact constants, which costs nothing there (the weight joins the last
 // product) and loses nothing near the range, where C vanishes.  With a clamp
 // and a full Newton step per pair instead, field and gradient of 1.2e6 points
-// and 1,900 sources took 2.39 ms against 2.14, the masked field of 1.2e6
-// points and 6,000 sources 4.82 against 4.28.
+// and 1,900 sources took 2.39 ms against 2.14 (1.78 since tiles run over the
+// sources they hold), the masked field of 1.2e6 points and 6,000 sources 4.82
+// against 4.28 (1.69 in blocks).
 template <typename T> __device__ __forceinline__ T rho_poly(T u, T r, T h3, T c0) {
   if constexpr (sizeof(T) == 4) return fma(r, u, c0);        // u = Q
   else return fma(r * u, h3, c0);                            // u = Q / 2
@@ -381,9 +382,9 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
   // Explicit points come without a box.  Where every source and every point
   // of the wave lies within half the range of the centre no pair is beyond it,
   // and the same sums go without the mask: the preparing launch leaves a flag
-  // per group of sources, the wave looks at its own points.  Scalar at 20,000
-  // points of 25,000 sources 370 us with the mask, 339 without; a product of
-  // 25,000 data 431 and 391, 100,000 points of 6,000 sources 390 and 351.
+  // per group of sources, the wave looks at its own points.  A product of
+  // 25,000 data 431 us with the mask, 391 without; 100,000 points of 6,000
+  // sources 390 and 351.
   bool inside = false;
   if constexpr (!LATTICE && MASKED) {
     bool out = a.src_out == nullptr;
@@ -528,8 +529,10 @@ __global__ __launch_bounds__(TS) void eval_kernel(EvalArgs a) {
 // points of the block).  The bound is that of a source beside the block at a
 // gap of g half widths, a = sqrt(1 + g^2).  Measured in 80-bit arithmetic for
 // unit weights at half width 0.036 of the range: N = 16, g = 3: 2e-17 for C
-// and 2e-15 for an orientation's term (values up to 3: the rounding of one
-// such term), 15 times more per 0.5 less of g; N = 8, g = 2.5: 8e-10 and
+// and 2e-15 for an orientation's term (computing one such term in FP64 rounds
+// it by 4e-16 rms and up to 3.4e-15, its largest part being 14; C by 1.5e-16
+// and 1.2e-15), for the worst source at that gap; four times less per 0.5 more
+// of g, 15 times more per 0.5 less.  N = 8, g = 2.5: 8e-10 and
 // 5e-8 (FP32 sums), 3 times more per 0.5.  The error grows with the square of
 // the half width, which the gap makes up for.
 // The interpolant passes rounding errors of the node sums on without growth
@@ -1258,8 +1261,10 @@ static int run_eval(gk_handle h, EvalArgs& a, bool lattice, int precision, bool 
 // direct kernel (f64 4.3e-13 s each, f32 3.1e-13, 1.4 times that with the
 // mask) over the groups of 192 (block, source) pairs spread evenly (an R
 // sequence) over the blocks and the source box.  Nodes are used without
-// gradient: for the same error a gradient needs about 20 nodes per axis, more
-// than most blocks have points.
+// gradient: derivatives of the interpolant are 4,000 times less exact (8e-12 of
+// an orientation's gradient with 16 nodes per axis, 4e-13 with 18, 6e-15 with
+// 20), and a form with 20 nodes, for blocks of well more than 8,000 points, is
+// not built.
 //   8e6 points, 25,000 sources, f64: 86.9 ms direct, 22.5 in blocks (12.4 near, 10.0 nodes)
 //   1e6 points, 6,000 sources, f32: 1.88 ms and 0.61
 //   2.1e6 points, 1,920 sources, f64: 1.98 ms and 1.10

@@ -25,7 +25,7 @@
 // by is that one read (8 bytes a point, 9 with a mask).  Per-point flags, edge
 // ids and cube cases in memory with scans over them moved about 500 bytes a
 // point: 200^3 cells with a mask took 400 us so and take 83 us now, of which the
-// packing 26 us (72 MB, 2.8 TB/s) and the writing pass 35 us.
+// packing 22 us (75 MB, 3.4 TB/s) and the writing pass 32 us.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -327,7 +327,7 @@ __device__ __forceinline__ uint32_t mc_vertex(const McArgs& a, int64_t p, int ax
 // crossed word holds a handful) and reached through chains of dependent loads,
 // so a block first lists them in LDS, LANES threads per word, and then gives
 // every vertex and every triangle corner a thread of its own: as one lane per
-// point, almost all idle, this pass took 75 us of 132 at 200^3, and takes 35 us
+// point, almost all idle, this pass took 75 us of 132 at 200^3, and takes 32 us
 // now.  Up to MC_SMALL words the blocks alone decide, and they take 2 words
 // (65^3 points, all of them crossed: the call 59 us, 70 with 16 words; 100^3,
 // one surface: 45 and 38).  Writes nothing when the results exceed the caller's
