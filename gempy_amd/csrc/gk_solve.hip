@@ -428,8 +428,10 @@ struct Solver {
       shift = f64 ? (shift == 0.0 ? 1e-13 : shift * 100.0) : shift * 4.0;
     }
     *info_out = info;
+    // the local preconditioner is built beside the factor, in buffers that the
+    // next solve may lay out otherwise: waited for also after a breakdown
+    if (pc_ready) GK_HIP(hipStreamWaitEvent(st, pc_ready, 0));
     if (info != 0) return GK_ERR_NOT_SPD;
-    if (pc_ready) GK_HIP(hipStreamWaitEvent(st, pc_ready, 0));    // local preconditioner built beside the factor
     return setup_drift();
   }
 

@@ -14,7 +14,7 @@ LIB = os.path.join(os.path.dirname(HERE), "gempy_amd", "libgkhip.so")
 _HEAD = """
 import ctypes as C, sys
 fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
-fake.fake_name.restype = C.c_char_p
+fake.fake_name.restype = fake.fake_log.restype = C.c_char_p
 lib = C.CDLL(sys.argv[2])
 lib.gk_last_error.restype = C.c_char_p
 h = C.c_void_p()

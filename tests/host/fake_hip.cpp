@@ -7,7 +7,9 @@
 //   * copies that the library makes to the device are kept (the last one of at
 //     least fake_watch bytes), and each launch notes whether a pointer in its
 //     first argument leads to those bytes, intact, in a live allocation
-//   * copies to the host take fake_d2h's bytes where set
+//   * copies to the host of as many bytes as fake_d2h was given take those
+//   * streams and events have names of their own, and fake_log tells what was
+//     put on which stream, a line each
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
 #include <cstdint>
@@ -20,18 +22,28 @@ struct Launch { std::string name; unsigned grid[3], block[3]; int watched; };
 static std::map<const void*, std::string> names;
 static std::map<char*, size_t> live;
 static std::vector<Launch> launches;
-static std::vector<char> watched, d2h;
+static std::vector<char> watched;
+static std::map<size_t, std::vector<char>> d2h;
+static std::string journal;
+static uintptr_t next_id = 1;
 static size_t watch_min = 0;
 static char *arena = nullptr, *top = nullptr;
 constexpr size_t ARENA = 8ull << 30;
 static dim3 cfg_grid, cfg_block;
+static hipStream_t cfg_stream;
+
+static void note(const char* what, hipStream_t s, const std::string& of) {
+  journal += std::string(what) + " stream" + std::to_string((uintptr_t)s) + " " + of + "\n";
+}
+static std::string event_name(hipEvent_t e) { return "event" + std::to_string((uintptr_t)e); }
 static char symbol[1 << 12];
 
 extern "C" {
 void fake_watch(size_t bytes) { watch_min = bytes; }
-void fake_d2h(const void* p, size_t n) { d2h.assign((const char*)p, (const char*)p + n); }
+void fake_d2h(const void* p, size_t n) { d2h[n].assign((const char*)p, (const char*)p + n); }
+const char* fake_log() { return journal.c_str(); }
 int fake_launches() { return (int)launches.size(); }
-void fake_clear() { launches.clear(); }
+void fake_clear() { launches.clear(); journal.clear(); }
 const char* fake_name(int i) { return launches[i].name.c_str(); }
 unsigned fake_grid(int i, int k) { return launches[i].grid[k]; }
 int fake_intact(int i) { return launches[i].watched; }
@@ -42,12 +54,15 @@ void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsig
   names[f] = name;
 }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
-hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) { cfg_grid = g; cfg_block = b; return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* st) {
-  *g = cfg_grid; *b = cfg_block; *s = 0; *st = nullptr;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t s) {
+  cfg_grid = g; cfg_block = b; cfg_stream = s;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t, hipStream_t) {
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* st) {
+  *g = cfg_grid; *b = cfg_block; *s = 0; *st = cfg_stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t, hipStream_t st) {
   Launch l{names.count(f) ? names[f] : "?", {g.x, g.y, g.z}, {b.x, b.y, b.z}, 0};
   if (!watched.empty())
     for (int i = 0; i < 16; ++i) {
@@ -57,6 +72,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t, h
         if (p >= base && p + watched.size() <= base + size && !memcmp(p, watched.data(), watched.size())) l.watched = 1;
     }
   launches.push_back(l);
+  note("launch", st, l.name);
   return hipSuccess;
 }
 hipError_t hipMalloc(void** p, size_t n) {
@@ -80,7 +96,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(1, n); retu
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
   if (k == hipMemcpyHostToDevice && watch_min && n >= watch_min) watched.assign((const char*)s, (const char*)s + n);
-  if (k == hipMemcpyDeviceToHost && d2h.size() == n) memcpy(d, d2h.data(), n);
+  if (k == hipMemcpyDeviceToHost && d2h.count(n)) memcpy(d, d2h[n].data(), n);
   else memcpy(d, s, n);
   return hipSuccess;
 }
@@ -93,14 +109,14 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; 
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "fake"; }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = nullptr; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)next_id++; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipEventCreate(hipEvent_t* e) { *e = nullptr; return hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = nullptr; return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) { note("wait", s, event_name(e)); return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)next_id++; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = (hipEvent_t)next_id++; return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { note("record", s, event_name(e)); return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { *t = 0; return hipSuccess; }
 }
