@@ -360,7 +360,7 @@ __global__ __launch_bounds__(64 * LI_WAVES) void local_inverse_kernel(Geo G, int
     const int m_all = __shfl(end, K - 1);
     __builtin_amdgcn_wave_barrier();
     for (int d = 0; d < rows; ++d) {
-      un[end - rows + d] = (int32_t)unknown_of(G.s, q, d);
+      un[end - rows + d] = q < n ? (int32_t)unknown_of(G.s, q, d) : -1;     // (no neighbour: a position is no number)
       orig[end - rows + d] = 3 * lane + d;
     }
     __builtin_amdgcn_wave_barrier();
@@ -633,7 +633,7 @@ __global__ void spai_apply_kernel(gk_system sys, int64_t n, const int32_t* idx, 
     const int64_t q = idx[p * K + j];
     double xq[3];
     for (int c = 0; c < 3; ++c) {
-      const int64_t uc = unknown_of(sys, q, c);
+      const int64_t uc = q < n ? unknown_of(sys, q, c) : -1;
       xq[c] = uc >= 0 ? u[uc] : 0.0;
     }
     const float* B = Y + (p * K + j) * O;
